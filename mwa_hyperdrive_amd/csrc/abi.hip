@@ -208,7 +208,8 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         // kernel over the class-0 tiles; the other baselines: per-tile kernel on a subset.
         // J_0 S J_0^H in the Hermitian form the tile-pair kernel reads (4 values per entry).
         DevBuf &coh0 = scratch.coh0;
-        e = coh0.reserve((size_t)n * ctx.nchan_pad * 4 * sizeof(double));
+        // (With the 8 channels past the last row that the kernel may read.)
+        e = coh0.reserve(((size_t)n * ctx.nchan_pad * 4 + 8 * 4) * sizeof(double));
         if (e != hipSuccess) return e;
         BeamDesc b0 = ctx.beam;
         b0.uniform_row = ctx.class_row0;
@@ -236,6 +237,8 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.tile_map = ctx.d_g0_tiles;
         t.ntiles_bl = ctx.ntiles;
         t.chunks = ctx.chunks;
+        t.narrow = ctx.narrow;
+        t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
         if (ev0 != nullptr) (void)hipEventRecord(ev0, stream);
         e = launch_direct_tiled(kind, t, stream);
         // Pairs of a class-r tile with a class-0 tile. With a table of J_r S J_0^H for every
@@ -352,6 +355,8 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.vis32 = vis32;
         t.vis64 = vis64;
         t.chunks = ctx.chunks;
+        t.narrow = ctx.narrow;
+        t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
         e = launch_direct_tiled(kind, t, stream);
     } else if (g_direct_variant != 1 && kind == KIND_SHAPELET) {
         ShapeletChanArgs s;
@@ -429,6 +434,8 @@ const char *abi_ctx(AbiState &st, const Addresses *a, const UVW *d_uvws, const J
     SM_TRY(hipMemcpy(st.freqs_pad.ptr, st.h_freqs_pad.data(), sizeof(double) * ctx.nchan_pad, hipMemcpyHostToDevice));
     ctx.d_freqs_pad = st.freqs_pad.as<double>();
     ctx.even = chunks_even(st.h_freqs_pad.data(), ctx.nchan);
+    ctx.even16 = chunks_even_width(st.h_freqs_pad.data(), ctx.nchan, 16);
+    ctx.narrow = narrow_steps(st.h_freqs_pad.data(), ctx.nchan);
     ctx.d_uvw = d_uvws;
     ctx.d_sbf = a->d_shapelet_basis_values;
     ctx.ntiles = ntiles;

@@ -14,6 +14,7 @@
 // Blocks are remapped so that all baseline blocks of a channel chunk land on the same XCD
 // and share that XCD's L2 copy of the chunk's coherency rows.
 #include <algorithm>
+#include <cmath>
 
 #include "sm_internal.h"
 #include "sm_jones.h"
@@ -421,13 +422,21 @@ std::vector<int2> even_chunks(const double *freqs, int nchan, int width) {
 // 8 (and with it 4) and 6; otherwise each channel gets its own sincos/exp. Evaluated on the
 // host copy of the padded frequencies.
 bool chunks_even(const double *freqs, int nchan) {
-    for (const int w : {SM_NCH, 6}) {
-        for (int f0 = 0; f0 < nchan; f0 += w) {
-            const double d = freqs[f0 + 1] - freqs[f0];
-            for (int k = 2; k < w && f0 + k < nchan; ++k)
-                if (freqs[f0 + k] != freqs[f0] + (double)k * d) return false;
-        }
+    return chunks_even_width(freqs, nchan, SM_NCH) && chunks_even_width(freqs, nchan, 6);
+}
+
+bool chunks_even_width(const double *freqs, int nchan, int width) {
+    for (int f0 = 0; f0 < nchan; f0 += width) {
+        const double d = freqs[f0 + 1] - freqs[f0];
+        for (int k = 2; k < width && f0 + k < nchan; ++k)
+            if (freqs[f0 + k] != freqs[f0] + (double)k * d) return false;
     }
+    return true;
+}
+
+bool narrow_steps(const double *freqs, int nchan) {
+    for (int f = 0; f < nchan; ++f)
+        if (!(std::fabs(freqs[f + 1] - freqs[f]) <= 1e-3 * freqs[f])) return false;
     return true;
 }
 

@@ -1,14 +1,15 @@
 // Faster FP64 direct kernels for the common case: one beam shared by every tile (or no
 // beam) and evenly spaced channels.
 //
-// k_direct_tiled (points, Gaussians): a block owns a 16 x 16 block of tile pairs and one
-// chunk of NCH channels (kTiledNchPoint, kTiledNchGaussian). The baseline phase factorises over antennas,
+// k_tiles_mfma (points, Gaussians): a block owns up to 16 x 16 tile pairs and one chunk of
+// channels. The baseline phase factorises over antennas,
 //   e^{i theta_pq f/c} = e^{i theta_p f/c} e^{-i theta_q f/c},  theta_t = u_t L + v_t M + w_t N,
 // (baseline uvw = tile1 - tile2, mdbook/src/defs/coords.md), so per component the block
-// evaluates the start phasor and the per-channel step for its 32 tiles into LDS (64
-// sincos shared by 256 baselines instead of 512), and each lane forms its baseline's
-// phasors with two complex products. Diagonal tile blocks are paired so a block keeps 240
-// of its 256 lanes busy.
+// evaluates the phasors of its 32 tiles (middle channel and channel step) into LDS (64
+// sincos shared by 256 baselines instead of 512), each lane forms its baseline's phasors from
+// them, and the FP64 matrix cores multiply them by the coherencies. Diagonal tile blocks are
+// paired so that 240 of 256 pairs are wanted ones. k_direct_tiled is the precision path's FP32
+// form for Gaussians, which keeps the products on the vector ALUs.
 //
 // k_shapelet_chan (shapelets): one wave per baseline, one lane per channel. The basis-table
 // positions x_pos = k f + 5000 of neighbouring channels fall in the same or adjacent table
@@ -26,16 +27,10 @@ constexpr int kWin = 32;  // shapelet table window per wave and axis, cells
 constexpr int kRows = 16; // shapelet table rows staged per wave
 constexpr int kWinPair = 24;  // shapelet table window per wave and axis of the two-channel kernel, cells
 constexpr int kCT = 32;   // components per LDS stage
-// Channels per lane in k_direct_tiled. Fewer channels hold fewer
-// accumulators (more waves per SIMD) but share each component's scalar coherency loads, phasor
-// reads and products, and a Gaussian's three exps, over fewer channels. Measured per C2 launch
-// (768 channels) with the Hermitian coherency table: points 21.4 ms with 4 channels, 19.4 ms
-// with 6, 17.4 ms with 8 (167 VGPRs, 3 waves per SIMD); Gaussians 15.1 ms with 4, 12.6 ms with 6
-// (161 VGPRs), 12.5 ms with 8. The FP32 Gaussians keep 6 (see launch_direct_tiled).
-constexpr int kTiledNchPoint = 8;
+// Channels per lane in k_direct_tiled (FP32 Gaussians). Measured per timestep of 256 tiles,
+// 384 channels and 10 000 Gaussians: 78.4 ms with 4, 76.2 ms with 6 (142 VGPRs), 115.9 ms with 8.
 constexpr int kTiledNchGaussian = 6;
-static_assert(kTiledNchPoint <= SM_NCH && kTiledNchGaussian <= SM_NCH,
-              "the padded channel count covers whole chunks of SM_NCH channels");
+static_assert(kTiledNchGaussian <= SM_NCH, "the padded channel count covers whole chunks of SM_NCH channels");
 
 // The kernels below come in two arithmetic types T. double: the FP64 direct kernels. float:
 // the precision path's kernels, in which the phases, their range reduction mod 2 pi, the table
@@ -277,6 +272,271 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
     }
 }
 
+// ------------------------------------------------------------------ FP64 tile pairs on MFMA
+// One visibility is V^e = sum_c C^e_c z_c over the four real coefficients e of the Hermitian
+// coherency: a 4 x K by K x N product with K the components and N the real and imaginary
+// parts of the baselines' phasors. v_mfma_f64_4x4x4 computes four such 4 x 4 x 4 blocks: lane l
+// supplies A = C^{l % 4} of component l / 16 and B = z of component l / 16 and baseline l % 16,
+// and accumulates e = l / 16 of baseline l % 16. The vector ALUs only form z.
+
+// z of the chunk's channels from the middle one outwards in both directions: evenly spaced
+// channels obey z_{k+1} = 2 cos(delta) z_k - z_{k-1}, one FMA per part, and starting in the middle
+// keeps the recurrence's error growth to (NCH / 2)^2 roundings. (a0, b0) are the tiles' phasors at
+// channel NCH / 2 - 1, (a1, b1) at one channel step's frequency: the step's small phase carries a
+// small rounding. Two neighbouring channels' phasors instead would have their independent phase
+// roundings, 1e-12 at 1e4 rad, extrapolated over the chunk.
+template <int NCH>
+__device__ __forceinline__ void chunk_phasors(double2 a0, double2 a1, double2 b0, double2 b1, double (&zr)[NCH],
+                                              double (&zi)[NCH]) {
+    constexpr int m = NCH / 2 - 1;
+    zr[m] = fma(a0.x, b0.x, a0.y * b0.y);
+    zi[m] = fma(a0.y, b0.x, -(a0.x * b0.y));
+    const double rr = fma(a1.x, b1.x, a1.y * b1.y), ri = fma(a1.y, b1.x, -(a1.x * b1.y));
+    zr[m + 1] = fma(zr[m], rr, -(zi[m] * ri));
+    zi[m + 1] = fma(zr[m], ri, zi[m] * rr);
+    const double c2 = 2.0 * rr;
+#pragma unroll
+    for (int k = m + 2; k < NCH; ++k) {
+        zr[k] = fma(c2, zr[k - 1], -zr[k - 2]);
+        zi[k] = fma(c2, zi[k - 1], -zi[k - 2]);
+    }
+#pragma unroll
+    for (int k = m - 1; k >= 0; --k) {
+        zr[k] = fma(c2, zr[k + 1], -zr[k + 2]);
+        zi[k] = fma(c2, zi[k + 1], -zi[k + 2]);
+    }
+}
+
+// What bounds it: FP64 issue. The matrix and vector FP64 instructions share one unit (16 FMAs
+// and 16 MFMAs per wave, measured: 36 and 111 ns apart, 141 ns together), which sustains 75
+// TFLOP/s on this MFMA against 62 on FMAs (the clock falls to 2.07 GHz under FMAs). A component
+// visibility's 8 accumulating FMAs become 2/64 MFMAs and the phasor's 4-instruction rotation the 2
+// FMAs of the recurrence. At 128 tiles, 768 channels: 5600 points 18.0 -> 13.7 ms (MFMA 53% and
+// other VALU 34% of the cycles, at 2.05 GHz), 2000 Gaussians 12.9 -> 7.8 ms (their exponentials
+// through table_exp: 10.1 -> 8.6 ms). Two waves per SIMD: the accumulators take 128 VGPRs. Four
+// waves of half the accumulators spill and run slower (15.5 and 23.7 ms).
+//
+// A block owns R = NG * WR rows of one 16 x 16 tile-pair block and one chunk of at most NCH
+// channels. WR waves split the rows (NG each); WC waves split the components (each takes every
+// WC-th group of four of a stage), their sums meeting in LDS at the end. A chunk's coherencies are
+// read NCH wide whatever its count (TiledArgs::coh); what the extra channels accumulate is dropped.
+template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW>
+__global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs a) {
+    constexpr int R = NG * WR, SUB = kTG / R, NT = 64 * WR * WC;
+    static_assert(kCT % (4 * WC) == 0, "a stage is whole groups of four components per wave");
+    struct Stage {
+        double2 p0[kCT][32], p1[kCT][32];  // tile phasors: the chunk's middle channel, one channel step
+        double c[kCT][NCH * 4 + 4];        // coherencies; the padding puts components on distinct banks
+    };
+    union Lds {
+        Stage st;
+        double red[WC > 1 ? WC : 1][NG][2][64];
+    };
+    __shared__ Lds L;
+    __shared__ double2 s_uv[32];
+    __shared__ double s_w[32];
+    __shared__ double2 s_sc[64];
+    __shared__ double s_exp[64];
+    const int total = a.npairs * a.nchunks * SUB;
+    int b = blockIdx.x;
+    if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
+    const int chunk = b / (a.npairs * SUB);
+    int f0, cnt;
+    chunk_range<NCH>(a.chunks, chunk, a.nchan, f0, cnt);
+    const int rem = b - chunk * (a.npairs * SUB);
+    const int row0 = (rem % SUB) * R;
+    const int4 pr = a.pairs[rem / SUB];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int wr = wave % WR, wc = wave / WR;
+    const int cq = lane & 15, ck = lane >> 4;
+    if (tid < 32) {
+        const int g = tid < 16 ? pr.y : pr.z;
+        int t = g * kTG + (tid & 15);
+        if (g < 0 || t >= a.ntiles) t = 0;
+        s_uv[tid] = make_double2(a.tile_uvw[3 * t], a.tile_uvw[3 * t + 1]);
+        s_w[tid] = a.tile_uvw[3 * t + 2];
+    }
+    if (tid < 64) {
+        s_sc[tid] = make_double2(kSinCos32[2 * tid], kSinCos32[2 * tid + 1]);
+        if (KIND == KIND_GAUSSIAN) s_exp[tid] = kExp64[tid];
+    }
+    // Tile slots of each (row, column): off-diagonal blocks pair group y's tile r with group
+    // z's tile cq; diagonal blocks hold group y's pairs above the diagonal and group z's below.
+    int sp[NG], sq[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int r = row0 + wr * NG + g;
+        const bool lower = pr.x != 0 && r > cq;
+        sp[g] = lower ? 16 + cq : r;
+        sq[g] = pr.x == 0 ? 16 + cq : (lower ? 16 + r : cq);
+    }
+    // Slots this block reads: its rows and group z's columns, or (diagonal) all of them.
+    const int nslot = pr.x == 0 ? R + 16 : 32;
+    __syncthreads();
+    const double *__restrict__ freqs = a.freqs;
+    const double F0 = freqs[f0];
+    const double DF = freqs[f0 + 1] - F0;
+    constexpr int m = NCH / 2 - 1;
+    const double fm0 = (F0 + m * DF) / SM_VEL_C, fm1 = DF / SM_VEL_C;
+    const double4 *__restrict__ lmn4 = a.lmn;
+    const double4 *__restrict__ shape = a.shape;
+    const double *__restrict__ coh = a.coh + (size_t)f0 * 4;
+    const size_t cstride = (size_t)a.nchan_pad * 4;
+    const double qmin = -800.0 / (F0 * F0), q0 = F0 * F0, q1 = DF * (2.0 * F0 + DF), q2 = 2.0 * DF * DF;
+
+    double acc[NCH][NG][2];
+#pragma unroll
+    for (int k = 0; k < NCH; ++k)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) acc[k][g][0] = acc[k][g][1] = 0.0;
+
+    for (int c0 = 0; c0 < a.ncomp; c0 += kCT) {
+        const int nc = a.ncomp - c0 < kCT ? a.ncomp - c0 : kCT;
+        const int nc4 = (nc + 3) & ~3;  // components past the last are staged as 0
+        for (int e = tid; e < nc4 * (NCH * 2); e += NT) {
+            const int cc = e / (NCH * 2), i = e % (NCH * 2);
+            double2 v = make_double2(0.0, 0.0);
+            if (cc < nc) v = reinterpret_cast<const double2 *>(coh + (size_t)(c0 + cc) * cstride)[i];
+            *reinterpret_cast<double2 *>(&L.st.c[cc][2 * i]) = v;
+        }
+#pragma unroll 2
+        for (int e = tid; e < nc4 * nslot; e += NT) {
+            const int cc = e / nslot, i = e - cc * nslot;
+            const int slot = pr.x != 0 ? i : (i < R ? row0 + i : i - R + 16);
+            double s0 = 0.0, c0_ = 0.0, s1 = 0.0, c1 = 0.0;
+            if (cc < nc) {
+                const double4 l = lmn4[c0 + cc];
+                const double2 uv = s_uv[slot];
+                const double th = uv.x * l.x + uv.y * l.y + s_w[slot] * l.z;
+                table_sincos(th * fm0, reinterpret_cast<const double *>(s_sc), s0, c0_);
+                table_sincos(th * fm1, reinterpret_cast<const double *>(s_sc), s1, c1);
+            }
+            L.st.p0[cc][slot] = make_double2(c0_, s0);
+            L.st.p1[cc][slot] = make_double2(c1, s1);
+        }
+        __syncthreads();
+#pragma unroll 2
+        for (int cs = 4 * wc; cs < nc; cs += 4 * WC) {
+            const int cc = cs + ck;
+            double A[NCH];
+#pragma unroll
+            for (int k = 0; k < NCH; ++k) A[k] = L.st.c[cc][4 * k + (lane & 3)];
+            double4 sh = make_double4(0.0, 0.0, 0.0, 0.0);
+            if (KIND == KIND_GAUSSIAN) sh = shape[min(c0 + cc, a.ncomp - 1)];
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                double zr[NCH], zi[NCH];
+                chunk_phasors<NCH>(L.st.p0[cc][sp[g]], L.st.p1[cc][sp[g]], L.st.p0[cc][sq[g]], L.st.p1[cc][sq[g]], zr,
+                                   zi);
+                if (KIND == KIND_GAUSSIAN) {
+                    const double2 tp = s_uv[sp[g]], tq = s_uv[sq[g]];
+                    const double bu = tp.x - tq.x, bv = tp.y - tq.y;
+                    double qf = sh.x * (bu * bu) + sh.y * (bu * bv) + sh.z * (bv * bv);
+                    // Below qmin the envelope is 0 at every channel of the chunk (e^-800 underflows).
+                    qf = qf < qmin ? qmin : qf;
+                    double env = table_exp(qf * q0, s_exp);
+                    // Descending channels give a positive exponent; the cap keeps 0 * er at 0.
+                    double er = table_exp(NARROW ? qf * q1 : fmin(qf * q1, 700.0), s_exp);
+                    const double eg = NARROW ? small_exp(qf * q2) : table_exp(qf * q2, s_exp);
+#pragma unroll
+                    for (int k = 0; k < NCH; ++k) {
+                        zr[k] *= env;
+                        zi[k] *= env;
+                        env *= er;
+                        er *= eg;
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < NCH; ++k) {
+                    acc[k][g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(A[k], zr[k], acc[k][g][0], 0, 0, 0);
+                    acc[k][g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(A[k], zi[k], acc[k][g][1], 0, 0, 0);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    // Lane l holds (re, im) of coefficient l / 16 for baseline l % 16: lanes of A = sum Re(C_XY) z
+    // and B = sum Im(C_XY) z exchange them (lane ^ 48) for XY = A + i B and YX = A - i B, and each
+    // lane writes one of the visibility's four entries.
+    auto store = [&](int g, int k, double re, double im) {
+        const int r = row0 + wr * NG + g;
+        int p, q;
+        bool valid;
+        if (pr.x == 0) {
+            p = pr.y * kTG + r;
+            q = pr.z * kTG + cq;
+            valid = q < a.ntiles;
+        } else if (r < cq) {
+            p = pr.y * kTG + r;
+            q = pr.y * kTG + cq;
+            valid = q < a.ntiles;
+        } else {
+            p = pr.z * kTG + cq;
+            q = pr.z * kTG + r;
+            valid = r > cq && pr.z >= 0 && q < a.ntiles;
+        }
+        const double ore = __shfl_xor(re, 48), oim = __shfl_xor(im, 48);
+        double vr = re, vi = im;
+        if (ck == 1) {
+            vr = re - oim;
+            vi = im + ore;
+        } else if (ck == 2) {
+            vr = ore + im;
+            vi = oim - re;
+        }
+        if (!valid) return;
+        if (a.tile_map != nullptr) {
+            p = a.tile_map[p];
+            q = a.tile_map[q];
+        }
+        const size_t nt = a.tile_map != nullptr ? (size_t)a.ntiles_bl : (size_t)a.ntiles;
+        const size_t bl = (size_t)p * nt - (size_t)p * (p + 1) / 2 + (size_t)(q - p - 1);
+        const size_t o = (size_t)(f0 + k) * a.nbl + bl;
+        float2 *v32 = reinterpret_cast<float2 *>(&a.vis32[o]) + ck;
+        float2 t = *v32;
+        t.x += (float)vr;
+        t.y += (float)vi;
+        *v32 = t;
+        if (a.vis64 != nullptr) {
+            double2 *v64 = reinterpret_cast<double2 *>(&a.vis64[o]) + ck;
+            double2 d = *v64;
+            d.x += vr;
+            d.y += vi;
+            *v64 = d;
+        }
+    };
+    if (WC == 1) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g)
+#pragma unroll
+            for (int k = 0; k < NCH; ++k)
+                if (k < cnt) store(g, k, acc[k][g][0], acc[k][g][1]);
+    } else {
+        // The WC waves' sums of each channel, added in wave order by the first NG waves.
+        static_assert(WC == 1 || (WR == 1 && WC >= NG), "one row group per adding wave");
+#pragma unroll
+        for (int k = 0; k < NCH; ++k) {
+            if (k >= cnt) break;
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                L.red[wc][g][0][lane] = acc[k][g][0];
+                L.red[wc][g][1][lane] = acc[k][g][1];
+            }
+            __syncthreads();
+            if (wc < NG) {
+                double re = 0.0, im = 0.0;
+#pragma unroll
+                for (int w = 0; w < WC; ++w) {
+                    re += L.red[w][wc][0][lane];
+                    im += L.red[w][wc][1][lane];
+                }
+                store(wc, k, re, im);
+            }
+            __syncthreads();
+        }
+    }
+}
+
 // Tile-group pairs: off-diagonal (0, g0, g1) with g0 < g1, then diagonal groups paired from
 // both ends (1, g, G-1-g), the middle one alone (1, g, -1) when G is odd.
 std::vector<int4> tile_pairs(int ntiles) {
@@ -289,30 +549,64 @@ std::vector<int4> tile_pairs(int ntiles) {
     return out;
 }
 
+template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW>
+static hipError_t launch_tiles_form(TiledArgs a, hipStream_t stream) {
+    a.nchunks = chunk_count(a.chunks, NCH, a.nchan);
+    hipLaunchKernelGGL((k_tiles_mfma<KIND, NCH, NG, WR, WC, NARROW>),
+                       dim3((unsigned)(a.npairs * a.nchunks * (kTG / (NG * WR)))), dim3(64 * WR * WC), 0, stream, a);
+    return hipGetLastError();
+}
+
+// Which form: the one with the smallest rounds x time of a round. A round is as many blocks as
+// the 256 CUs hold at once; its time per component was measured on 128 tiles, 768 channels, 5600
+// points and 2000 Gaussians. Two row groups of 16 channels share a Gaussian's exponentials and
+// a phasor's set-up over the most channels (points 13.7 ms, Gaussians 7.8 ms; four row groups of 8
+// channels 13.7 and 8.3 ms). Splitting the components over eight waves costs 1.5 times that on a
+// full chip (21.3 and 11.8 ms; 4 channels 23.6 and 18.1 ms), but its blocks are 4 rows high: on 32
+// channels (72 blocks of the widest form) it takes 1.01 and 0.57 ms against 1.56 and 0.93 ms, and
+// on 2 channels, 4 wide, 13 us for 90 points against 32 us.
+template <int KIND, bool NARROW> static hipError_t launch_tiles(const TiledArgs &a, hipStream_t stream) {
+    constexpr bool g = KIND == KIND_GAUSSIAN;
+    struct Form {
+        int nch, sub, resident;
+        double us;  // per component and round
+    };
+    const Form forms[4] = {{16, 2, 512, g ? 0.554 : 0.348},
+                           {8, 1, 512, g ? 0.591 : 0.349},
+                           {8, 4, 256, g ? 0.109 : 0.0704},
+                           {4, 4, 512, g ? 0.168 : 0.0780}};
+    int best = -1;
+    double t_best = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        if (i == 0 && !a.even16) continue;
+        const long blocks = (long)a.npairs * forms[i].sub * chunk_count(a.chunks, forms[i].nch, a.nchan);
+        const double t = (double)((blocks + forms[i].resident - 1) / forms[i].resident) * forms[i].us;
+        if (best < 0 || t < t_best) {
+            best = i;
+            t_best = t;
+        }
+    }
+    switch (best) {
+    case 0: return launch_tiles_form<KIND, 16, 2, 4, 1, NARROW>(a, stream);
+    case 1: return launch_tiles_form<KIND, 8, 4, 4, 1, NARROW>(a, stream);
+    case 2: return launch_tiles_form<KIND, 8, 4, 1, 8, NARROW>(a, stream);
+    default: return launch_tiles_form<KIND, 4, 4, 1, 8, NARROW>(a, stream);
+    }
+}
+
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a_in, hipStream_t stream) {
     if (a_in.ncomp <= 0 || a_in.nbl <= 0 || a_in.nchan <= 0) return hipSuccess;
     TiledArgs a = a_in;
-    // FP32 Gaussians take 6 channels per lane too (142 VGPRs with the two-level accumulators,
-    // 3 waves per SIMD). Measured per C5 timestep: 78.4 ms with 4, 76.2 ms with 6, 115.9 ms
-    // with 8.
-    const int nch = kind == KIND_GAUSSIAN ? kTiledNchGaussian : kTiledNchPoint;
-    a.nchunks = chunk_count(a.chunks, nch, a.nchan);
-    const int total = a.npairs * a.nchunks;
     if (a.coh32 != nullptr) {
-        if (kind == KIND_GAUSSIAN)
-            hipLaunchKernelGGL((k_direct_tiled<KIND_GAUSSIAN, kTiledNchGaussian, float>), dim3(total), dim3(256), 0,
-                               stream, a);
-        else
-            hipLaunchKernelGGL((k_direct_tiled<KIND_POINT, kTiledNchPoint, float>), dim3(total), dim3(256), 0, stream,
-                               a);
-    } else if (kind == KIND_GAUSSIAN) {
-        hipLaunchKernelGGL((k_direct_tiled<KIND_GAUSSIAN, kTiledNchGaussian, double>), dim3(total), dim3(256), 0,
-                           stream, a);
-    } else {
-        hipLaunchKernelGGL((k_direct_tiled<KIND_POINT, kTiledNchPoint, double>), dim3(total), dim3(256), 0, stream,
-                           a);
+        if (kind != KIND_GAUSSIAN) return hipErrorInvalidValue;  // FP32 points take the MFMA point path
+        a.nchunks = chunk_count(a.chunks, kTiledNchGaussian, a.nchan);
+        hipLaunchKernelGGL((k_direct_tiled<KIND_GAUSSIAN, kTiledNchGaussian, float>), dim3(a.npairs * a.nchunks),
+                           dim3(256), 0, stream, a);
+        return hipGetLastError();
     }
-    return hipGetLastError();
+    return kind == KIND_GAUSSIAN ? (a.narrow ? launch_tiles<KIND_GAUSSIAN, true>(a, stream)
+                                             : launch_tiles<KIND_GAUSSIAN, false>(a, stream))
+                                 : launch_tiles<KIND_POINT, true>(a, stream);
 }
 
 // ------------------------------------------------------------------ pairs with own beams

@@ -210,13 +210,13 @@ struct SmModeller {
     std::vector<int> unique_tile_total;  // unique row -> total-array tile
     std::vector<int> freq_map;
     std::vector<double> ufreqs;
-    bool even = false;
+    bool even = false, narrow = false;
     // device
     DevBuf d_freqs, d_xyz, d_bl_tiles, d_bl_rows, d_tile_rows, d_freq_map, d_ufreqs, d_delays, d_gains, d_sbf;
     DevBuf d_udelays, d_ugains;  // the unique tiles' delays [n_utile][16] and gains [n_utile][32]
     DevBuf d_sbf32;  // the basis table in FP32 (precision path)
-    DevBuf d_chunks4, d_chunks6, d_chunks8;  // evenly spaced channel runs of at most 4, 6 and 8 channels
-    int nchunks4 = 0, nchunks6 = 0, nchunks8 = 0;
+    DevBuf d_chunks4, d_chunks6, d_chunks8, d_chunks16;  // evenly spaced runs of at most 4, 6, 8 and 16 channels
+    int nchunks4 = 0, nchunks6 = 0, nchunks8 = 0, nchunks16 = 0;
     DevBuf d_uvw, d_vis32, d_vis64, d_accum, d_tile_uvw, d_pairs;
     // split-precision point path
     DevBuf d_fblocks, d_fblock_of, d_fout, d_fscratch, d_fkbuf, d_fcohf, d_fmap;
@@ -506,6 +506,7 @@ extern "C" const char *sm_new(const SmObsParams *p, const SmComponent *comps, co
     m->freqs_pad.resize(m->nchan_pad);
     pad_freqs(m->freqs.data(), m->nchan, m->freqs_pad.data());
     m->even = chunks_even(m->freqs_pad.data(), m->nchan);
+    m->narrow = narrow_steps(m->freqs_pad.data(), m->nchan);
     if (p->num_flagged_tiles > 0) m->flagged.assign(p->flagged_tiles, p->flagged_tiles + p->num_flagged_tiles);
     m->pc_ra = p->phase_centre_ra;
     m->pc_dec = p->phase_centre_dec;
@@ -576,12 +577,15 @@ extern "C" const char *sm_new(const SmObsParams *p, const SmComponent *comps, co
         const std::vector<int2> c4 = even_chunks(m->freqs_pad.data(), m->nchan, 4);
         const std::vector<int2> c6 = even_chunks(m->freqs_pad.data(), m->nchan, 6);
         const std::vector<int2> c8 = even_chunks(m->freqs_pad.data(), m->nchan, 8);
+        const std::vector<int2> c16 = even_chunks(m->freqs_pad.data(), m->nchan, 16);
         m->nchunks4 = (int)c4.size();
         m->nchunks6 = (int)c6.size();
         m->nchunks8 = (int)c8.size();
+        m->nchunks16 = (int)c16.size();
         SM_NEW_TRY(upload(m->d_chunks4, c4));
         SM_NEW_TRY(upload(m->d_chunks6, c6));
         SM_NEW_TRY(upload(m->d_chunks8, c8));
+        SM_NEW_TRY(upload(m->d_chunks16, c16));
     }
     SM_NEW_TRY(m->d_sbf32.reserve(sizeof(float) * (size_t)SM_SBF_N * SM_SBF_L));
     SM_NEW_TRY(launch_to_f32((size_t)SM_SBF_N * SM_SBF_L, m->d_sbf.as<double>(), m->d_sbf32.as<float>(), 0));
@@ -796,7 +800,10 @@ static const char *model_timestep_device(SmModeller *m, double lst, double latit
     ctx.chunks.n6 = m->nchunks6;
     ctx.chunks.c8 = m->d_chunks8.as<int2>();
     ctx.chunks.n8 = m->nchunks8;
+    ctx.chunks.c16 = m->d_chunks16.as<int2>();
+    ctx.chunks.n16 = m->nchunks16;
     ctx.even = true;
+    ctx.narrow = m->narrow;
     ctx.d_uvw = uvw;
     ctx.d_sbf = m->d_sbf.as<double>();
     ctx.d_tile_uvw = tile_uvw;

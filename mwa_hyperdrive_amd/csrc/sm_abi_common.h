@@ -29,6 +29,8 @@ struct ModelCtx {
     const double *d_freqs_pad = nullptr;
     bool even = false;   // every chunk evenly spaced (always, with chunk tables)
     ChunkTabs chunks;    // channel chunks of evenly spaced runs, or null (fixed chunks)
+    bool even16 = false; // fixed chunks of 16 channels are evenly spaced (chunk tables need no such test)
+    bool narrow = false; // every channel step at most a thousandth of its frequency (narrow_steps)
     const UVW *d_uvw = nullptr;
     const double *d_sbf = nullptr;
     BeamDesc beam{};

@@ -60,9 +60,9 @@ struct BeamDesc {
     int row0 = -1;
 };
 
-// Channel chunks of the direct kernels. With tables: runs of at most 4 (c4), 6 (c6) or 8 (c8)
-// evenly spaced channels, (first channel, count), so that a flagged channel only shortens
-// the runs around it; every chunk is evenly spaced. Null tables: fixed chunks of 4, 6 or 8
+// Channel chunks of the direct kernels. With tables: runs of at most 4 (c4), 6 (c6), 8 (c8) or
+// 16 (c16) evenly spaced channels, (first channel, count), so that a flagged channel only shortens
+// the runs around it; every chunk is evenly spaced. Null tables: fixed chunks of 4, 6, 8 or 16
 // consecutive channels, evenly spaced or not. A chunk reads up to 8 channels from its first
 // one, inside the padded channel count (pad_channels adds 8).
 struct ChunkTabs {
@@ -72,24 +72,26 @@ struct ChunkTabs {
     int n6 = 0;
     const int2 *c8 = nullptr;
     int n8 = 0;
+    const int2 *c16 = nullptr;
+    int n16 = 0;
 };
 
 // Runs of at most `width` channels f0, f0 + 1, ... with freqs[f0 + k] == freqs[f0] + k (freqs[f0 + 1]
 // - freqs[f0]) exactly, covering all nchan channels in order.
 std::vector<int2> even_chunks(const double *freqs, int nchan, int width);
 
-// Number of chunks of width nch (4, 6 or 8).
+// Number of chunks of width nch (4, 6, 8 or 16).
 __host__ __device__ inline int chunk_count(const ChunkTabs &t, int nch, int nchan) {
-    const int2 *tab = nch == 4 ? t.c4 : (nch == 6 ? t.c6 : t.c8);
-    if (tab != nullptr) return nch == 4 ? t.n4 : (nch == 6 ? t.n6 : t.n8);
+    const int2 *tab = nch == 4 ? t.c4 : (nch == 6 ? t.c6 : (nch == 8 ? t.c8 : t.c16));
+    if (tab != nullptr) return nch == 4 ? t.n4 : (nch == 6 ? t.n6 : (nch == 8 ? t.n8 : t.n16));
     return (nchan + nch - 1) / nch;
 }
 
 // First channel and channel count of chunk `chunk` of width NCH.
 template <int NCH>
 __device__ __forceinline__ void chunk_range(const ChunkTabs &t, int chunk, int nchan, int &f0, int &cnt) {
-    static_assert(NCH == 4 || NCH == 6 || NCH == 8, "chunk tables exist for widths 4, 6 and 8");
-    const int2 *tab = NCH == 4 ? t.c4 : (NCH == 6 ? t.c6 : t.c8);
+    static_assert(NCH == 4 || NCH == 6 || NCH == 8 || NCH == 16, "chunk tables exist for widths 4, 6, 8 and 16");
+    const int2 *tab = NCH == 4 ? t.c4 : (NCH == 6 ? t.c6 : (NCH == 8 ? t.c8 : t.c16));
     if (tab != nullptr) {
         const int2 c = tab[chunk];
         f0 = c.x;
@@ -179,6 +181,10 @@ hipError_t launch_coherency(int ncomp, int nchan, int nchan_pad, const double *d
                             BeamDesc beam, bool apply_beam, double *d_coh, hipStream_t stream, bool hermitian = false);
 hipError_t launch_direct(Kind kind, bool per_tile, bool even, const DirectArgs &a, hipStream_t stream);
 bool chunks_even(const double *freqs_padded, int nchan);
+// Whether every fixed chunk of `width` channels is evenly spaced.
+bool chunks_even_width(const double *freqs_padded, int nchan, int width);
+// Whether every channel's step to the next is at most a thousandth of its frequency.
+bool narrow_steps(const double *freqs_padded, int nchan);
 hipError_t launch_autos(int ntiles, int nchan, int ncomp, const double *d_coh, int nchan_pad, BeamDesc beam,
                         bool coh_has_beam, JonesF32 *vis32, JonesF64 *vis64, double *accum64, bool demote_now,
                         hipStream_t stream);

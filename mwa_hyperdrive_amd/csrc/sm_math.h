@@ -122,10 +122,60 @@ SM_HD inline void table_sincos(double x, const double *tab, double &s, double &c
     c = fma(C, cr, -(S * sr));
 }
 
+// 2^(j / 64) for j = 0 .. 63, each rounded to nearest from a 60-digit evaluation.
+#define SM_EXP64_TABLE \
+    1.0, 1.0108892860517005, 1.0218971486541166, 1.0330248790212284, \
+    1.0442737824274138, 1.0556451783605572, 1.0671404006768237, 1.0787607977571199, \
+    1.0905077326652577, 1.102382583307841, 1.1143867425958924, 1.1265216186082418, \
+    1.1387886347566916, 1.1511892299529827, 1.1637248587775775, 1.1763969916502812, \
+    1.189207115002721, 1.202156731452703, 1.215247359980469, 1.22848053610687, \
+    1.241857812073484, 1.255380757024691, 1.2690509571917332, 1.2828700160787783, \
+    1.2968395546510096, 1.3109612115247644, 1.3252366431597413, 1.339667524053303, \
+    1.3542555469368927, 1.3690024229745905, 1.383909881963832, 1.3989796725383112, \
+    1.4142135623730951, 1.42961333839197, 1.4451808069770467, 1.460917794180647, \
+    1.4768261459394993, 1.4929077282912648, 1.5091644275934228, 1.5255981507445384, \
+    1.5422108254079407, 1.559004400237837, 1.5759808451078865, 1.593142151342267, \
+    1.6104903319492543, 1.6280274218573478, 1.645755478153965, 1.6636765803267364, \
+    1.681792830507429, 1.7001063537185235, 1.718619298122478, 1.7373338352737062, \
+    1.7562521603732995, 1.7753764925265212, 1.7947090750031072, 1.8142521755003989, \
+    1.8340080864093424, 1.8539791250833855, 1.8741676341103, 1.8945759815869656, \
+    1.9152065613971474, 1.9360617934922943, 1.9571441241754002, 1.978456026387951
+
+// FP64 e^x with a table-driven reduction (P. T. P. Tang, "Table-driven implementation of the
+// exponential function in IEEE floating-point arithmetic", ACM TOMS 15, 1989):
+// x = k ln2/64 + r with |r| <= ln2/128 (1 + eps), e^x = 2^(k >> 6) T[k mod 64] e^r with the
+// Taylor series of e^r to r^5 (remainder below 4e-17). ln2/64 is split in two doubles, both and
+// 64/ln2 rounded from 60 digits. Underflows to 0; x below -800 or above 700 is outside its range
+// (a NaN gives NaN). About 17 instructions.
+SM_HD inline double table_exp(double x, const double *tab) {
+    const double k = rint(x * 92.33248261689366);
+    double r = fma(-k, 0.010830424696249145, x);
+    r = fma(-k, 3.623510646634843e-19, r);
+    double p = 0.008333333333333333;
+    p = fma(p, r, 0.041666666666666664);
+    p = fma(p, r, 0.16666666666666666);
+    p = fma(p, r, 0.5);
+    p = fma(p * r, r, r);
+    const int i = (int)k;
+    const double t = tab[i & 63];
+    return ldexp(fma(t, p, t), i >> 6);
+}
+
+// e^x for |x| <= 2e-3: the Taylor series to x^5 (remainder below 1e-19).
+SM_HD inline double small_exp(double x) {
+    double p = 0.008333333333333333;
+    p = fma(p, x, 0.041666666666666664);
+    p = fma(p, x, 0.16666666666666666);
+    p = fma(p, x, 0.5);
+    p = fma(p, x, 1.0);
+    return fma(p, x, 1.0);
+}
+
 #ifdef __HIPCC__
 // The device copy of SM_SINCOS32_TABLE for table_sincos, one per translation unit; 16-byte
 // aligned, so a lane reads its (sin, cos) pair in one load.
 [[maybe_unused]] static __device__ const double kSinCos32[128] __attribute__((aligned(16))) = {SM_SINCOS32_TABLE};
+[[maybe_unused]] static __device__ const double kExp64[64] = {SM_EXP64_TABLE};
 #endif
 
 }  // namespace sm

@@ -18,7 +18,8 @@ struct TiledArgs {
     // The Hermitian form of the coherency table, [ncomp][nchan_pad][4] = (Re XX, Re XY, Im XY,
     // Re YY) of J S J^H (launch_coherency with `hermitian`). Valid because the same J stands on
     // both sides (one shared beam, or class 0's beam for pairs of two class-0 tiles) and S is
-    // Hermitian, so XX and YY are real and YX = conj(XY).
+    // Hermitian, so XX and YY are real and YX = conj(XY). Kernels read 16 channels from a chunk's
+    // first one: the buffer holds at least 8 more channels after the last row.
     const double *coh;
     // FP32 arithmetic (phases and their range reduction still FP64): the same table in FP32.
     // Null selects the FP64 kernels.
@@ -30,6 +31,11 @@ struct TiledArgs {
     const int *tile_map = nullptr;
     int ntiles_bl = 0;
     ChunkTabs chunks;  // channel chunks; the fixed chunks must then be evenly spaced
+    // Every chunk's channel step is at most a thousandth of its first frequency (narrow_steps):
+    // a Gaussian's second envelope ratio is then within 2e-3 of 1.
+    bool narrow = false;
+    // Chunks of 16 channels are evenly spaced too (always with chunk tables).
+    bool even16 = false;
 };
 
 struct ShapeletChanArgs {
