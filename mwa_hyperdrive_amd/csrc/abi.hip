@@ -142,12 +142,13 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const bool shared_tiled = ctx.d_bl_subset == nullptr && g_direct_variant == 0 && kind != KIND_SHAPELET &&
                               !per_tile && ctx.even && ctx.d_tile_uvw != nullptr && ctx.d_pairs != nullptr &&
                               ctx.ntiles >= 2;
-    // Shared-beam shapelets on the two-channels-per-lane kernel read the Hermitian form too.
+    // Shared-beam shapelets read the Hermitian form too, in planes.
     const bool shared_shapelet =
         ctx.d_bl_subset == nullptr && g_direct_variant != 1 && kind == KIND_SHAPELET && !per_tile;
     const bool hermitian = shared_tiled || shared_shapelet;
     e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, ctx.beam, !per_tile, coh.as<double>(),
-                         stream, hermitian);
+                         stream,
+                         shared_shapelet ? COH_HERMITIAN_PLANES : (shared_tiled ? COH_HERMITIAN : COH_FULL));
     if (e != hipSuccess) return e;
     // Per-tile shapelets with beam-row classes: J_r S J_0^H per class for the channel-per-lane
     // kernel, when the table fits (otherwise the kernel forms J_p S J_q^H per visibility).
@@ -214,7 +215,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         BeamDesc b0 = ctx.beam;
         b0.uniform_row = ctx.class_row0;
         e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, b0, true, coh0.as<double>(), stream,
-                             true);
+                             COH_HERMITIAN);
         if (e == hipSuccess && f32) e = to_f32(scratch.coh0_32, coh_n / 2, coh0.as<double>(), stream);
         if (e != hipSuccess) return e;
         TiledArgs t;
@@ -365,6 +366,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         s.nchan_pad = ctx.nchan_pad;
         s.ncomp = n;
         s.ngroups = (ctx.nchan + 63) / 64;
+        s.step = ctx.step;
         s.freqs = ctx.d_freqs_pad;
         s.uvw = ctx.d_uvw;
         s.lmn = in.lmn;
@@ -436,6 +438,7 @@ const char *abi_ctx(AbiState &st, const Addresses *a, const UVW *d_uvws, const J
     ctx.even = chunks_even(st.h_freqs_pad.data(), ctx.nchan);
     ctx.even16 = chunks_even_width(st.h_freqs_pad.data(), ctx.nchan, 16);
     ctx.narrow = narrow_steps(st.h_freqs_pad.data(), ctx.nchan);
+    ctx.step = mean_step(st.h_freqs_pad.data(), ctx.nchan);
     ctx.d_uvw = d_uvws;
     ctx.d_sbf = a->d_shapelet_basis_values;
     ctx.ntiles = ntiles;

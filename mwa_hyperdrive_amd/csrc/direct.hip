@@ -24,18 +24,27 @@ namespace sm {
 
 // ------------------------------------------------------------------ coherency table
 // coh[c][f] = J S J^H (one shared beam row) or S; S from the power-law / curved-power-law
-// parameters at 150 MHz or the list table (src/gpu/model.cu:16-28,137-167). With `hermitian`,
-// 4 values per entry instead of 8: Re XX, Re XY, Im XY, Re YY (the tile-pair kernels' form;
-// J S J^H with the same J on both sides is Hermitian, as S is).
+// parameters at 150 MHz or the list table (src/gpu/model.cu:16-28,137-167). The Hermitian forms
+// hold 4 values per entry instead of 8, Re XX, Re XY, Im XY, Re YY (J S J^H with the same J on both
+// sides is Hermitian, as S is).
 __global__ void k_coherency(int ncomp, int nchan, int nchan_pad, const double *__restrict__ freqs, FluxBuckets fb,
-                            BeamDesc beam, int apply_beam, int hermitian, double *__restrict__ coh) {
+                            BeamDesc beam, int apply_beam, int form, double *__restrict__ coh) {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)ncomp * nchan_pad) return;
     const int c = (int)(idx / nchan_pad);
     const int f = (int)(idx % nchan_pad);
-    double *out = coh + idx * (hermitian ? 4 : 8);
+    double *out = coh + idx * (form == COH_FULL ? 8 : 4);
+    double *out2 = out + 2;  // the second half of the Hermitian form
+    if (form == COH_HERMITIAN_PLANES) {
+        out = coh + ((size_t)c * 2 * nchan_pad + f) * 2;
+        out2 = out + 2 * (size_t)nchan_pad;
+    }
     if (f >= nchan) {
-        for (int e = 0; e < (hermitian ? 4 : 8); ++e) out[e] = 0.0;
+        if (form == COH_FULL) {
+            for (int e = 0; e < 8; ++e) out[e] = 0.0;
+        } else {
+            out[0] = out[1] = out2[0] = out2[1] = 0.0;
+        }
         return;
     }
     const double freq = freqs[f];
@@ -68,11 +77,11 @@ __global__ void k_coherency(int ncomp, int nchan, int nchan_pad, const double *_
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = s[e];
     }
-    if (hermitian) {
+    if (form != COH_FULL) {
         out[0] = o[0];
         out[1] = o[2];
-        out[2] = o[3];
-        out[3] = o[6];
+        out2[0] = o[3];
+        out2[1] = o[6];
     } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = o[e];
@@ -152,12 +161,12 @@ hipError_t launch_class_coherency(int nclass, int ncomp, int nchan, int nchan_pa
 }
 
 hipError_t launch_coherency(int ncomp, int nchan, int nchan_pad, const double *d_freqs, FluxBuckets fb,
-                            BeamDesc beam, bool apply_beam, double *d_coh, hipStream_t stream, bool hermitian) {
+                            BeamDesc beam, bool apply_beam, double *d_coh, hipStream_t stream, CohForm form) {
     if (ncomp <= 0) return hipSuccess;
     const size_t n = (size_t)ncomp * nchan_pad;
     const unsigned blocks = (unsigned)((n + 255) / 256);
     hipLaunchKernelGGL(k_coherency, dim3(blocks), dim3(256), 0, stream, ncomp, nchan, nchan_pad, d_freqs, fb, beam,
-                       apply_beam ? 1 : 0, hermitian ? 1 : 0, d_coh);
+                       apply_beam ? 1 : 0, (int)form, d_coh);
     return hipGetLastError();
 }
 

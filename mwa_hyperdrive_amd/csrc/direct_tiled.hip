@@ -11,10 +11,11 @@
 // paired so that 240 of 256 pairs are wanted ones. k_direct_tiled is the precision path's FP32
 // form for Gaussians, which keeps the products on the vector ALUs.
 //
-// k_shapelet_chan (shapelets): one wave per baseline, one lane per channel. The basis-table
-// positions x_pos = k f + 5000 of neighbouring channels fall in the same or adjacent table
-// cells, so each coefficient's table reads coalesce across the wave instead of touching
-// 64 unrelated cache lines.
+// k_shapelets (shapelets, one beam or none): the coefficient sums are formed once per run of
+// channels within a cell of the basis table. k_shapelet_chan_tiles (per-tile beams): one wave per
+// baseline, one lane per channel; the basis-table positions x_pos = k f + 5000 of neighbouring
+// channels fall in the same or adjacent table cells, so each coefficient's table reads coalesce
+// across the wave instead of touching 64 unrelated cache lines.
 #include "sm_internal.h"
 #include "sm_jones.h"
 #include "sm_math.h"
@@ -25,7 +26,6 @@ namespace sm {
 constexpr int kTG = 16;   // tiles per group
 constexpr int kWin = 32;  // shapelet table window per wave and axis, cells
 constexpr int kRows = 16; // shapelet table rows staged per wave
-constexpr int kWinPair = 24;  // shapelet table window per wave and axis of the two-channel kernel, cells
 constexpr int kCT = 32;   // components per LDS stage
 // Channels per lane in k_direct_tiled (FP32 Gaussians). Measured per timestep of 256 tiles,
 // 384 channels and 10 000 Gaussians: 78.4 ms with 4, 76.2 ms with 6 (142 VGPRs), 115.9 ms with 8.
@@ -1399,297 +1399,6 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
     }
 }
 
-// Shared beam: one wave per baseline and 128 channels, two adjacent channels per lane
-// (channels 2 l and 2 l + 1 of the group on lane l). The table cells are read for both channels
-// at once: adjacent channels' positions differ by |k| df, below one cell (checked per component),
-// so both fall in cells i0 and i0 + 1 with i0 the lower of their two cells. The staged window
-// holds each cell's value and its difference to the next cell, formed once per component, and
-// the lane reads T[i0], T[i0 + 1] - T[i0] and T[i0 + 2] - T[i0 + 1] per axis and coefficient
-// (24 bytes for two channels, against 16 per channel reading two values). A channel in cell
-// i0 interpolates
-//   u = T[i0] + (T[i0+1] - T[i0]) w,
-// as the single-channel form does, and one in cell i0 + 1 takes
-//   u = (T[i0] + (T[i0+1] - T[i0])) + (T[i0+2] - T[i0+1]) w,
-// equal to T[i0+1] + (T[i0+2] - T[i0+1]) w up to the rounding of T[i0] + (T[i0+1] - T[i0]).
-// The coherency table is in the Hermitian form (Re XX, Re XY, Im XY, Re YY; J S J^H with one
-// beam on both sides), so each channel accumulates with 8 FMAs per component.
-
-// A staged basis-table cell: the value T[i] and the difference T[i + 1] - T[i].
-template <class T> struct __attribute__((aligned(2 * sizeof(T)))) CellTD {
-    T t, d;
-};
-
-template <class T>
-__device__ __forceinline__ void shapelet_pair(const ShapeletChanArgs &a) {
-    const int ngroups = (a.nchan + 127) / 128;
-    const int nbx = (a.nbl + 3) / 4;
-    const int total = nbx * ngroups;
-    int b = blockIdx.x;
-    if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
-    const int group = b / nbx;
-    const int bx = b - group * nbx;
-    const int lane = threadIdx.x & 63;
-    const int bl = bx * 4 + (int)(threadIdx.x >> 6);
-    if (bl >= a.nbl) return;  // whole wave; the kernel has no barriers
-    const int fa_raw = group * 128 + 2 * lane;
-    const bool valid_a = fa_raw < a.nchan, valid_b = fa_raw + 1 < a.nchan;
-    const int fa = valid_a ? fa_raw : a.nchan - 1;
-    const int fb = valid_b ? fa_raw + 1 : a.nchan - 1;
-    const double freq_a = a.freqs[fa], freq_b = a.freqs[fb];
-    const double fc_a = freq_a / SM_VEL_C, fc_b = freq_b / SM_VEL_C;
-    const UVW uvw = a.uvw[bl];
-    const PackedCoeff *__restrict__ packed = a.packed;
-    const T *__restrict__ sbf = pick<T>(a.sbf, a.sbf32);
-    const T *__restrict__ coh_t = pick<T>(a.coh, a.coh32);
-    // Per-wave windows of the basis table (kRows rows x kWinPair cells per axis), each cell
-    // holding T[i] and T[i + 1] - T[i]: 48 KB per block in FP64, so three blocks share a CU.
-    __shared__ CellTD<T> wx_lds[4][kRows][kWinPair], wy_lds[4][kRows][kWinPair];
-    const int wv = threadIdx.x >> 6;
-    // The wave's lowest and highest channel frequency and its largest step between a lane's
-    // two channels (channels past the last repeat it).
-    double fmin_w = fmin(freq_a, freq_b), fmax_w = fmax(freq_a, freq_b), dfmax_w = fabs(freq_b - freq_a);
-    for (int o = 32; o > 0; o >>= 1) {
-        fmin_w = fmin(fmin_w, __shfl_xor(fmin_w, o));
-        fmax_w = fmax(fmax_w, __shfl_xor(fmax_w, o));
-        dfmax_w = fmax(dfmax_w, __shfl_xor(dfmax_w, o));
-    }
-    // FP64 with the same step between the two channels on every lane (evenly spaced channels):
-    // channel b's phasor is channel a's turned by exp(i theta df / c), the turn formed once per
-    // component in the batch below, instead of a second phase reduction and sincos.
-    const double df_ref = __shfl(freq_b - freq_a, 0);
-    const bool rot = std::is_same<T, double>::value && __all(!valid_b || freq_b - freq_a == df_ref);
-    const double dfc_rot = df_ref / SM_VEL_C;
-    T acc[2][8], tot[2][8];
-#pragma unroll
-    for (int ch = 0; ch < 2; ++ch)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[ch][e] = tot[ch][e] = T(0);
-    const int blu = __builtin_amdgcn_readfirstlane(bl);
-    // Shapelet UVs: formed here from the baseline's tile XYZs and each component's (HA, Dec)
-    // when those are given; else read from bl_uv.
-    const bool uv_here = a.hadec != nullptr;
-    double x1 = 0, y1 = 0, z1 = 0, x2 = 0, y2 = 0, z2 = 0;
-    if (uv_here) {
-        const int2 t = a.bl_tiles[blu];
-        x1 = a.xyz[3 * t.x];
-        y1 = a.xyz[3 * t.x + 1];
-        z1 = a.xyz[3 * t.x + 2];
-        x2 = a.xyz[3 * t.y];
-        y2 = a.xyz[3 * t.y + 1];
-        z2 = a.xyz[3 * t.y + 2];
-    }
-    const double4 *__restrict__ hd4 = reinterpret_cast<const double4 *>(a.hadec);
-    // As in shapelet_chan: the wave-uniform per-component values, formed by lane l for
-    // component 64 q + l and read back by lane.
-    double th_lane = 0.0, xk_lane = 0.0, yk_lane = 0.0, rs_lane = 0.0, rc_lane = 1.0;
-    int wx_lane = 0, wy_lane = 0;
-    auto load_batch = [&](int q) {
-        const int cl = min((q << 6) + lane, a.ncomp - 1);
-        const double4 l = a.lmn[cl];
-        const double4 sh = a.shape[cl];
-        const double2 suv =
-            uv_here ? shapelet_uv(hd4[cl], x1, y1, z1, x2, y2, z2) : a.bl_uv[(size_t)cl * a.nbl + blu];
-        th_lane = uvw.u * l.x + uvw.v * l.y + uvw.w * l.z;
-        if (rot) sincos_phase(th_lane * dfc_rot, rs_lane, rc_lane);
-        const double xk = (suv.x * sh.x + suv.y * sh.y) * sh.z;
-        const double yk = (suv.x * sh.y - suv.y * sh.x) * sh.w;
-        const double xa = xk * fmin_w + SM_SBF_C, xb = xk * fmax_w + SM_SBF_C;
-        const double ya = yk * fmin_w + SM_SBF_C, yb = yk * fmax_w + SM_SBF_C;
-        const int ix0 = (int)fmin(fmax(floor(fmin(xa, xb)), 0.0), (double)(SM_SBF_L - 2));
-        const int ix1 = (int)fmin(fmax(floor(fmax(xa, xb)), 0.0), (double)(SM_SBF_L - 2));
-        const int iy0 = (int)fmin(fmax(floor(fmin(ya, yb)), 0.0), (double)(SM_SBF_L - 2));
-        const int iy1 = (int)fmin(fmax(floor(fmax(ya, yb)), 0.0), (double)(SM_SBF_L - 2));
-        xk_lane = xk;
-        yk_lane = yk;
-        wx_lane = ix0 | ((ix1 - ix0 + 2) << 16);
-        wy_lane = iy0 | ((iy1 - iy0 + 2) << 16);
-    };
-    int4 pr_next = a.prange[0];
-    for (int c = 0; c < a.ncomp; ++c) {
-        const int4 pr4 = pr_next;
-        pr_next = a.prange[c + 1 < a.ncomp ? c + 1 : c];
-        if ((c & 63) == 0) load_batch(c >> 6);
-        const int src = c & 63;
-        const double theta = readlane_f64(th_lane, src);
-        const double xk = readlane_f64(xk_lane, src), yk = readlane_f64(yk_lane, src);
-        const int wxp = __builtin_amdgcn_readlane(wx_lane, src), wyp = __builtin_amdgcn_readlane(wy_lane, src);
-        T zr[2], zi[2];
-        sincos_phase(theta * fc_a, zi[0], zr[0]);
-        if (rot) {
-            const double rs = readlane_f64(rs_lane, src), rc = readlane_f64(rc_lane, src);
-            zr[1] = (T)((double)zr[0] * rc - (double)zi[0] * rs);
-            zi[1] = (T)((double)zr[0] * rs + (double)zi[0] * rc);
-        } else {
-            sincos_phase(theta * fc_b, zi[1], zr[1]);
-        }
-        const double xpa = xk * freq_a + SM_SBF_C, xpb = xk * freq_b + SM_SBF_C;
-        const double ypa = yk * freq_a + SM_SBF_C, ypb = yk * freq_b + SM_SBF_C;
-        const double fxa = floor(xpa), fxb = floor(xpb), fya = floor(ypa), fyb = floor(ypb);
-        const int ixa = (int)fmin(fmax(fxa, 0.0), (double)(SM_SBF_L - 2));
-        const int ixb = (int)fmin(fmax(fxb, 0.0), (double)(SM_SBF_L - 2));
-        const int iya = (int)fmin(fmax(fya, 0.0), (double)(SM_SBF_L - 2));
-        const int iyb = (int)fmin(fmax(fyb, 0.0), (double)(SM_SBF_L - 2));
-        const T wxa = (T)(xpa - fxa), wxb = (T)(xpb - fxb), wya = (T)(ypa - fya), wyb = (T)(ypb - fyb);
-        const int xw = wxp >> 16, yw = wyp >> 16;
-        // One component's coherencies for both channels (Hermitian form, 4 values each).
-        T cq[2][4];
-        {
-            const T *s_a = coh_t + ((size_t)c * a.nchan_pad + fa) * 4;
-            const T *s_b = coh_t + ((size_t)c * a.nchan_pad + fb) * 4;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                cq[0][e] = s_a[e];
-                cq[1][e] = s_b[e];
-            }
-        }
-        T er[2], ei[2];
-        // Staged path: both windows, one extra cell for T[i0 + 2], fit the LDS copy, and the
-        // two channels of a lane are less than half a cell apart on both axes (so their cells
-        // differ by at most one, with a wide margin for rounding).
-        const bool near = fabs(xk) * dfmax_w < 0.5 && fabs(yk) * dfmax_w < 0.5;
-        if (near && xw + 1 <= kWinPair && yw + 1 <= kWinPair && pr4.w <= kRows) {
-            const int bx0 = wxp & 0xffff, by0 = wyp & 0xffff;
-            const int xs = xw + 1, ys = yw + 1;  // staged cells per axis
-            // As in shapelet_chan: lane -> (row lane >> lw, cell lane & (2^lw - 1)). A lane past
-            // the window or past row pr4.w - 1 reads an in-bounds cell that is never written; the
-            // last cell is at most SM_SBF_L, in the row or at the next row's first cell, and the
-            // difference it enters is only multiplied by a zero weight when outside the row.
-            // T[i + 1] comes from the next lane of the row; the difference formed with the next
-            // row's lane at cell 2^lw - 1 >= xs - 1 is never read (the loop reads differences
-            // at cells up to xs - 2).
-            const int wm = max(xs, ys);
-            const int lw = wm <= 4 ? 2 : (wm <= 8 ? 3 : (wm <= 16 ? 4 : 5));
-            const int rstep = 64 >> lw;
-            const int j = lane & ((1 << lw) - 1), rl = lane >> lw;
-            const int jxc = min(j, xs - 1), jyc = min(j, ys - 1);
-            static_assert(kRows + 16 < SM_SBF_N, "staged rows and the next row must exist in the basis table");
-            const unsigned ox = (unsigned)((rl * SM_SBF_L + bx0 + jxc) * sizeof(T));
-            const unsigned oy = (unsigned)((rl * SM_SBF_L + by0 + jyc) * sizeof(T));
-            const char *sbf_b = reinterpret_cast<const char *>(sbf);
-            constexpr int kBatch = 2;
-            for (int i0 = 0; i0 < pr4.w; i0 += kBatch * rstep) {
-                T tx[kBatch], ty[kBatch];
-#pragma unroll
-                for (int i = 0; i < kBatch; ++i) {
-                    const int base = i0 + i * rstep;
-                    const unsigned step = (unsigned)(base * SM_SBF_L * sizeof(T));
-                    if (base < pr4.w) {
-                        tx[i] = *reinterpret_cast<const T *>(sbf_b + (ox + step));
-                        ty[i] = *reinterpret_cast<const T *>(sbf_b + (oy + step));
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < kBatch; ++i) {
-                    const int base = i0 + i * rstep, r = base + rl;
-                    if (base < pr4.w) {  // wave-uniform: every lane takes part in the shuffles
-                        const T tx1 = __shfl_down(tx[i], 1), ty1 = __shfl_down(ty[i], 1);
-                        if (r < pr4.w) {
-                            if (j < xs) wx_lds[wv][r][j] = CellTD<T>{tx[i], tx1 - tx[i]};
-                            if (j < ys) wy_lds[wv][r][j] = CellTD<T>{ty[i], ty1 - ty[i]};
-                        }
-                    }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // Each channel's weights on (T[i0+1] - T[i0]) and (T[i0+2] - T[i0+1]).
-            const int ix0l = min(ixa, ixb), iy0l = min(iya, iyb);
-            const int jx = ix0l - bx0, jy = iy0l - by0;
-            const bool xa_lo = ixa == ix0l, xb_lo = ixb == ix0l, ya_lo = iya == iy0l, yb_lo = iyb == iy0l;
-            const T ax_a = xa_lo ? wxa : T(1), bx_a = xa_lo ? T(0) : wxa;
-            const T ax_b = xb_lo ? wxb : T(1), bx_b = xb_lo ? T(0) : wxb;
-            const T ay_a = ya_lo ? wya : T(1), by_a = ya_lo ? T(0) : wya;
-            const T ay_b = yb_lo ? wyb : T(1), by_b = yb_lo ? T(0) : wyb;
-#pragma unroll
-            for (int pt = 0; pt < 2; ++pt) {
-                const PackedCoeff *cp = packed + pr4.x + (pt ? pr4.y : 0);
-                const int cnt = pt ? pr4.z : pr4.y;
-                T acc_a = T(0), acc_b = T(0);
-#pragma unroll 4
-                for (int k = 0; k < cnt; ++k) {
-                    double val;
-                    int n1, n2;
-                    load_packed_uniform(cp + k, val, n1, n2);
-                    const CellTD<T> cx = wx_lds[wv][n1][jx], cy = wy_lds[wv][n2][jy];
-                    const T dx12 = wx_lds[wv][n1][jx + 1].d, dy12 = wy_lds[wv][n2][jy + 1].d;
-                    const T u_a = fma_t(dx12, bx_a, fma_t(cx.d, ax_a, cx.t));
-                    const T u_b = fma_t(dx12, bx_b, fma_t(cx.d, ax_b, cx.t));
-                    const T v_a = fma_t(dy12, by_a, fma_t(cy.d, ay_a, cy.t));
-                    const T v_b = fma_t(dy12, by_b, fma_t(cy.d, ay_b, cy.t));
-                    acc_a += ((T)val * u_a) * v_a;
-                    acc_b += ((T)val * u_b) * v_b;
-                }
-                (pt ? ei : er)[0] = acc_a;
-                (pt ? ei : er)[1] = acc_b;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        } else {
-            // Rare: one coefficient at a time from the table in memory, per channel.
-            const int ixs[2] = {ixa, ixb}, iys[2] = {iya, iyb};
-            const T wxs[2] = {wxa, wxb}, wys[2] = {wya, wyb};
-#pragma unroll
-            for (int ch = 0; ch < 2; ++ch) {
-#pragma unroll
-                for (int pt = 0; pt < 2; ++pt) {
-                    const PackedCoeff *cp = packed + pr4.x + (pt ? pr4.y : 0);
-                    const int cnt = pt ? pr4.z : pr4.y;
-                    T accp = T(0);
-#pragma unroll 1
-                    for (int k = 0; k < cnt; ++k) {
-                        double val;
-                        int n1, n2;
-                        load_packed_uniform(cp + k, val, n1, n2);
-                        const T *bxp = sbf + n1 * SM_SBF_L + ixs[ch], *byp = sbf + n2 * SM_SBF_L + iys[ch];
-                        const T u_value = bxp[0] + (bxp[1] - bxp[0]) * wxs[ch];
-                        const T v_value = byp[0] + (byp[1] - byp[0]) * wys[ch];
-                        accp += ((T)val * u_value) * v_value;
-                    }
-                    (pt ? ei : er)[ch] = accp;
-                }
-            }
-        }
-#pragma unroll
-        for (int ch = 0; ch < 2; ++ch) {
-            const T pr = zr[ch] * er[ch] - zi[ch] * ei[ch];
-            const T pi = zr[ch] * ei[ch] + zi[ch] * er[ch];
-            acc[ch][0] = fma_t(cq[ch][0], pr, acc[ch][0]);
-            acc[ch][1] = fma_t(cq[ch][0], pi, acc[ch][1]);
-            acc[ch][2] = fma_t(cq[ch][1], pr, acc[ch][2]);
-            acc[ch][3] = fma_t(cq[ch][1], pi, acc[ch][3]);
-            acc[ch][4] = fma_t(cq[ch][2], pr, acc[ch][4]);
-            acc[ch][5] = fma_t(cq[ch][2], pi, acc[ch][5]);
-            acc[ch][6] = fma_t(cq[ch][3], pr, acc[ch][6]);
-            acc[ch][7] = fma_t(cq[ch][3], pi, acc[ch][7]);
-        }
-        if ((c & 15) == 15) flush_stage(acc, tot);
-    }
-#pragma unroll
-    for (int ch = 0; ch < 2; ++ch) {
-        if (!(ch ? valid_b : valid_a)) continue;
-        const size_t o = (size_t)(ch ? fb : fa) * a.nbl + bl;
-        T s8[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s8[e] = two_level_sum(acc[ch][e], tot[ch][e]);
-        // XX, XY = A + i B, YX = A - i B, YY.
-        const T v[8] = {s8[0], s8[1], s8[2] - s8[5], s8[3] + s8[4], s8[2] + s8[5], s8[3] - s8[4], s8[6], s8[7]};
-        float *v32 = reinterpret_cast<float *>(&a.vis32[o]);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v32[e] += (float)v[e];
-        if (a.vis64 != nullptr) {
-            double *v64 = reinterpret_cast<double *>(&a.vis64[o]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v64[e] += (double)v[e];
-        }
-    }
-}
-
-// Shared beam.
-__global__ __launch_bounds__(256) void k_shapelet_chan(const ShapeletChanArgs a) { shapelet_pair<double>(a); }
-__global__ __launch_bounds__(256) void k_shapelet_chan32(const ShapeletChanArgs a) { shapelet_pair<float>(a); }
-
 // Per-tile beams: held to 128 VGPRs (4 waves per SIMD, a few spilled values) instead of the
 // 164 the compiler picks (3 waves). Measured on the 256-tile, 384-channel case: 129 -> 111 ms
 // per timestep.
@@ -1704,17 +1413,405 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     shapelet_chan<true, float>(a);
 }
 
+// Shapelets with one beam on both sides (Hermitian coherencies) or none. One lane per channel (SL
+// slots of 64 / LB channels), LB baselines per wave.
+//
+// A component's basis-table positions x(f) = xk f + 5000 and y(f) are linear in frequency and the
+// basis functions are interpolated linearly, so while both positions stay in one pair of table
+// cells the envelope sum_k c_k B_n1(x) B_n2(y) is the same bilinear function of the two
+// fractions, i.e. one quadratic in f. Along the band (x, y) walks monotonically through the
+// table, so the cell pairs it visits ("segments") are numbered by the cell edges crossed since the
+// lowest frequency, s = |ix - ixa| + |iy - iya|. Components are taken in batches of at most 32
+// segments; per batch the wave
+//   1. sums the coefficients once per segment and part (real, imaginary), one lane each, into the
+//      quadratic's three coefficients, in FP64,
+//   2. evaluates them at every channel (4 FMAs) with the phasor and the coherency.
+// Where an x and a y edge are crossed within rounding of one channel, the channel and the lane that
+// sums its segment may order them differently; the two bilinear forms then meet at that channel.
+// Positions outside the table, or more than kShSeg segments, take the per-channel sums.
+//
+// The values of the next components are formed by one lane each and read back from LDS. The phasor
+// is a sincos at the first slot, turned by the slots' common step by the recurrence
+// z_{k+1} = 2 cos(delta) z_k - z_{k-1} (unevenly spaced channels: a sincos each).
+//
+// Bound by step 1, whose reads are scattered (16 bytes per lane, about 40 cycles of the address
+// unit per wave instruction), and by the latency of step 2's chain at 3 - 4 waves per SIMD: of
+// 13.5 ms on 1400 components, 128 tiles and 384 channels of 80 kHz, 4.9 ms are coefficient sums
+// and 2.9 ms phasors. Summing the coefficients per channel, from table windows staged in LDS, took
+// 21.7 ms there, and 4.0 against 0.9 ms on 24 channels of 40 kHz. Slower in step 1: windows staged
+// in LDS (22 ms), the basis functions by their recurrence in registers (15.6 ms).
+constexpr int kShItems = 32;  // (component, baseline) pairs whose values are formed at a time
+constexpr int kShSeg = 64;    // segment quadratics per wave
+constexpr int kShCoef = 128;  // staged coefficients per wave
+
+struct __attribute__((aligned(16))) ShVal {
+    double xk, yk, theta, c2, rr, ri;
+    int ixa, iya;    // cells at the lowest frequency
+    int edges, off;  // edges crossed on x | on y << 16; segments of the pairs before this one
+    int4 coef;       // launch_pack_coeffs' range
+};
+
+// Basis-table position of frequency f, rounded alike everywhere.
+__device__ __forceinline__ double table_pos(double k, double f) { return fma(k, f, SM_SBF_C); }
+
+__device__ __forceinline__ int cell_of(double pos) {
+    return (int)fmin(fmax(floor(pos), 0.0), (double)(SM_SBF_L - 2));
+}
+
+// A table cell's value and its neighbour's, read together.
+struct __attribute__((packed, aligned(8))) CellPair {
+    double v, next;
+};
+
+template <class T, int SL, int LB, int WPS>
+__global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a) {
+    constexpr int LPB = 64 / LB, SPAN = SL * LPB, VC = kShItems / LB;
+    __shared__ ShVal s_val[4][kShItems];
+    __shared__ __attribute__((aligned(16))) T s_seg[4][kShSeg][6];
+    __shared__ PackedCoeff s_coef[4][kShCoef];
+    __shared__ double2 s_sc[64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (threadIdx.x < 64) s_sc[lane] = make_double2(kSinCos32[2 * lane], kSinCos32[2 * lane + 1]);
+    __syncthreads();
+    const double *sc_tab = reinterpret_cast<const double *>(s_sc);
+    const int ngroups = (a.nchan + SPAN - 1) / SPAN;
+    const int nbx = (a.nbl + 4 * LB - 1) / (4 * LB);
+    const int total = nbx * ngroups;
+    int b = blockIdx.x;
+    if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
+    const int group = b / nbx;
+    const int bl0 = ((b - group * nbx) * 4 + wv) * LB;  // the wave's first baseline
+    if (bl0 >= a.nbl) return;                         // whole wave; no barriers below
+    const int bsub = lane / LPB;  // this lane's baseline as a channel
+    const int ch0 = group * SPAN + (lane & (LPB - 1));
+    double freq[SL];
+    T tk[SL];
+#pragma unroll
+    for (int k = 0; k < SL; ++k) freq[k] = a.freqs[min(ch0 + k * LPB, a.nchan - 1)];
+    // The span's lowest and highest frequency, and whether its slots are one step apart.
+    double fmin_w = freq[0], fmax_w = freq[0];
+#pragma unroll
+    for (int k = 1; k < SL; ++k) {
+        fmin_w = fmin(fmin_w, freq[k]);
+        fmax_w = fmax(fmax_w, freq[k]);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        fmin_w = fmin(fmin_w, __shfl_xor(fmin_w, o));
+        fmax_w = fmax(fmax_w, __shfl_xor(fmax_w, o));
+    }
+    const double step = __shfl(freq[SL > 1 ? 1 : 0] - freq[0], 0);
+    bool rot = true;
+#pragma unroll
+    for (int k = 1; k < SL; ++k) rot = rot && (ch0 + k * LPB >= a.nchan || freq[k] - freq[k - 1] == step);
+    rot = __all(rot);
+    // Quadratics are in t = (f - fmin) / unit, t <= 1.
+    const double unit = fmax_w > fmin_w ? fmax_w - fmin_w : 1.0;
+#pragma unroll
+    for (int k = 0; k < SL; ++k) tk[k] = (T)((freq[k] - fmin_w) / unit);
+
+    const PackedCoeff *__restrict__ packed = a.packed;
+    const double *__restrict__ sbf = a.sbf;
+    const char *__restrict__ sbf_b = reinterpret_cast<const char *>(a.sbf);
+    const T *__restrict__ coh_t = pick<T>(a.coh, a.coh32);
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+
+    T acc[SL][8], tot[SL][8];
+#pragma unroll
+    for (int k = 0; k < SL; ++k)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[k][e] = tot[k][e] = T(0);
+
+    for (int c0 = 0; c0 < a.ncomp; c0 += VC) {
+        // Values of (component, baseline) pair `lane`, and the running count of segments.
+        int upto = 0;  // segments of the pairs up to and with this lane's
+        int coef_lo = 0, coef_hi = 0;
+        bool fast = true;
+        wave_sync();
+        if (lane < kShItems) {
+            const int c = min(c0 + lane / LB, a.ncomp - 1);
+            const int obl = min(bl0 + lane % LB, a.nbl - 1);
+            const int2 ot = a.bl_tiles != nullptr ? a.bl_tiles[obl] : make_int2(0, 0);
+            const UVW uvw = a.uvw[obl];
+            const double4 l = a.lmn[c], sh = a.shape[c];
+            const double4 *__restrict__ hd4 = reinterpret_cast<const double4 *>(a.hadec);
+            const double2 suv = a.hadec != nullptr
+                                    ? shapelet_uv(hd4[c], a.xyz[3 * ot.x], a.xyz[3 * ot.x + 1], a.xyz[3 * ot.x + 2],
+                                                  a.xyz[3 * ot.y], a.xyz[3 * ot.y + 1], a.xyz[3 * ot.y + 2])
+                                    : a.bl_uv[(size_t)c * a.nbl + obl];
+            ShVal v;
+            v.xk = (suv.x * sh.x + suv.y * sh.y) * sh.z;
+            v.yk = (suv.x * sh.y - suv.y * sh.x) * sh.w;
+            v.theta = uvw.u * l.x + uvw.v * l.y + uvw.w * l.z;
+            table_sincos(v.theta * (step / SM_VEL_C), sc_tab, v.ri, v.rr);
+            v.c2 = 2.0 * v.rr;
+            const double xa = table_pos(v.xk, fmin_w), xb = table_pos(v.xk, fmax_w);
+            const double ya = table_pos(v.yk, fmin_w), yb = table_pos(v.yk, fmax_w);
+            v.ixa = cell_of(xa);
+            v.iya = cell_of(ya);
+            const int nx = abs(cell_of(xb) - v.ixa), ny = abs(cell_of(yb) - v.iya);
+            const double lo = 1.0, hi = (double)(SM_SBF_L - 2);
+            fast = xa >= lo && xb >= lo && ya >= lo && yb >= lo && xa < hi && xb < hi && ya < hi && yb < hi &&
+                   nx + ny + 1 <= kShSeg / LB;
+            v.edges = fast ? nx | ny << 16 : 0;
+            v.coef = a.prange[c];
+            coef_lo = v.coef.x;
+            coef_hi = v.coef.x + v.coef.y + v.coef.z;
+            upto = fast ? nx + ny + 1 : 0;
+            const int own = upto;
+            for (int o = 1; o < kShItems; o <<= 1) {
+                const int before = __shfl_up(upto, o);
+                if (lane >= o) upto += before;
+            }
+            v.off = upto - own;
+            s_val[wv][lane] = v;
+        }
+        wave_sync();
+        const int nitem = min(VC, a.ncomp - c0) * LB;
+        for (int i0 = 0; i0 < nitem;) {
+            // The batch: pairs i0 .. i1 - 1, as many as 32 segments hold, or one component of up
+            // to kShSeg (two passes), or one component without segments (direct).
+            const int base = i0 > 0 ? __builtin_amdgcn_readlane(upto, i0 - 1) : 0;
+            const unsigned long long over = __ballot(lane >= i0 && (!fast || upto - base > 32));
+            int i1 = min((over != 0 ? __ffsll(over) - 1 : 64) / LB * LB, nitem);
+            const bool direct = i1 <= i0 && __any(lane >= i0 && lane < i0 + LB && !fast);
+            if (i1 <= i0) i1 = i0 + LB;
+            if (!direct) {
+                // 1. One segment and part per lane.
+                const int nseg = __builtin_amdgcn_readlane(upto, i1 - 1) - base;
+                const int cfirst = __builtin_amdgcn_readlane(coef_lo, i0);
+                const int ncoef = __builtin_amdgcn_readlane(coef_hi, i1 - 1) - cfirst;
+                const bool staged = ncoef <= kShCoef;
+                if (staged) {
+#pragma unroll
+                    for (int j = 0; j < kShCoef; j += 64)
+                        if (j + lane < ncoef)
+                            reinterpret_cast<int4 *>(s_coef[wv])[j + lane] =
+                                reinterpret_cast<const int4 *>(packed)[cfirst + j + lane];
+                    wave_sync();
+                }
+                for (int sf = lane >> 1; __any(sf < nseg); sf += 32) {
+                    if (sf >= nseg) continue;
+                    const int part = lane & 1;
+                    int it = i0;
+                    for (int i = i0 + 1; i < i1; ++i)
+                        it += __builtin_amdgcn_readlane(upto, i - 1) - base <= sf ? 1 : 0;
+                    const ShVal &v = s_val[wv][it];
+                    const int sg = sf - (v.off - base);
+                    const double xk = v.xk, yk = v.yk;
+                    const double xa = table_pos(xk, fmin_w), ya = table_pos(yk, fmin_w);
+                    const double X = xk * unit, Y = yk * unit;
+                    // Edges of x among the first sg crossed: edge i of x at t = (ux + i) / |X|.
+                    const int nx = v.edges & 0xffff, ny = v.edges >> 16;
+                    const double ux = X >= 0.0 ? v.ixa + 1 - xa : xa - v.ixa, uy = Y >= 0.0 ? v.iya + 1 - ya : ya - v.iya;
+                    const double rx = fabs(X), ry = fabs(Y);
+                    int ex = max(0, sg - ny);
+                    const int ex_max = min(sg, nx);
+                    ex = min(ex_max, max(ex, (int)((sg * rx + ux * ry - uy * rx) / fmax(rx + ry, 1e-300))));
+                    while (ex > max(0, sg - ny) && (ux + (ex - 1)) * ry > (uy + (sg - ex)) * rx) --ex;
+                    while (ex < ex_max && (uy + (sg - ex - 1)) * rx > (ux + ex) * ry) ++ex;
+                    const int ix = X >= 0.0 ? v.ixa + ex : v.ixa - ex, iy = Y >= 0.0 ? v.iya + (sg - ex) : v.iya - (sg - ex);
+                    const unsigned ox = 8u * (unsigned)ix, oy = 8u * (unsigned)iy;  // byte offsets, 32-bit: the table is 8 MB
+                    const int4 cr = v.coef;
+                    const int first = cr.x + (part ? cr.y : 0), cnt = part ? cr.z : cr.y;
+                    double s00 = 0.0, s10 = 0.0, s01 = 0.0, s11 = 0.0;
+                    // Four coefficients at a time, their eight table reads in flight together (the
+                    // scheduling barrier keeps the compiler from waiting for each read in turn).
+                    auto add4 = [&](const PackedCoeff *cp, int j) {
+                        double val[4], x[4][2], y[4][2];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const PackedCoeff cf = cp[min(j + u, cnt - 1)];
+                            val[u] = j + u < cnt ? cf.value : 0.0;
+                            const CellPair tx = *reinterpret_cast<const CellPair *>(
+                                sbf_b + (ox + __umul24((unsigned)cf.n1, 8u * SM_SBF_L)));
+                            const CellPair ty = *reinterpret_cast<const CellPair *>(
+                                sbf_b + (oy + __umul24((unsigned)cf.n2, 8u * SM_SBF_L)));
+                            x[u][0] = tx.v;
+                            x[u][1] = tx.next;
+                            y[u][0] = ty.v;
+                            y[u][1] = ty.next;
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const double vx = val[u] * x[u][0], vd = val[u] * (x[u][1] - x[u][0]);
+                            const double yd = y[u][1] - y[u][0];
+                            s00 = fma(vx, y[u][0], s00);
+                            s01 = fma(vx, yd, s01);
+                            s10 = fma(vd, y[u][0], s10);
+                            s11 = fma(vd, yd, s11);
+                        }
+                    };
+                    if (staged) {
+#pragma unroll 1
+                        for (int j = 0; j < cnt; j += 4) add4(s_coef[wv] + (first - cfirst), j);
+                    } else {
+#pragma unroll 1
+                        for (int j = 0; j < cnt; j += 4) add4(packed + first, j);
+                    }
+                    // The bilinear form at fractions wx = wx0 + X t, wy = wy0 + Y t.
+                    const double wx0 = fma(xk, fmin_w, SM_SBF_C - ix), wy0 = fma(yk, fmin_w, SM_SBF_C - iy);
+                    const double a0 = fma(wx0, s10, s00), a1 = fma(wx0, s11, s01), d = fma(wy0, s11, s10);
+                    T *o = s_seg[wv][sf] + 3 * part;
+                    o[0] = (T)fma(wy0, a1, a0);
+                    o[1] = (T)fma(Y, a1, X * d);
+                    o[2] = (T)(X * Y * s11);
+                }
+                wave_sync();
+            }
+            // 2. Channels.
+#pragma unroll 1
+            for (int i = i0; i < i1; i += LB) {
+                const int c = c0 + i / LB;
+                const ShVal &v = s_val[wv][i + bsub];
+                T cq[SL][4];
+#pragma unroll
+                for (int k = 0; k < SL; ++k) {
+                    const T *q = coh_t + ((size_t)c * 2 * a.nchan_pad + min(ch0 + k * LPB, a.nchan - 1)) * 2;
+                    cq[k][0] = q[0];
+                    cq[k][1] = q[1];
+                    cq[k][2] = q[2 * a.nchan_pad];
+                    cq[k][3] = q[2 * a.nchan_pad + 1];
+                }
+                const double theta = v.theta, xk = v.xk, yk = v.yk;
+                T er[SL], ei[SL];
+                if (!direct) {
+                    const T *sb = s_seg[wv][v.off - base];
+                    const int ixa = v.ixa, iya = v.iya;
+#pragma unroll
+                    for (int k = 0; k < SL; ++k) {
+                        const int sg = abs((int)table_pos(xk, freq[k]) - ixa) + abs((int)table_pos(yk, freq[k]) - iya);
+                        const T *q = sb + 6 * sg;
+                        er[k] = fma_t(tk[k], fma_t(tk[k], q[2], q[1]), q[0]);
+                        ei[k] = fma_t(tk[k], fma_t(tk[k], q[5], q[4]), q[3]);
+                    }
+                } else {
+                    // Rare: one coefficient at a time from the table in memory, per channel.
+                    const int4 cr = v.coef;
+#pragma unroll
+                    for (int k = 0; k < SL; ++k) {
+                        const double xp = table_pos(xk, freq[k]), yp = table_pos(yk, freq[k]);
+                        const double wx = xp - floor(xp), wy = yp - floor(yp);
+                        const double *bx = sbf + cell_of(xp), *by = sbf + cell_of(yp);
+                        double sum[2];
+#pragma unroll
+                        for (int pt = 0; pt < 2; ++pt) {
+                            const int first = cr.x + (pt ? cr.y : 0), cnt = pt ? cr.z : cr.y;
+                            sum[pt] = 0.0;
+#pragma unroll 1
+                            for (int j = 0; j < cnt; ++j) {
+                                const PackedCoeff cf = packed[first + j];
+                                const double *tx = bx + cf.n1 * SM_SBF_L, *ty = by + cf.n2 * SM_SBF_L;
+                                const double u = tx[0] + (tx[1] - tx[0]) * wx, w = ty[0] + (ty[1] - ty[0]) * wy;
+                                sum[pt] += (cf.value * u) * w;
+                            }
+                        }
+                        er[k] = (T)sum[0];
+                        ei[k] = (T)sum[1];
+                    }
+                }
+                double zr[SL], zi[SL];
+                table_sincos(theta * (freq[0] / SM_VEL_C), sc_tab, zi[0], zr[0]);
+                if (SL > 1) {
+                    if (rot) {
+                        const double rr = v.rr, ri = v.ri, c2 = v.c2;
+                        zr[SL > 1 ? 1 : 0] = zr[0] * rr - zi[0] * ri;
+                        zi[SL > 1 ? 1 : 0] = zr[0] * ri + zi[0] * rr;
+#pragma unroll
+                        for (int k = 2; k < SL; ++k) {
+                            zr[k] = fma(c2, zr[k - 1], -zr[k - 2]);
+                            zi[k] = fma(c2, zi[k - 1], -zi[k - 2]);
+                        }
+                    } else {
+#pragma unroll
+                        for (int k = 1; k < SL; ++k)
+                            table_sincos(theta * (freq[k] / SM_VEL_C), sc_tab, zi[k], zr[k]);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < SL; ++k) {
+                    const T zrk = (T)zr[k], zik = (T)zi[k];
+                    const T pr = zrk * er[k] - zik * ei[k];
+                    const T pi = zrk * ei[k] + zik * er[k];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        acc[k][2 * e] = fma_t(cq[k][e], pr, acc[k][2 * e]);
+                        acc[k][2 * e + 1] = fma_t(cq[k][e], pi, acc[k][2 * e + 1]);
+                    }
+                }
+                if ((c & 15) == 15) flush_stage(acc, tot);
+            }
+            wave_sync();
+            i0 = i1;
+        }
+    }
+    const int bl = bl0 + bsub;
+    if (bl >= a.nbl) return;
+#pragma unroll
+    for (int k = 0; k < SL; ++k) {
+        const int f = ch0 + k * LPB;
+        if (f >= a.nchan) continue;
+        T v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = two_level_sum(acc[k][e], tot[k][e]);
+        // XX, XY = A + i B, YX = A - i B, YY.
+        const T ar = v[2], ai = v[3], br = v[4], bi = v[5];
+        v[2] = ar - bi;
+        v[3] = ai + br;
+        v[4] = ar + bi;
+        v[5] = ai - br;
+        const size_t o = (size_t)f * a.nbl + bl;
+        float *v32 = reinterpret_cast<float *>(&a.vis32[o]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v32[e] += (float)v[e];
+        if (a.vis64 != nullptr) {
+            double *v64 = reinterpret_cast<double *>(&a.vis64[o]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v64[e] += (double)v[e];
+        }
+    }
+}
+
+template <class T, int SL, int LB, int WPS>
+static hipError_t launch_shapelets_form(const ShapeletChanArgs &a, hipStream_t stream) {
+    const long total = (long)((a.nbl + 4 * LB - 1) / (4 * LB)) * ((a.nchan + SL * 64 / LB - 1) / (SL * 64 / LB));
+    hipLaunchKernelGGL((k_shapelets<T, SL, LB, WPS>), dim3((unsigned)total), dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
+// The forms by channel count and step: fewer, wider groups share the phasors' start and the
+// component's values among more channels; narrow ones hold fewer segments, the cost that grows
+// with the step. Measured with 128 tiles within 1.5 km and 200 components (ms, FP64; FP32 within
+// 3%), as <slots, baselines per wave>:
+//   channels x step     <1,2>  <2,2>  <1,1>   one wave per baseline, adjacent channels
+//   32 x 40 kHz          0.59   0.73   0.73   2.19
+//   96 x 20 kHz          1.22   1.11   1.28   2.29
+//   384 x 20 kHz         4.05   2.81   3.30   5.85
+//   384 x 80 kHz         5.36   4.82   4.82   7.30
+//   384 x 160 kHz        7.73   8.27   7.33   10.06 (FP32: 7.28 against 7.26)
+// The weights are straight lines through these and nine more points, per group, in ms.
+template <class T> static hipError_t launch_shapelets(const ShapeletChanArgs &a, hipStream_t stream) {
+    const double khz = 1e-3 * a.step;
+    const double w32 = ((a.nchan + 31) / 32) * (0.275 + 0.0021 * khz);
+    const int g64 = (a.nchan + 63) / 64;
+    const double w64 = g64 * (0.30 + 0.0064 * khz), w64one = g64 * (0.42 + 0.0047 * khz);
+    if (w64 < w32 && w64 < w64one) return launch_shapelets_form<T, 2, 2, 3>(a, stream);
+    if (w64one < w32) return launch_shapelets_form<T, 1, 1, 4>(a, stream);
+    return launch_shapelets_form<T, 1, 2, 4>(a, stream);
+}
+
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream) {
     if (a.ncomp <= 0 || a.nbl <= 0 || a.nchan <= 0) return hipSuccess;
-    // Per-tile beams: a.ngroups groups of 64 channels; shared beam: groups of 128 channels.
-    const int total = ((a.nbl + 3) / 4) * (per_tile ? a.ngroups : (a.nchan + 127) / 128);
     const bool f32 = a.coh32 != nullptr;
     if (f32 && (a.sbf32 == nullptr || (per_tile && a.beam.coh_cls != nullptr && a.coh_cls32 == nullptr)))
         return hipErrorInvalidValue;
-    if (per_tile)
-        hipLaunchKernelGGL(f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles, dim3(total), dim3(256), 0, stream, a);
-    else
-        hipLaunchKernelGGL(f32 ? k_shapelet_chan32 : k_shapelet_chan, dim3(total), dim3(256), 0, stream, a);
+    if (!per_tile) return f32 ? launch_shapelets<float>(a, stream) : launch_shapelets<double>(a, stream);
+    const int total = ((a.nbl + 3) / 4) * a.ngroups;
+    hipLaunchKernelGGL(f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles, dim3(total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -804,6 +804,7 @@ static const char *model_timestep_device(SmModeller *m, double lst, double latit
     ctx.chunks.n16 = m->nchunks16;
     ctx.even = true;
     ctx.narrow = m->narrow;
+    ctx.step = mean_step(m->freqs_pad.data(), m->nchan);
     ctx.d_uvw = uvw;
     ctx.d_sbf = m->d_sbf.as<double>();
     ctx.d_tile_uvw = tile_uvw;

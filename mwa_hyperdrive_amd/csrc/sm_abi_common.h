@@ -31,6 +31,7 @@ struct ModelCtx {
     ChunkTabs chunks;    // channel chunks of evenly spaced runs, or null (fixed chunks)
     bool even16 = false; // fixed chunks of 16 channels are evenly spaced (chunk tables need no such test)
     bool narrow = false; // every channel step at most a thousandth of its frequency (narrow_steps)
+    double step = 0.0;   // mean channel spacing [Hz]
     const UVW *d_uvw = nullptr;
     const double *d_sbf = nullptr;
     BeamDesc beam{};

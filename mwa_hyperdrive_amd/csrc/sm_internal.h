@@ -165,6 +165,12 @@ struct DirectArgs {
     ChunkTabs chunks;  // channel chunks (evenly spaced runs), or fixed chunks when null
 };
 
+// Layouts of a coherency table: [component][channel][8]; the four Hermitian values
+// [component][channel][4] (the tile-pair kernels: 32 contiguous bytes per channel); or those as
+// two planes [component][2][channel][2] (the shapelet kernel: a lane's two 16-byte loads are
+// contiguous across the wave).
+enum CohForm { COH_FULL = 0, COH_HERMITIAN = 1, COH_HERMITIAN_PLANES = 2 };
+
 // Launchers (direct.hip). All enqueue on `stream` and return hipSuccess or an error.
 hipError_t launch_pack_coeffs(int ncomp, const int2 *d_range, const ShapeletCoeff *d_coeffs, int4 *d_prange,
                               PackedCoeff *d_packed, hipStream_t stream);
@@ -178,13 +184,17 @@ hipError_t launch_pair_coherency(int ncomp, int nchan, int nchan_pad, const doub
 // Component ranges for a baseline subset of nsub baselines (1 when they fill the GPU).
 int direct_subset_split(int nsub, int nchan, int ncomp);
 hipError_t launch_coherency(int ncomp, int nchan, int nchan_pad, const double *d_freqs, FluxBuckets fb,
-                            BeamDesc beam, bool apply_beam, double *d_coh, hipStream_t stream, bool hermitian = false);
+                            BeamDesc beam, bool apply_beam, double *d_coh, hipStream_t stream,
+                            CohForm form = COH_FULL);
 hipError_t launch_direct(Kind kind, bool per_tile, bool even, const DirectArgs &a, hipStream_t stream);
 bool chunks_even(const double *freqs_padded, int nchan);
 // Whether every fixed chunk of `width` channels is evenly spaced.
 bool chunks_even_width(const double *freqs_padded, int nchan, int width);
 // Whether every channel's step to the next is at most a thousandth of its frequency.
 bool narrow_steps(const double *freqs_padded, int nchan);
+inline double mean_step(const double *freqs, int nchan) {
+    return nchan > 1 ? fabs(freqs[nchan - 1] - freqs[0]) / (nchan - 1) : 0.0;
+}
 hipError_t launch_autos(int ntiles, int nchan, int ncomp, const double *d_coh, int nchan_pad, BeamDesc beam,
                         bool coh_has_beam, JonesF32 *vis32, JonesF64 *vis64, double *accum64, bool demote_now,
                         hipStream_t stream);

@@ -39,9 +39,9 @@ struct TiledArgs {
 };
 
 struct ShapeletChanArgs {
-    // ngroups: groups of 64 channels of the per-tile kernels (the shared-beam kernel takes
-    // groups of 128, two channels per lane, and forms its own count).
+    // ngroups: groups of 64 channels of the per-tile kernels (the shared-beam kernel forms its own).
     int nbl, nchan, nchan_pad, ncomp, ngroups;
+    double step = 0.0;  // mean channel spacing [Hz]
     const double *freqs;
     const UVW *uvw;           // [nbl]
     const double4 *lmn;
@@ -62,7 +62,7 @@ struct ShapeletChanArgs {
     JonesF32 *vis32;
     JonesF64 *vis64;
     // FP32 arithmetic with FP64 phases and table positions: coherency, per-class coherency
-    // and basis table in FP32. Null coh32 selects the FP64 kernels.
+    // and (per-tile beams) basis table in FP32. Null coh32 selects the FP64 kernels.
     const float *coh32 = nullptr;
     const float *coh_cls32 = nullptr;  // [nclass][ncomp][nchan_pad][8] when beam.coh_cls is set
     const float *sbf32 = nullptr;      // [SM_SBF_N][SM_SBF_L]
