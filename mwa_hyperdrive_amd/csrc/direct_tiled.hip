@@ -274,10 +274,11 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
 
 // ------------------------------------------------------------------ FP64 tile pairs on MFMA
 // One visibility is V^e = sum_c C^e_c z_c over the four real coefficients e of the Hermitian
-// coherency: a 4 x K by K x N product with K the components and N the real and imaginary
+// coherency: an N x K by K x 4 product with K the components and N the real and imaginary
 // parts of the baselines' phasors. v_mfma_f64_4x4x4 computes four such 4 x 4 x 4 blocks: lane l
-// supplies A = C^{l % 4} of component l / 16 and B = z of component l / 16 and baseline l % 16,
-// and accumulates e = l / 16 of baseline l % 16. The vector ALUs only form z.
+// supplies z of component l / 16 and baseline 4 (l % 4) + (l / 4) % 4 and C^{l % 4} of component
+// l / 16, and accumulates e = l % 4 of baseline l / 4: a wave's stores are contiguous. The vector
+// ALUs only form z.
 
 // z of the chunk's channels from the middle one outwards in both directions: evenly spaced
 // channels obey z_{k+1} = 2 cos(delta) z_k - z_{k-1}, one FMA per part, and starting in the middle
@@ -324,13 +325,14 @@ template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW>
 __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs a) {
     constexpr int R = NG * WR, SUB = kTG / R, NT = 64 * WR * WC;
     static_assert(kCT % (4 * WC) == 0, "a stage is whole groups of four components per wave");
+    constexpr int KR = WC > 1 ? WC / NG : 1;  // channels reduced at a time (WC > 1)
     struct Stage {
         double2 p0[kCT][32], p1[kCT][32];  // tile phasors: the chunk's middle channel, one channel step
         double c[kCT][NCH * 4 + 4];        // coherencies; the padding puts components on distinct banks
     };
     union Lds {
         Stage st;
-        double red[WC > 1 ? WC : 1][NG][2][64];
+        double red[WC > 1 ? WC : 1][KR][NG][2][64];
     };
     __shared__ Lds L;
     __shared__ double2 s_uv[32];
@@ -348,7 +350,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
     const int4 pr = a.pairs[rem / SUB];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int wr = wave % WR, wc = wave / WR;
-    const int cq = lane & 15, ck = lane >> 4;
+    const int cq = 4 * (lane & 3) + ((lane >> 2) & 3), ck = lane >> 4;
     if (tid < 32) {
         const int g = tid < 16 ? pr.y : pr.z;
         int t = g * kTG + (tid & 15);
@@ -448,90 +450,110 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
                 }
 #pragma unroll
                 for (int k = 0; k < NCH; ++k) {
-                    acc[k][g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(A[k], zr[k], acc[k][g][0], 0, 0, 0);
-                    acc[k][g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(A[k], zi[k], acc[k][g][1], 0, 0, 0);
+                    acc[k][g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(zr[k], A[k], acc[k][g][0], 0, 0, 0);
+                    acc[k][g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(zi[k], A[k], acc[k][g][1], 0, 0, 0);
                 }
             }
         }
         __syncthreads();
     }
-    // Lane l holds (re, im) of coefficient l / 16 for baseline l % 16: lanes of A = sum Re(C_XY) z
-    // and B = sum Im(C_XY) z exchange them (lane ^ 48) for XY = A + i B and YX = A - i B, and each
-    // lane writes one of the visibility's four entries.
-    auto store = [&](int g, int k, double re, double im) {
+    // Lane l holds (re, im) of coefficient l % 4 for baseline l / 4 of its row: lanes of A = sum
+    // Re(C_XY) z and B = sum Im(C_XY) z exchange them (lane ^ 3) for XY = A + i B and YX = A - i B,
+    // and each lane adds to one of the visibility's four entries, 512 contiguous bytes per wave. The
+    // entries of several channels are read before the first is written, or each would wait for its
+    // own: 2 points on 384 channels 114 -> 58 us, with 16 separate spans per wave instruction before.
+    const int sc = lane >> 2, se = lane & 3;
+    auto entry = [&](int g, size_t &o) {  // the lane's entry of row g at channel f0; whether there is one
         const int r = row0 + wr * NG + g;
         int p, q;
         bool valid;
         if (pr.x == 0) {
             p = pr.y * kTG + r;
-            q = pr.z * kTG + cq;
+            q = pr.z * kTG + sc;
             valid = q < a.ntiles;
-        } else if (r < cq) {
+        } else if (r < sc) {
             p = pr.y * kTG + r;
-            q = pr.y * kTG + cq;
+            q = pr.y * kTG + sc;
             valid = q < a.ntiles;
         } else {
-            p = pr.z * kTG + cq;
+            p = pr.z * kTG + sc;
             q = pr.z * kTG + r;
-            valid = r > cq && pr.z >= 0 && q < a.ntiles;
+            valid = r > sc && pr.z >= 0 && q < a.ntiles;
         }
-        const double ore = __shfl_xor(re, 48), oim = __shfl_xor(im, 48);
-        double vr = re, vi = im;
-        if (ck == 1) {
-            vr = re - oim;
-            vi = im + ore;
-        } else if (ck == 2) {
-            vr = ore + im;
-            vi = oim - re;
-        }
-        if (!valid) return;
+        if (!valid) p = 0, q = 1;
         if (a.tile_map != nullptr) {
             p = a.tile_map[p];
             q = a.tile_map[q];
         }
         const size_t nt = a.tile_map != nullptr ? (size_t)a.ntiles_bl : (size_t)a.ntiles;
         const size_t bl = (size_t)p * nt - (size_t)p * (p + 1) / 2 + (size_t)(q - p - 1);
-        const size_t o = (size_t)(f0 + k) * a.nbl + bl;
-        float2 *v32 = reinterpret_cast<float2 *>(&a.vis32[o]) + ck;
-        float2 t = *v32;
-        t.x += (float)vr;
-        t.y += (float)vi;
-        *v32 = t;
-        if (a.vis64 != nullptr) {
-            double2 *v64 = reinterpret_cast<double2 *>(&a.vis64[o]) + ck;
-            double2 d = *v64;
-            d.x += vr;
-            d.y += vi;
-            *v64 = d;
-        }
+        o = ((size_t)f0 * a.nbl + bl) * 4 + se;
+        return valid;
+    };
+    float2 *const vis32 = reinterpret_cast<float2 *>(a.vis32);
+    double2 *const vis64 = reinterpret_cast<double2 *>(a.vis64);
+    const size_t fstride = (size_t)a.nbl * 4;
+    auto add = [&](bool on, size_t o, float2 t, double2 d, double re, double im) {
+        const double ore = __shfl_xor(re, 3), oim = __shfl_xor(im, 3);
+        const double vr = se == 1 ? re - oim : (se == 2 ? ore + im : re);
+        const double vi = se == 1 ? im + ore : (se == 2 ? oim - re : im);
+        if (!on) return;
+        vis32[o] = make_float2(t.x + (float)vr, t.y + (float)vi);
+        if (vis64 != nullptr) vis64[o] = make_double2(d.x + vr, d.y + vi);
     };
     if (WC == 1) {
+        constexpr int KB = 8;  // channels read at a time
 #pragma unroll
-        for (int g = 0; g < NG; ++g)
+        for (int g = 0; g < NG; ++g) {
+            size_t o;
+            const bool valid = entry(g, o);
 #pragma unroll
-            for (int k = 0; k < NCH; ++k)
-                if (k < cnt) store(g, k, acc[k][g][0], acc[k][g][1]);
-    } else {
-        // The WC waves' sums of each channel, added in wave order by the first NG waves.
-        static_assert(WC == 1 || (WR == 1 && WC >= NG), "one row group per adding wave");
+            for (int k0 = 0; k0 < NCH; k0 += KB) {
+                float2 t[KB];
+                double2 d[KB];
 #pragma unroll
-        for (int k = 0; k < NCH; ++k) {
-            if (k >= cnt) break;
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                L.red[wc][g][0][lane] = acc[k][g][0];
-                L.red[wc][g][1][lane] = acc[k][g][1];
-            }
-            __syncthreads();
-            if (wc < NG) {
-                double re = 0.0, im = 0.0;
-#pragma unroll
-                for (int w = 0; w < WC; ++w) {
-                    re += L.red[w][wc][0][lane];
-                    im += L.red[w][wc][1][lane];
+                for (int k = 0; k < KB; ++k) {
+                    const bool on = valid && k0 + k < cnt;
+                    t[k] = on ? vis32[o + (k0 + k) * fstride] : make_float2(0.0f, 0.0f);
+                    d[k] = on && vis64 != nullptr ? vis64[o + (k0 + k) * fstride] : make_double2(0.0, 0.0);
                 }
-                store(wc, k, re, im);
+#pragma unroll
+                for (int k = 0; k < KB; ++k)
+                    add(valid && k0 + k < cnt, o + (k0 + k) * fstride, t[k], d[k], acc[k0 + k][g][0], acc[k0 + k][g][1]);
             }
+        }
+    } else {
+        // The WC waves' sums of KR channels at a time, added in wave order, one (channel, row) per wave.
+        static_assert(WC == 1 || (WR == 1 && WC == KR * NG && NCH % KR == 0), "one row and channel per adding wave");
+        const int kr = wc / NG, gr = wc % NG;
+        size_t o;
+        const bool valid = entry(gr, o);
+        float2 t[NCH / KR];
+        double2 d[NCH / KR];
+#pragma unroll
+        for (int i = 0; i < NCH / KR; ++i) {
+            const bool on = valid && i * KR + kr < cnt;
+            t[i] = on ? vis32[o + (i * KR + kr) * fstride] : make_float2(0.0f, 0.0f);
+            d[i] = on && vis64 != nullptr ? vis64[o + (i * KR + kr) * fstride] : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int i = 0; i < NCH / KR; ++i) {
+            if (i * KR >= cnt) break;
+#pragma unroll
+            for (int k = 0; k < KR; ++k)
+#pragma unroll
+                for (int g = 0; g < NG; ++g) {
+                    L.red[wc][k][g][0][lane] = acc[i * KR + k][g][0];
+                    L.red[wc][k][g][1][lane] = acc[i * KR + k][g][1];
+                }
+            __syncthreads();
+            double re = 0.0, im = 0.0;
+#pragma unroll
+            for (int w = 0; w < WC; ++w) {
+                re += L.red[w][kr][gr][0][lane];
+                im += L.red[w][kr][gr][1][lane];
+            }
+            add(valid && i * KR + kr < cnt, o + (i * KR + kr) * fstride, t[i], d[i], re, im);
             __syncthreads();
         }
     }
@@ -557,30 +579,34 @@ static hipError_t launch_tiles_form(TiledArgs a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Which form: the one with the smallest rounds x time of a round. A round is as many blocks as
-// the 256 CUs hold at once; its time per component was measured on 128 tiles, 768 channels, 5600
-// points and 2000 Gaussians. Two row groups of 16 channels share a Gaussian's exponentials and
-// a phasor's set-up over the most channels (points 13.7 ms, Gaussians 7.8 ms; four row groups of 8
-// channels 13.7 and 8.3 ms). Splitting the components over eight waves costs 1.5 times that on a
-// full chip (21.3 and 11.8 ms; 4 channels 23.6 and 18.1 ms), but its blocks are 4 rows high: on 32
-// channels (72 blocks of the widest form) it takes 1.01 and 0.57 ms against 1.56 and 0.93 ms, and
-// on 2 channels, 4 wide, 13 us for 90 points against 32 us.
+// Which form: the one with the smallest estimated time, from its blocks in units of what the 256
+// CUs hold at once (r), the time to start and end a block, and the time per component when the chip
+// is full and when a CU holds one block; all measured on 128 tiles. Two row groups of 16 channels
+// share a Gaussian's exponentials and a phasor's set-up over the most channels (768 channels, 5600
+// points 13.7 ms, 2000 Gaussians 7.8 ms; four row groups of 8 channels 13.7 and 8.3 ms). Two row
+// groups of 8 channels fill the chip sooner: 128 points and Gaussians on 32 channels 25 and 38 us,
+// against 38 and 59 us. Splitting the components over eight waves costs 1.5 times the widest form's
+// time on a full chip, but its blocks are 4 rows high: 90 points on 2 channels take 13 us, 4 wide,
+// against 32 us.
 template <int KIND, bool NARROW> static hipError_t launch_tiles(const TiledArgs &a, hipStream_t stream) {
     constexpr bool g = KIND == KIND_GAUSSIAN;
     struct Form {
         int nch, sub, resident;
-        double us;  // per component and round
+        double fixed, full, single;  // us: per round; per component and round; per component, one block a CU
     };
-    const Form forms[4] = {{16, 2, 512, g ? 0.554 : 0.348},
-                           {8, 1, 512, g ? 0.591 : 0.349},
-                           {8, 4, 256, g ? 0.109 : 0.0704},
-                           {4, 4, 512, g ? 0.168 : 0.0780}};
+    const Form forms[5] = {{16, 2, 512, 12.0, g ? 0.554 : 0.348, g ? 0.39 : 0.24},
+                           {8, 1, 512, 12.0, g ? 0.591 : 0.349, g ? 0.41 : 0.24},
+                           {8, 2, 768, 9.0, g ? 0.47 : 0.27, g ? 0.235 : 0.15},
+                           {8, 4, 256, 5.9, g ? 0.109 : 0.0704, g ? 0.109 : 0.0704},
+                           {4, 4, 512, 4.8, g ? 0.168 : 0.0780, g ? 0.07 : 0.05}};
     int best = -1;
     double t_best = 0.0;
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 5; ++i) {
         if (i == 0 && !a.even16) continue;
-        const long blocks = (long)a.npairs * forms[i].sub * chunk_count(a.chunks, forms[i].nch, a.nchan);
-        const double t = (double)((blocks + forms[i].resident - 1) / forms[i].resident) * forms[i].us;
+        const Form &f = forms[i];
+        const double r = (double)a.npairs * f.sub * chunk_count(a.chunks, f.nch, a.nchan) / f.resident;
+        const double rounds = r <= 1.0 ? r : 0.5 * (r + ceil(r));
+        const double t = fmax(r, 1.0) * f.fixed + a.ncomp * fmax(f.single, f.full * rounds);
         if (best < 0 || t < t_best) {
             best = i;
             t_best = t;
@@ -589,7 +615,8 @@ template <int KIND, bool NARROW> static hipError_t launch_tiles(const TiledArgs 
     switch (best) {
     case 0: return launch_tiles_form<KIND, 16, 2, 4, 1, NARROW>(a, stream);
     case 1: return launch_tiles_form<KIND, 8, 4, 4, 1, NARROW>(a, stream);
-    case 2: return launch_tiles_form<KIND, 8, 4, 1, 8, NARROW>(a, stream);
+    case 2: return launch_tiles_form<KIND, 8, 2, 4, 1, NARROW>(a, stream);
+    case 3: return launch_tiles_form<KIND, 8, 4, 1, 8, NARROW>(a, stream);
     default: return launch_tiles_form<KIND, 4, 4, 1, 8, NARROW>(a, stream);
     }
 }
