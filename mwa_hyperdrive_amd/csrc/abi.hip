@@ -142,13 +142,14 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const bool shared_tiled = ctx.d_bl_subset == nullptr && g_direct_variant == 0 && kind != KIND_SHAPELET &&
                               !per_tile && ctx.even && ctx.d_tile_uvw != nullptr && ctx.d_pairs != nullptr &&
                               ctx.ntiles >= 2;
-    // Shared-beam shapelets read the Hermitian form too, in planes.
+    // Shared-beam shapelets read the Hermitian form too, in FP64 as planes.
     const bool shared_shapelet =
         ctx.d_bl_subset == nullptr && g_direct_variant != 1 && kind == KIND_SHAPELET && !per_tile;
     const bool hermitian = shared_tiled || shared_shapelet;
+    const bool f32 = ctx.fp32 && kind != KIND_POINT && ctx.d_bl_subset == nullptr && g_direct_variant == 0;
+    const bool planes = shared_shapelet && !(f32 && ctx.d_sbf32 != nullptr);
     e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, ctx.beam, !per_tile, coh.as<double>(),
-                         stream,
-                         shared_shapelet ? COH_HERMITIAN_PLANES : (shared_tiled ? COH_HERMITIAN : COH_FULL));
+                         stream, planes ? COH_HERMITIAN_PLANES : (hermitian ? COH_HERMITIAN : COH_FULL));
     if (e != hipSuccess) return e;
     // Per-tile shapelets with beam-row classes: J_r S J_0^H per class for the channel-per-lane
     // kernel, when the table fits (otherwise the kernel forms J_p S J_q^H per visibility).
@@ -168,7 +169,6 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         beam.row0 = ctx.class_row0;
     }
     const size_t coh_n = (size_t)n * ctx.nchan_pad * 8;
-    const bool f32 = ctx.fp32 && kind != KIND_POINT && ctx.d_bl_subset == nullptr && g_direct_variant == 0;
     // Shapelet coefficients in the kernels' packed form.
     DevBuf &prange = scratch.prange, &packed = scratch.packed;
     const int4 *d_prange = nullptr;

@@ -11,9 +11,9 @@
 // paired so that 240 of 256 pairs are wanted ones. k_direct_tiled is the precision path's FP32
 // form for Gaussians, which keeps the products on the vector ALUs.
 //
-// k_shapelets (shapelets, one beam or none): the coefficient sums are formed once per run of
-// channels within a cell of the basis table. k_shapelet_chan_tiles (per-tile beams): one wave per
-// baseline, one lane per channel; the basis-table positions x_pos = k f + 5000 of neighbouring
+// k_shapelets (shapelets, one beam or none, FP64): the coefficient sums are formed once per run of
+// channels within a cell of the basis table. k_shapelet_chan_tiles (per-tile beams) and
+// k_shapelet_chan32: one wave per baseline, one or two channels per lane; the basis-table positions x_pos = k f + 5000 of neighbouring
 // channels fall in the same or adjacent table cells, so each coefficient's table reads coalesce
 // across the wave instead of touching 64 unrelated cache lines.
 #include "sm_internal.h"
@@ -26,6 +26,7 @@ namespace sm {
 constexpr int kTG = 16;   // tiles per group
 constexpr int kWin = 32;  // shapelet table window per wave and axis, cells
 constexpr int kRows = 16; // shapelet table rows staged per wave
+constexpr int kWinPair = 24;  // shapelet table window per wave and axis of the two-channel kernel, cells
 constexpr int kCT = 32;   // components per LDS stage
 // Channels per lane in k_direct_tiled (FP32 Gaussians). Measured per timestep of 256 tiles,
 // 384 channels and 10 000 Gaussians: 78.4 ms with 4, 76.2 ms with 6 (142 VGPRs), 115.9 ms with 8.
@@ -1426,6 +1427,280 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
     }
 }
 
+// Shared beam, FP32: one wave per baseline and 128 channels, two adjacent channels per lane
+// (channels 2 l and 2 l + 1 of the group on lane l). The table cells are read for both channels
+// at once: adjacent channels' positions differ by |k| df, below one cell (checked per component),
+// so both fall in cells i0 and i0 + 1 with i0 the lower of their two cells. The staged window
+// holds each cell's value and its difference to the next cell, formed once per component, and
+// the lane reads T[i0], T[i0 + 1] - T[i0] and T[i0 + 2] - T[i0 + 1] per axis and coefficient
+// (24 bytes for two channels, against 16 per channel reading two values). A channel in cell
+// i0 interpolates
+//   u = T[i0] + (T[i0+1] - T[i0]) w,
+// as the single-channel form does, and one in cell i0 + 1 takes
+//   u = (T[i0] + (T[i0+1] - T[i0])) + (T[i0+2] - T[i0+1]) w,
+// equal to T[i0+1] + (T[i0+2] - T[i0+1]) w up to the rounding of T[i0] + (T[i0+1] - T[i0]).
+// The coherency table is in the Hermitian form (Re XX, Re XY, Im XY, Re YY; J S J^H with one
+// beam on both sides), so each channel accumulates with 8 FMAs per component.
+
+// A staged basis-table cell: the value T[i] and the difference T[i + 1] - T[i].
+struct __attribute__((aligned(8))) CellTD {
+    float t, d;
+};
+
+__global__ __launch_bounds__(256) void k_shapelet_chan32(const ShapeletChanArgs a) {
+    using T = float;
+    const int ngroups = (a.nchan + 127) / 128;
+    const int nbx = (a.nbl + 3) / 4;
+    const int total = nbx * ngroups;
+    int b = blockIdx.x;
+    if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
+    const int group = b / nbx;
+    const int bx = b - group * nbx;
+    const int lane = threadIdx.x & 63;
+    const int bl = bx * 4 + (int)(threadIdx.x >> 6);
+    if (bl >= a.nbl) return;  // whole wave; the kernel has no barriers
+    const int fa_raw = group * 128 + 2 * lane;
+    const bool valid_a = fa_raw < a.nchan, valid_b = fa_raw + 1 < a.nchan;
+    const int fa = valid_a ? fa_raw : a.nchan - 1;
+    const int fb = valid_b ? fa_raw + 1 : a.nchan - 1;
+    const double freq_a = a.freqs[fa], freq_b = a.freqs[fb];
+    const double fc_a = freq_a / SM_VEL_C, fc_b = freq_b / SM_VEL_C;
+    const UVW uvw = a.uvw[bl];
+    const PackedCoeff *__restrict__ packed = a.packed;
+    const T *__restrict__ sbf = a.sbf32;
+    const T *__restrict__ coh_t = a.coh32;
+    // Per-wave windows of the basis table (kRows rows x kWinPair cells per axis), each cell
+    // holding T[i] and T[i + 1] - T[i].
+    __shared__ CellTD wx_lds[4][kRows][kWinPair], wy_lds[4][kRows][kWinPair];
+    const int wv = threadIdx.x >> 6;
+    // The wave's lowest and highest channel frequency and its largest step between a lane's
+    // two channels (channels past the last repeat it).
+    double fmin_w = fmin(freq_a, freq_b), fmax_w = fmax(freq_a, freq_b), dfmax_w = fabs(freq_b - freq_a);
+    for (int o = 32; o > 0; o >>= 1) {
+        fmin_w = fmin(fmin_w, __shfl_xor(fmin_w, o));
+        fmax_w = fmax(fmax_w, __shfl_xor(fmax_w, o));
+        dfmax_w = fmax(dfmax_w, __shfl_xor(dfmax_w, o));
+    }
+    T acc[2][8], tot[2][8];
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[ch][e] = tot[ch][e] = T(0);
+    const int blu = __builtin_amdgcn_readfirstlane(bl);
+    // Shapelet UVs: formed here from the baseline's tile XYZs and each component's (HA, Dec)
+    // when those are given; else read from bl_uv.
+    const bool uv_here = a.hadec != nullptr;
+    double x1 = 0, y1 = 0, z1 = 0, x2 = 0, y2 = 0, z2 = 0;
+    if (uv_here) {
+        const int2 t = a.bl_tiles[blu];
+        x1 = a.xyz[3 * t.x];
+        y1 = a.xyz[3 * t.x + 1];
+        z1 = a.xyz[3 * t.x + 2];
+        x2 = a.xyz[3 * t.y];
+        y2 = a.xyz[3 * t.y + 1];
+        z2 = a.xyz[3 * t.y + 2];
+    }
+    const double4 *__restrict__ hd4 = reinterpret_cast<const double4 *>(a.hadec);
+    // As in shapelet_chan: the wave-uniform per-component values, formed by lane l for
+    // component 64 q + l and read back by lane.
+    double th_lane = 0.0, xk_lane = 0.0, yk_lane = 0.0;
+    int wx_lane = 0, wy_lane = 0;
+    auto load_batch = [&](int q) {
+        const int cl = min((q << 6) + lane, a.ncomp - 1);
+        const double4 l = a.lmn[cl];
+        const double4 sh = a.shape[cl];
+        const double2 suv =
+            uv_here ? shapelet_uv(hd4[cl], x1, y1, z1, x2, y2, z2) : a.bl_uv[(size_t)cl * a.nbl + blu];
+        th_lane = uvw.u * l.x + uvw.v * l.y + uvw.w * l.z;
+        const double xk = (suv.x * sh.x + suv.y * sh.y) * sh.z;
+        const double yk = (suv.x * sh.y - suv.y * sh.x) * sh.w;
+        const double xa = xk * fmin_w + SM_SBF_C, xb = xk * fmax_w + SM_SBF_C;
+        const double ya = yk * fmin_w + SM_SBF_C, yb = yk * fmax_w + SM_SBF_C;
+        const int ix0 = (int)fmin(fmax(floor(fmin(xa, xb)), 0.0), (double)(SM_SBF_L - 2));
+        const int ix1 = (int)fmin(fmax(floor(fmax(xa, xb)), 0.0), (double)(SM_SBF_L - 2));
+        const int iy0 = (int)fmin(fmax(floor(fmin(ya, yb)), 0.0), (double)(SM_SBF_L - 2));
+        const int iy1 = (int)fmin(fmax(floor(fmax(ya, yb)), 0.0), (double)(SM_SBF_L - 2));
+        xk_lane = xk;
+        yk_lane = yk;
+        wx_lane = ix0 | ((ix1 - ix0 + 2) << 16);
+        wy_lane = iy0 | ((iy1 - iy0 + 2) << 16);
+    };
+    int4 pr_next = a.prange[0];
+    for (int c = 0; c < a.ncomp; ++c) {
+        const int4 pr4 = pr_next;
+        pr_next = a.prange[c + 1 < a.ncomp ? c + 1 : c];
+        if ((c & 63) == 0) load_batch(c >> 6);
+        const int src = c & 63;
+        const double theta = readlane_f64(th_lane, src);
+        const double xk = readlane_f64(xk_lane, src), yk = readlane_f64(yk_lane, src);
+        const int wxp = __builtin_amdgcn_readlane(wx_lane, src), wyp = __builtin_amdgcn_readlane(wy_lane, src);
+        T zr[2], zi[2];
+        sincos_phase(theta * fc_a, zi[0], zr[0]);
+        sincos_phase(theta * fc_b, zi[1], zr[1]);
+        const double xpa = xk * freq_a + SM_SBF_C, xpb = xk * freq_b + SM_SBF_C;
+        const double ypa = yk * freq_a + SM_SBF_C, ypb = yk * freq_b + SM_SBF_C;
+        const double fxa = floor(xpa), fxb = floor(xpb), fya = floor(ypa), fyb = floor(ypb);
+        const int ixa = (int)fmin(fmax(fxa, 0.0), (double)(SM_SBF_L - 2));
+        const int ixb = (int)fmin(fmax(fxb, 0.0), (double)(SM_SBF_L - 2));
+        const int iya = (int)fmin(fmax(fya, 0.0), (double)(SM_SBF_L - 2));
+        const int iyb = (int)fmin(fmax(fyb, 0.0), (double)(SM_SBF_L - 2));
+        const T wxa = (T)(xpa - fxa), wxb = (T)(xpb - fxb), wya = (T)(ypa - fya), wyb = (T)(ypb - fyb);
+        const int xw = wxp >> 16, yw = wyp >> 16;
+        // One component's coherencies for both channels (Hermitian form, 4 values each).
+        T cq[2][4];
+        {
+            const T *s_a = coh_t + ((size_t)c * a.nchan_pad + fa) * 4;
+            const T *s_b = coh_t + ((size_t)c * a.nchan_pad + fb) * 4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                cq[0][e] = s_a[e];
+                cq[1][e] = s_b[e];
+            }
+        }
+        T er[2], ei[2];
+        // Staged path: both windows, one extra cell for T[i0 + 2], fit the LDS copy, and the
+        // two channels of a lane are less than half a cell apart on both axes (so their cells
+        // differ by at most one, with a wide margin for rounding).
+        const bool near = fabs(xk) * dfmax_w < 0.5 && fabs(yk) * dfmax_w < 0.5;
+        if (near && xw + 1 <= kWinPair && yw + 1 <= kWinPair && pr4.w <= kRows) {
+            const int bx0 = wxp & 0xffff, by0 = wyp & 0xffff;
+            const int xs = xw + 1, ys = yw + 1;  // staged cells per axis
+            // As in shapelet_chan: lane -> (row lane >> lw, cell lane & (2^lw - 1)). A lane past
+            // the window or past row pr4.w - 1 reads an in-bounds cell that is never written; the
+            // last cell is at most SM_SBF_L, in the row or at the next row's first cell, and the
+            // difference it enters is only multiplied by a zero weight when outside the row.
+            // T[i + 1] comes from the next lane of the row; the difference formed with the next
+            // row's lane at cell 2^lw - 1 >= xs - 1 is never read (the loop reads differences
+            // at cells up to xs - 2).
+            const int wm = max(xs, ys);
+            const int lw = wm <= 4 ? 2 : (wm <= 8 ? 3 : (wm <= 16 ? 4 : 5));
+            const int rstep = 64 >> lw;
+            const int j = lane & ((1 << lw) - 1), rl = lane >> lw;
+            const int jxc = min(j, xs - 1), jyc = min(j, ys - 1);
+            static_assert(kRows + 16 < SM_SBF_N, "staged rows and the next row must exist in the basis table");
+            const unsigned ox = (unsigned)((rl * SM_SBF_L + bx0 + jxc) * sizeof(T));
+            const unsigned oy = (unsigned)((rl * SM_SBF_L + by0 + jyc) * sizeof(T));
+            const char *sbf_b = reinterpret_cast<const char *>(sbf);
+            constexpr int kBatch = 2;
+            for (int i0 = 0; i0 < pr4.w; i0 += kBatch * rstep) {
+                T tx[kBatch], ty[kBatch];
+#pragma unroll
+                for (int i = 0; i < kBatch; ++i) {
+                    const int base = i0 + i * rstep;
+                    const unsigned step = (unsigned)(base * SM_SBF_L * sizeof(T));
+                    if (base < pr4.w) {
+                        tx[i] = *reinterpret_cast<const T *>(sbf_b + (ox + step));
+                        ty[i] = *reinterpret_cast<const T *>(sbf_b + (oy + step));
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < kBatch; ++i) {
+                    const int base = i0 + i * rstep, r = base + rl;
+                    if (base < pr4.w) {  // wave-uniform: every lane takes part in the shuffles
+                        const T tx1 = __shfl_down(tx[i], 1), ty1 = __shfl_down(ty[i], 1);
+                        if (r < pr4.w) {
+                            if (j < xs) wx_lds[wv][r][j] = CellTD{tx[i], tx1 - tx[i]};
+                            if (j < ys) wy_lds[wv][r][j] = CellTD{ty[i], ty1 - ty[i]};
+                        }
+                    }
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // Each channel's weights on (T[i0+1] - T[i0]) and (T[i0+2] - T[i0+1]).
+            const int ix0l = min(ixa, ixb), iy0l = min(iya, iyb);
+            const int jx = ix0l - bx0, jy = iy0l - by0;
+            const bool xa_lo = ixa == ix0l, xb_lo = ixb == ix0l, ya_lo = iya == iy0l, yb_lo = iyb == iy0l;
+            const T ax_a = xa_lo ? wxa : T(1), bx_a = xa_lo ? T(0) : wxa;
+            const T ax_b = xb_lo ? wxb : T(1), bx_b = xb_lo ? T(0) : wxb;
+            const T ay_a = ya_lo ? wya : T(1), by_a = ya_lo ? T(0) : wya;
+            const T ay_b = yb_lo ? wyb : T(1), by_b = yb_lo ? T(0) : wyb;
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt) {
+                const PackedCoeff *cp = packed + pr4.x + (pt ? pr4.y : 0);
+                const int cnt = pt ? pr4.z : pr4.y;
+                T acc_a = T(0), acc_b = T(0);
+#pragma unroll 4
+                for (int k = 0; k < cnt; ++k) {
+                    double val;
+                    int n1, n2;
+                    load_packed_uniform(cp + k, val, n1, n2);
+                    const CellTD cx = wx_lds[wv][n1][jx], cy = wy_lds[wv][n2][jy];
+                    const T dx12 = wx_lds[wv][n1][jx + 1].d, dy12 = wy_lds[wv][n2][jy + 1].d;
+                    const T u_a = fma_t(dx12, bx_a, fma_t(cx.d, ax_a, cx.t));
+                    const T u_b = fma_t(dx12, bx_b, fma_t(cx.d, ax_b, cx.t));
+                    const T v_a = fma_t(dy12, by_a, fma_t(cy.d, ay_a, cy.t));
+                    const T v_b = fma_t(dy12, by_b, fma_t(cy.d, ay_b, cy.t));
+                    acc_a += ((T)val * u_a) * v_a;
+                    acc_b += ((T)val * u_b) * v_b;
+                }
+                (pt ? ei : er)[0] = acc_a;
+                (pt ? ei : er)[1] = acc_b;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        } else {
+            // Rare: one coefficient at a time from the table in memory, per channel.
+            const int ixs[2] = {ixa, ixb}, iys[2] = {iya, iyb};
+            const T wxs[2] = {wxa, wxb}, wys[2] = {wya, wyb};
+#pragma unroll
+            for (int ch = 0; ch < 2; ++ch) {
+#pragma unroll
+                for (int pt = 0; pt < 2; ++pt) {
+                    const PackedCoeff *cp = packed + pr4.x + (pt ? pr4.y : 0);
+                    const int cnt = pt ? pr4.z : pr4.y;
+                    T accp = T(0);
+#pragma unroll 1
+                    for (int k = 0; k < cnt; ++k) {
+                        double val;
+                        int n1, n2;
+                        load_packed_uniform(cp + k, val, n1, n2);
+                        const T *bxp = sbf + n1 * SM_SBF_L + ixs[ch], *byp = sbf + n2 * SM_SBF_L + iys[ch];
+                        const T u_value = bxp[0] + (bxp[1] - bxp[0]) * wxs[ch];
+                        const T v_value = byp[0] + (byp[1] - byp[0]) * wys[ch];
+                        accp += ((T)val * u_value) * v_value;
+                    }
+                    (pt ? ei : er)[ch] = accp;
+                }
+            }
+        }
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch) {
+            const T pr = zr[ch] * er[ch] - zi[ch] * ei[ch];
+            const T pi = zr[ch] * ei[ch] + zi[ch] * er[ch];
+            acc[ch][0] = fma_t(cq[ch][0], pr, acc[ch][0]);
+            acc[ch][1] = fma_t(cq[ch][0], pi, acc[ch][1]);
+            acc[ch][2] = fma_t(cq[ch][1], pr, acc[ch][2]);
+            acc[ch][3] = fma_t(cq[ch][1], pi, acc[ch][3]);
+            acc[ch][4] = fma_t(cq[ch][2], pr, acc[ch][4]);
+            acc[ch][5] = fma_t(cq[ch][2], pi, acc[ch][5]);
+            acc[ch][6] = fma_t(cq[ch][3], pr, acc[ch][6]);
+            acc[ch][7] = fma_t(cq[ch][3], pi, acc[ch][7]);
+        }
+        if ((c & 15) == 15) flush_stage(acc, tot);
+    }
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) {
+        if (!(ch ? valid_b : valid_a)) continue;
+        const size_t o = (size_t)(ch ? fb : fa) * a.nbl + bl;
+        T s8[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s8[e] = two_level_sum(acc[ch][e], tot[ch][e]);
+        // XX, XY = A + i B, YX = A - i B, YY.
+        const T v[8] = {s8[0], s8[1], s8[2] - s8[5], s8[3] + s8[4], s8[2] + s8[5], s8[3] - s8[4], s8[6], s8[7]};
+        float *v32 = reinterpret_cast<float *>(&a.vis32[o]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v32[e] += (float)v[e];
+        if (a.vis64 != nullptr) {
+            double *v64 = reinterpret_cast<double *>(&a.vis64[o]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v64[e] += (double)v[e];
+        }
+    }
+}
+
 // Per-tile beams: held to 128 VGPRs (4 waves per SIMD, a few spilled values) instead of the
 // 164 the compiler picks (3 waves). Measured on the 256-tile, 384-channel case: 129 -> 111 ms
 // per timestep.
@@ -1490,11 +1765,11 @@ struct __attribute__((packed, aligned(8))) CellPair {
     double v, next;
 };
 
-template <class T, int SL, int LB, int WPS>
+template <int SL, int LB, int WPS>
 __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a) {
     constexpr int LPB = 64 / LB, SPAN = SL * LPB, VC = kShItems / LB;
     __shared__ ShVal s_val[4][kShItems];
-    __shared__ __attribute__((aligned(16))) T s_seg[4][kShSeg][6];
+    __shared__ __attribute__((aligned(16))) double s_seg[4][kShSeg][6];
     __shared__ PackedCoeff s_coef[4][kShCoef];
     __shared__ double2 s_sc[64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1508,11 +1783,10 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
     if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
     const int group = b / nbx;
     const int bl0 = ((b - group * nbx) * 4 + wv) * LB;  // the wave's first baseline
-    if (bl0 >= a.nbl) return;                         // whole wave; no barriers below
+    if (bl0 >= a.nbl) return;                           // whole wave; no barriers below
     const int bsub = lane / LPB;  // this lane's baseline as a channel
     const int ch0 = group * SPAN + (lane & (LPB - 1));
-    double freq[SL];
-    T tk[SL];
+    double freq[SL], tk[SL];
 #pragma unroll
     for (int k = 0; k < SL; ++k) freq[k] = a.freqs[min(ch0 + k * LPB, a.nchan - 1)];
     // The span's lowest and highest frequency, and whether its slots are one step apart.
@@ -1534,23 +1808,23 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
     // Quadratics are in t = (f - fmin) / unit, t <= 1.
     const double unit = fmax_w > fmin_w ? fmax_w - fmin_w : 1.0;
 #pragma unroll
-    for (int k = 0; k < SL; ++k) tk[k] = (T)((freq[k] - fmin_w) / unit);
+    for (int k = 0; k < SL; ++k) tk[k] = (freq[k] - fmin_w) / unit;
 
     const PackedCoeff *__restrict__ packed = a.packed;
     const double *__restrict__ sbf = a.sbf;
     const char *__restrict__ sbf_b = reinterpret_cast<const char *>(a.sbf);
-    const T *__restrict__ coh_t = pick<T>(a.coh, a.coh32);
+    const double *__restrict__ coh = a.coh;
     auto wave_sync = [] {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
 
-    T acc[SL][8], tot[SL][8];
+    double acc[SL][8];
 #pragma unroll
     for (int k = 0; k < SL; ++k)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[k][e] = tot[k][e] = T(0);
+        for (int e = 0; e < 8; ++e) acc[k][e] = 0.0;
 
     for (int c0 = 0; c0 < a.ncomp; c0 += VC) {
         // Values of (component, baseline) pair `lane`, and the running count of segments.
@@ -1683,10 +1957,10 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
                     // The bilinear form at fractions wx = wx0 + X t, wy = wy0 + Y t.
                     const double wx0 = fma(xk, fmin_w, SM_SBF_C - ix), wy0 = fma(yk, fmin_w, SM_SBF_C - iy);
                     const double a0 = fma(wx0, s10, s00), a1 = fma(wx0, s11, s01), d = fma(wy0, s11, s10);
-                    T *o = s_seg[wv][sf] + 3 * part;
-                    o[0] = (T)fma(wy0, a1, a0);
-                    o[1] = (T)fma(Y, a1, X * d);
-                    o[2] = (T)(X * Y * s11);
+                    double *o = s_seg[wv][sf] + 3 * part;
+                    o[0] = fma(wy0, a1, a0);
+                    o[1] = fma(Y, a1, X * d);
+                    o[2] = (X * Y * s11);
                 }
                 wave_sync();
             }
@@ -1695,26 +1969,26 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
             for (int i = i0; i < i1; i += LB) {
                 const int c = c0 + i / LB;
                 const ShVal &v = s_val[wv][i + bsub];
-                T cq[SL][4];
+                double cq[SL][4];
 #pragma unroll
                 for (int k = 0; k < SL; ++k) {
-                    const T *q = coh_t + ((size_t)c * 2 * a.nchan_pad + min(ch0 + k * LPB, a.nchan - 1)) * 2;
+                    const double *q = coh + ((size_t)c * 2 * a.nchan_pad + min(ch0 + k * LPB, a.nchan - 1)) * 2;
                     cq[k][0] = q[0];
                     cq[k][1] = q[1];
                     cq[k][2] = q[2 * a.nchan_pad];
                     cq[k][3] = q[2 * a.nchan_pad + 1];
                 }
                 const double theta = v.theta, xk = v.xk, yk = v.yk;
-                T er[SL], ei[SL];
+                double er[SL], ei[SL];
                 if (!direct) {
-                    const T *sb = s_seg[wv][v.off - base];
+                    const double *sb = s_seg[wv][v.off - base];
                     const int ixa = v.ixa, iya = v.iya;
 #pragma unroll
                     for (int k = 0; k < SL; ++k) {
                         const int sg = abs((int)table_pos(xk, freq[k]) - ixa) + abs((int)table_pos(yk, freq[k]) - iya);
-                        const T *q = sb + 6 * sg;
-                        er[k] = fma_t(tk[k], fma_t(tk[k], q[2], q[1]), q[0]);
-                        ei[k] = fma_t(tk[k], fma_t(tk[k], q[5], q[4]), q[3]);
+                        const double *q = sb + 6 * sg;
+                        er[k] = fma(tk[k], fma(tk[k], q[2], q[1]), q[0]);
+                        ei[k] = fma(tk[k], fma(tk[k], q[5], q[4]), q[3]);
                     }
                 } else {
                     // Rare: one coefficient at a time from the table in memory, per channel.
@@ -1737,8 +2011,8 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
                                 sum[pt] += (cf.value * u) * w;
                             }
                         }
-                        er[k] = (T)sum[0];
-                        ei[k] = (T)sum[1];
+                        er[k] = sum[0];
+                        ei[k] = sum[1];
                     }
                 }
                 double zr[SL], zi[SL];
@@ -1761,16 +2035,14 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
                 }
 #pragma unroll
                 for (int k = 0; k < SL; ++k) {
-                    const T zrk = (T)zr[k], zik = (T)zi[k];
-                    const T pr = zrk * er[k] - zik * ei[k];
-                    const T pi = zrk * ei[k] + zik * er[k];
+                    const double pr = zr[k] * er[k] - zi[k] * ei[k];
+                    const double pi = zr[k] * ei[k] + zi[k] * er[k];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        acc[k][2 * e] = fma_t(cq[k][e], pr, acc[k][2 * e]);
-                        acc[k][2 * e + 1] = fma_t(cq[k][e], pi, acc[k][2 * e + 1]);
+                        acc[k][2 * e] = fma(cq[k][e], pr, acc[k][2 * e]);
+                        acc[k][2 * e + 1] = fma(cq[k][e], pi, acc[k][2 * e + 1]);
                     }
                 }
-                if ((c & 15) == 15) flush_stage(acc, tot);
             }
             wave_sync();
             i0 = i1;
@@ -1782,11 +2054,11 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
     for (int k = 0; k < SL; ++k) {
         const int f = ch0 + k * LPB;
         if (f >= a.nchan) continue;
-        T v[8];
+        double v[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = two_level_sum(acc[k][e], tot[k][e]);
+        for (int e = 0; e < 8; ++e) v[e] = acc[k][e];
         // XX, XY = A + i B, YX = A - i B, YY.
-        const T ar = v[2], ai = v[3], br = v[4], bi = v[5];
+        const double ar = v[2], ai = v[3], br = v[4], bi = v[5];
         v[2] = ar - bi;
         v[3] = ai + br;
         v[4] = ar + bi;
@@ -1798,15 +2070,15 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
         if (a.vis64 != nullptr) {
             double *v64 = reinterpret_cast<double *>(&a.vis64[o]);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v64[e] += (double)v[e];
+            for (int e = 0; e < 8; ++e) v64[e] += v[e];
         }
     }
 }
 
-template <class T, int SL, int LB, int WPS>
+template <int SL, int LB, int WPS>
 static hipError_t launch_shapelets_form(const ShapeletChanArgs &a, hipStream_t stream) {
     const long total = (long)((a.nbl + 4 * LB - 1) / (4 * LB)) * ((a.nchan + SL * 64 / LB - 1) / (SL * 64 / LB));
-    hipLaunchKernelGGL((k_shapelets<T, SL, LB, WPS>), dim3((unsigned)total), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((k_shapelets<SL, LB, WPS>), dim3((unsigned)total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
@@ -1819,16 +2091,16 @@ static hipError_t launch_shapelets_form(const ShapeletChanArgs &a, hipStream_t s
 //   96 x 20 kHz          1.22   1.11   1.28   2.29
 //   384 x 20 kHz         4.05   2.81   3.30   5.85
 //   384 x 80 kHz         5.36   4.82   4.82   7.30
-//   384 x 160 kHz        7.73   8.27   7.33   10.06 (FP32: 7.28 against 7.26)
+//   384 x 160 kHz        7.73   8.27   7.33   10.06
 // The weights are straight lines through these and nine more points, per group, in ms.
-template <class T> static hipError_t launch_shapelets(const ShapeletChanArgs &a, hipStream_t stream) {
+static hipError_t launch_shapelets(const ShapeletChanArgs &a, hipStream_t stream) {
     const double khz = 1e-3 * a.step;
     const double w32 = ((a.nchan + 31) / 32) * (0.275 + 0.0021 * khz);
     const int g64 = (a.nchan + 63) / 64;
     const double w64 = g64 * (0.30 + 0.0064 * khz), w64one = g64 * (0.42 + 0.0047 * khz);
-    if (w64 < w32 && w64 < w64one) return launch_shapelets_form<T, 2, 2, 3>(a, stream);
-    if (w64one < w32) return launch_shapelets_form<T, 1, 1, 4>(a, stream);
-    return launch_shapelets_form<T, 1, 2, 4>(a, stream);
+    if (w64 < w32 && w64 < w64one) return launch_shapelets_form<2, 2, 3>(a, stream);
+    if (w64one < w32) return launch_shapelets_form<1, 1, 4>(a, stream);
+    return launch_shapelets_form<1, 2, 4>(a, stream);
 }
 
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream) {
@@ -1836,9 +2108,10 @@ hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStr
     const bool f32 = a.coh32 != nullptr;
     if (f32 && (a.sbf32 == nullptr || (per_tile && a.beam.coh_cls != nullptr && a.coh_cls32 == nullptr)))
         return hipErrorInvalidValue;
-    if (!per_tile) return f32 ? launch_shapelets<float>(a, stream) : launch_shapelets<double>(a, stream);
-    const int total = ((a.nbl + 3) / 4) * a.ngroups;
-    hipLaunchKernelGGL(f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles, dim3(total), dim3(256), 0, stream, a);
+    if (!per_tile && !f32) return launch_shapelets(a, stream);
+    // Per-tile beams: a.ngroups groups of 64 channels; FP32 shared beam: groups of 128 channels.
+    const int total = ((a.nbl + 3) / 4) * (per_tile ? a.ngroups : (a.nchan + 127) / 128);
+    hipLaunchKernelGGL(!per_tile ? k_shapelet_chan32 : (f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles), dim3(total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -39,7 +39,7 @@ struct TiledArgs {
 };
 
 struct ShapeletChanArgs {
-    // ngroups: groups of 64 channels of the per-tile kernels (the shared-beam kernel forms its own).
+    // ngroups: groups of 64 channels of the per-tile kernels (the shared-beam kernels form their own).
     int nbl, nchan, nchan_pad, ncomp, ngroups;
     double step = 0.0;  // mean channel spacing [Hz]
     const double *freqs;
@@ -62,7 +62,7 @@ struct ShapeletChanArgs {
     JonesF32 *vis32;
     JonesF64 *vis64;
     // FP32 arithmetic with FP64 phases and table positions: coherency, per-class coherency
-    // and (per-tile beams) basis table in FP32. Null coh32 selects the FP64 kernels.
+    // and basis table in FP32. Null coh32 selects the FP64 kernels.
     const float *coh32 = nullptr;
     const float *coh_cls32 = nullptr;  // [nclass][ncomp][nchan_pad][8] when beam.coh_cls is set
     const float *sbf32 = nullptr;      // [SM_SBF_N][SM_SBF_L]
