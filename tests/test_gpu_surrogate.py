@@ -191,3 +191,28 @@ def test_modeller_with_surrogate_beam():
           f"{bound:.3e} from max |dJ| {d:.3e}); exact beam {rel_err(ref64, o64):.3e}")
     assert np.isfinite(w64).all()
     assert 0.0 < err <= bound
+
+
+# The weight gradients' batch slices: below one slice, one row over, ragged last slices and empty
+# ones; widths of one and several 64-wide tiles. A component of an FP32 sum of n products is within
+# about sqrt(n) 6e-8 of its largest, well below 1e-4 of the layer's largest gradient.
+@pytest.mark.parametrize("hidden,n", [(256, 1), (256, 127), (256, 129), (256, 4097), (65, 1000), (7, 8193)])
+def test_gradient_slices_vs_fp64(hidden, n):
+    s = sg.BeamSurrogate(seed=5, hidden=hidden, depth=2)
+    flat = torch.tensor(s.get_params(), dtype=torch.float64, requires_grad=True)
+    x, y = sg.samples(3, 0, n)
+    loss, g = s.gradients(x, y)
+    h, o, dims = x.cpu().double(), 0, [53, hidden, hidden, 8]
+    edges = [0]
+    for i, (a, b) in enumerate(zip(dims, dims[1:])):
+        w = flat[o:o + a * b].reshape(b, a)
+        h = h @ w.T + flat[o + a * b:o + a * b + b]
+        h = torch.nn.functional.silu(h) if i < 2 else h
+        edges += [o + a * b, o + a * b + b]
+        o += a * b + b
+    ref = ((h - y.cpu().double()) ** 2).mean()
+    ref.backward()
+    assert abs(loss - ref.item()) <= 1e-5 * ref.item()
+    want = flat.grad.numpy()
+    for lo, hi in zip(edges, edges[1:]):
+        assert np.abs(g[lo:hi] - want[lo:hi]).max() <= 1e-4 * np.abs(want[lo:hi]).max()
