@@ -1,5 +1,6 @@
 // Kernel-level drop-ins with the reference's signatures (src/gpu/model.h:33-56) and the
 // shared per-component-type driver used by both these and the SkyModeller handle.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -773,8 +774,14 @@ extern "C" const char *model_autos(int num_tiles, int num_freqs, const double *f
     SM_TRY(hipMemcpy(tmap.data(), tile_map, sizeof(int) * (max_total + 1), hipMemcpyDeviceToHost));
     std::vector<int> rows(num_tiles);
     for (int t = 0; t < num_tiles; ++t) rows[t] = tmap[unflagged_to_total[t]];
-    SM_TRY(st.tile_rows.reserve(sizeof(int) * num_tiles));
-    SM_TRY(hipMemcpy(st.tile_rows.ptr, rows.data(), sizeof(int) * num_tiles, hipMemcpyHostToDevice));
+    // Each tile's index into the distinct rows, then those rows.
+    std::vector<int> used(rows);
+    std::sort(used.begin(), used.end());
+    used.erase(std::unique(used.begin(), used.end()), used.end());
+    for (int &r : rows) r = (int)(std::lower_bound(used.begin(), used.end(), r) - used.begin());
+    rows.insert(rows.end(), used.begin(), used.end());
+    SM_TRY(st.tile_rows.reserve(sizeof(int) * rows.size()));
+    SM_TRY(hipMemcpy(st.tile_rows.ptr, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice));
     const size_t nvis = (size_t)num_tiles * num_freqs;
     SM_TRY(st.accum.reserve(sizeof(double) * 8 * nvis));
     SM_TRY(hipMemsetAsync(st.accum.ptr, 0, sizeof(double) * 8 * nvis, 0));
@@ -803,8 +810,9 @@ extern "C" const char *model_autos(int num_tiles, int num_freqs, const double *f
         SM_TRY(launch_coherency(counts[ty], num_freqs, nchan_pad, st.freqs_pad.as<double>(), fbs[ty], beam, false,
                                 st.coh.as<double>(), 0));
         beam.dir_offset = dir_off;
-        SM_TRY(launch_autos(num_tiles, num_freqs, counts[ty], st.coh.as<double>(), nchan_pad, beam, false, vis_fb,
-                            nullptr, st.accum.as<double>(), false, 0));
+        SM_TRY(launch_autos(num_tiles, (int)used.size(), st.tile_rows.as<int>() + num_tiles, num_freqs, counts[ty],
+                            st.coh.as<double>(), nchan_pad, beam, vis_fb, nullptr, st.accum.as<double>(),
+                            st.scratch.accum, 0));
         dir_off += counts[ty];
     }
     SM_TRY(launch_autos_demote((int)nvis, st.accum.as<double>(), vis_fb, nullptr, 0));

@@ -1123,8 +1123,8 @@ extern "C" const char *sm_model_timestep_autos_with(SmModeller *m, double lst, d
         SM_TRY(launch_coherency(n, m->nchan, m->nchan_pad, m->d_freqs.as<double>(), in.fb, none, false,
                                 d.coh.as<double>(), 0));
         b.uniform_row = -1;
-        SM_TRY(launch_autos(m->nt, m->nchan, n, d.coh.as<double>(), m->nchan_pad, b, false, m->d_vis32.as<JonesF32>(),
-                            d64, nullptr, true, 0));
+        SM_TRY(launch_autos(m->nt, m->n_utile, nullptr, m->nchan, n, d.coh.as<double>(), m->nchan_pad, b,
+                            m->d_vis32.as<JonesF32>(), d64, nullptr, m->scratch.accum, 0));
     }
     SM_TRY(hipMemcpy(vis_fb, m->d_vis32.ptr, sizeof(JonesF32) * nvis, hipMemcpyDeviceToHost));
     if (vis_fb_f64 != nullptr)

@@ -195,9 +195,11 @@ bool narrow_steps(const double *freqs_padded, int nchan);
 inline double mean_step(const double *freqs, int nchan) {
     return nchan > 1 ? fabs(freqs[nchan - 1] - freqs[0]) / (nchan - 1) : 0.0;
 }
-hipError_t launch_autos(int ntiles, int nchan, int ncomp, const double *d_coh, int nchan_pad, BeamDesc beam,
-                        bool coh_has_beam, JonesF32 *vis32, JonesF64 *vis64, double *accum64, bool demote_now,
-                        hipStream_t stream);
+// Adds each tile's auto-correlation: to accum64 if given (demoted later by launch_autos_demote), else
+// to vis32 and, if given, vis64. The tiles' beam rows are beam.tile_rows, each below nrows, of the
+// rows d_row_list (null: of the beam's first nrows). part: workspace.
+hipError_t launch_autos(int ntiles, int nrows, const int *d_row_list, int nchan, int ncomp, const double *d_coh, int nchan_pad, BeamDesc beam,
+                        JonesF32 *vis32, JonesF64 *vis64, double *accum64, struct DevBuf &part, hipStream_t stream);
 hipError_t launch_autos_demote(int n, const double *accum64, JonesF32 *vis32, JonesF64 *vis64, hipStream_t stream);
 hipError_t launch_shapelet_bl_uv(int ncomp, int ntiles, int nbl, const double *d_comp_hadec, const double *d_xyz,
                                  const int2 *d_bl_tiles, double2 *d_bl_uv, hipStream_t stream);
