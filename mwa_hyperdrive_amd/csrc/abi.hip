@@ -277,7 +277,8 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
                 r.vis32 = vis32;
                 r.vis64 = vis64;
                 r.chunks = ctx.chunks;
-                e = launch_direct_rect(kind, r, stream);
+                r.narrow = ctx.narrow;
+                e = launch_direct_rect(kind, r, &scratch.accum, stream);
             }
         }
         for (int sgi = 0; sgi < nseg && e == hipSuccess && !rect; ++sgi) {

@@ -309,6 +309,27 @@ __device__ __forceinline__ void chunk_phasors(double2 a0, double2 a1, double2 b0
     }
 }
 
+// z of the chunk's channels times a Gaussian's envelope e^{q f^2}, q = A u^2 + B u v + C v^2 (sh), by its
+// ratios from channel to channel: q0, q1 and q2 are f^2 at the first channel and its first and second
+// differences, qmin the q below which the envelope is 0 at every channel (e^-800 underflows).
+template <int NCH, bool NARROW>
+__device__ __forceinline__ void gaussian_envelopes(double4 sh, double bu, double bv, double qmin, double q0, double q1,
+                                                   double q2, const double *s_exp, double (&zr)[NCH], double (&zi)[NCH]) {
+    double qf = sh.x * (bu * bu) + sh.y * (bu * bv) + sh.z * (bv * bv);
+    qf = qf < qmin ? qmin : qf;
+    double env = table_exp(qf * q0, s_exp);
+    // Descending channels give a positive exponent; the cap keeps 0 * er at 0.
+    double er = table_exp(NARROW ? qf * q1 : fmin(qf * q1, 700.0), s_exp);
+    const double eg = NARROW ? small_exp(qf * q2) : table_exp(qf * q2, s_exp);
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+        zr[k] *= env;
+        zi[k] *= env;
+        env *= er;
+        er *= eg;
+    }
+}
+
 // What bounds it: FP64 issue. The matrix and vector FP64 instructions share one unit (16 FMAs
 // and 16 MFMAs per wave, measured: 36 and 111 ns apart, 141 ns together), which sustains 75
 // TFLOP/s on this MFMA against 62 on FMAs (the clock falls to 2.07 GHz under FMAs). A component
@@ -434,20 +455,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
                 if (KIND == KIND_GAUSSIAN) {
                     const double2 tp = s_uv[sp[g]], tq = s_uv[sq[g]];
                     const double bu = tp.x - tq.x, bv = tp.y - tq.y;
-                    double qf = sh.x * (bu * bu) + sh.y * (bu * bv) + sh.z * (bv * bv);
-                    // Below qmin the envelope is 0 at every channel of the chunk (e^-800 underflows).
-                    qf = qf < qmin ? qmin : qf;
-                    double env = table_exp(qf * q0, s_exp);
-                    // Descending channels give a positive exponent; the cap keeps 0 * er at 0.
-                    double er = table_exp(NARROW ? qf * q1 : fmin(qf * q1, 700.0), s_exp);
-                    const double eg = NARROW ? small_exp(qf * q2) : table_exp(qf * q2, s_exp);
-#pragma unroll
-                    for (int k = 0; k < NCH; ++k) {
-                        zr[k] *= env;
-                        zi[k] *= env;
-                        env *= er;
-                        er *= eg;
-                    }
+                    gaussian_envelopes<NCH, NARROW>(sh, bu, bv, qmin, q0, q1, q2, s_exp, zr, zi);
                 }
 #pragma unroll
                 for (int k = 0; k < NCH; ++k) {
@@ -967,26 +975,225 @@ hipError_t launch_pair_jones(Kind kind, const PairJonesArgs &a_in, DevBuf *accum
 }
 
 // ------------------------------------------------------------------ row tiles x class 0
-// k_direct_rect: a block owns 4 row tiles (one per wave) and 64 class-0 column tiles (one
-// per lane) for one channel chunk. Every lane of a wave shares its row's class, so the
-// coherency J_r S J_0^H arrives through scalar loads as in k_direct_tiled. The kernel forms
-// V_pq for the ordered pair (p = row tile, q = column tile); where the array orders the
-// baseline the other way (q < p) it stores V_qp = V_pq^H, which holds because the
-// instrumental coherency S is Hermitian (XY and YX are conjugates).
+// Pairs of a row tile (outside class 0) with a class-0 column tile: V_pq = sum_c C_c z_c with the
+// full coherency C = J_r S J_0^H of the row's class. Where the array orders the baseline the other
+// way (q < p), V_qp = V_pq^H is stored, which holds because the instrumental coherency S is
+// Hermitian (XY and YX are conjugates).
+//
+// FP64, k_rect_mfma: the tile-pair kernel's scheme (k_tiles_mfma) with the four complex entries of C
+// as the second operand and 16 columns of one row in a matrix instruction, four per channel (re and
+// im of z by re and im of C). A wave has one row and 16 CG columns, so a component's C, staged in LDS,
+// serves CG groups; a block has WR rows, which share the columns' phasors. Slices of the components
+// (blockIdx / per_slice) fill the chip when there are few row tiles; their sums meet in `part`.
+// Bound by FP64 issue: per component and channel 128 pairs take 128 matrix cycles a SIMD, their
+// phasors about 50. 26 rows by 230 columns, 96 channels: 50000 points 43.0 -> 27.6 ms, 10000 Gaussians
+// 14.1 -> 7.6 ms, against one lane per column on the vector ALUs. The blocks of one XCD sharing C took
+// 37.5 to 31 ms of points, reading it a stage ahead the rest. Measured slower: 8 rows a block (33.4 and
+// 9.4 ms); 4 column groups (26.4 and 11.2 ms); three waves a SIMD (26.5 and 9.7 ms).
+constexpr int kRectNch = 8;  // channels per chunk
+constexpr int kRectC = 16;   // components per LDS stage
+constexpr int kRectCG = 2;    // column groups per wave
+constexpr int kRectWR = 4;   // rows, one wave each, per block
+
+// Entry se of the baseline (row ri, column cj) at channel 0: its index in the visibilities, and
+// whether the array has the baseline the other way round (then the transposed entry's, conjugated).
+__device__ __forceinline__ size_t rect_entry(const RectArgs &a, int ri, int cj, int se, bool &flip) {
+    const int p = a.row_tiles[ri], q = a.col_tiles[cj];
+    flip = q < p;
+    const int lo = flip ? q : p, hi = flip ? p : q;
+    const size_t bl = (size_t)lo * a.ntiles_bl - (size_t)lo * (lo + 1) / 2 + (size_t)(hi - lo - 1);
+    return bl * 4 + (flip ? ((se & 1) << 1) | (se >> 1) : se);
+}
+
+template <int KIND, bool NARROW>
+__global__ __launch_bounds__(64 * kRectWR, 2) void k_rect_mfma(const RectArgs a, int per_slice, int slice_len, double2 *part) {
+    constexpr int WR = kRectWR, NCH = kRectNch, CG = kRectCG, NC = 16 * CG, NS = WR + NC, NT = 64 * WR;
+    static_assert(NCH * 4 == 32 && kRectC % 4 == 0, "half a wave reads a component's C");
+    __shared__ double2 s_p0[kRectC][NS], s_p1[kRectC][NS];  // tile phasors: rows, then columns (see Stage of k_tiles_mfma)
+    __shared__ double2 s_c[WR][kRectC][NCH * 4 + 4];        // C; the padding puts components on distinct banks
+    __shared__ double2 s_uv[NS];
+    __shared__ double s_w[NS];
+    __shared__ double2 s_sc[64];
+    __shared__ double s_exp[64];
+    __shared__ int s_cls[WR];
+    const int nrg = (a.n_row + WR - 1) / WR, ncg = (a.n_col + NC - 1) / NC;
+    // Consecutive blocks of one XCD (blockIdx modulo 8) take the column groups of the same rows,
+    // channels and components, which share their C in its L2.
+    const int total = gridDim.x / 8 * 8;
+    const int vb = (int)blockIdx.x < total ? (int)(blockIdx.x & 7) * (total >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    const int slice = vb / per_slice, b = vb - slice * per_slice;
+    const int chunk = b / (nrg * ncg), rem = b - chunk * (nrg * ncg);
+    const int rg = rem / ncg, cg = rem - rg * ncg;
+    int f0, cnt;
+    chunk_range<NCH>(a.chunks, chunk, a.nchan, f0, cnt);
+    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    if (tid < NS) {
+        const int t = tid < WR ? a.row_tiles[min(rg * WR + tid, a.n_row - 1)]
+                               : a.col_tiles[min(cg * NC + tid - WR, a.n_col - 1)];
+        s_uv[tid] = make_double2(a.tile_uvw[3 * t], a.tile_uvw[3 * t + 1]);
+        s_w[tid] = a.tile_uvw[3 * t + 2];
+        if (tid < WR) s_cls[tid] = a.row_cls[min(rg * WR + tid, a.n_row - 1)];
+    }
+    if (tid < 64) {
+        s_sc[tid] = make_double2(kSinCos32[2 * tid], kSinCos32[2 * tid + 1]);
+        if (KIND == KIND_GAUSSIAN) s_exp[tid] = kExp64[tid];
+    }
+    __syncthreads();
+    const int rows = min(WR, a.n_row - rg * WR);  // rows of this block
+    const bool row_ok = w < rows;
+    const int cq = 4 * (lane & 3) + ((lane >> 2) & 3), ck = lane >> 4, se = lane & 3;
+    const double F0 = a.freqs[f0], DF = a.freqs[f0 + 1] - F0;
+    const double fm0 = (F0 + (NCH / 2 - 1) * DF) / SM_VEL_C, fm1 = DF / SM_VEL_C;
+    const double qmin = -800.0 / (F0 * F0), q0 = F0 * F0, q1 = DF * (2.0 * F0 + DF), q2 = 2.0 * DF * DF;
+    const double4 *__restrict__ lmn4 = a.lmn;
+    const double4 *__restrict__ shape = a.shape;
+    const double2 *__restrict__ coh = reinterpret_cast<const double2 *>(a.coh_cls);
+
+    double re[NCH][CG], im[NCH][CG];
+#pragma unroll
+    for (int k = 0; k < NCH; ++k)
+#pragma unroll
+        for (int g = 0; g < CG; ++g) re[k][g] = im[k][g] = 0.0;
+
+    const int c_end = min(a.ncomp, (slice + 1) * slice_len);
+    // Each wave stages its row's C, read one stage ahead. Components past the last are staged as 0.
+    constexpr int PER = kRectC * NCH * 4 / 64;
+    const double2 *__restrict__ crow = coh + (size_t)s_cls[w] * a.ncomp * a.nchan_pad * 4 + (size_t)f0 * 4 + (lane & 31);
+    const size_t cstride = (size_t)a.nchan_pad * 4;
+    double2 cv[PER];
+    auto read_c = [&](int c0) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int c = c0 + 2 * i + (lane >> 5);
+            cv[i] = row_ok && c < c_end ? crow[c * cstride] : make_double2(0.0, 0.0);
+        }
+    };
+    read_c(slice * slice_len);
+    for (int c0 = slice * slice_len; c0 < c_end; c0 += kRectC) {
+        const int nc = min(kRectC, c_end - c0), nc4 = (nc + 3) & ~3;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) s_c[w][2 * i + (lane >> 5)][lane & 31] = cv[i];
+        for (int e = tid; e < nc4 * NS; e += NT) {
+            const int cc = e / NS, slot = e - cc * NS;
+            double s0 = 0.0, c0_ = 0.0, s1 = 0.0, c1 = 0.0;
+            if (cc < nc) {
+                const double4 l = lmn4[c0 + cc];
+                const double2 uv = s_uv[slot];
+                const double th = uv.x * l.x + uv.y * l.y + s_w[slot] * l.z;
+                table_sincos(th * fm0, reinterpret_cast<const double *>(s_sc), s0, c0_);
+                table_sincos(th * fm1, reinterpret_cast<const double *>(s_sc), s1, c1);
+            }
+            s_p0[cc][slot] = make_double2(c0_, s0);
+            s_p1[cc][slot] = make_double2(c1, s1);
+        }
+        __syncthreads();
+        if (row_ok) {
+            read_c(c0 + kRectC);
+            for (int cs = 0; cs < nc; cs += 4) {
+                const int cc = cs + ck;
+                double2 C[NCH];
+#pragma unroll
+                for (int k = 0; k < NCH; ++k) C[k] = s_c[w][cc][4 * k + se];
+                double4 sh = make_double4(0.0, 0.0, 0.0, 0.0);
+                if (KIND == KIND_GAUSSIAN) sh = shape[min(c0 + cc, a.ncomp - 1)];
+#pragma unroll
+                for (int g = 0; g < CG; ++g) {
+                    const int sq = WR + 16 * g + cq;
+                    double zr[NCH], zi[NCH];
+                    chunk_phasors<NCH>(s_p0[cc][w], s_p1[cc][w], s_p0[cc][sq], s_p1[cc][sq], zr, zi);
+                    if (KIND == KIND_GAUSSIAN) {
+                        const double2 tp = s_uv[w], tq = s_uv[sq];
+                        gaussian_envelopes<NCH, NARROW>(sh, tp.x - tq.x, tp.y - tq.y, qmin, q0, q1, q2, s_exp, zr, zi);
+                    }
+#pragma unroll
+                    for (int k = 0; k < NCH; ++k) {
+                        re[k][g] = __builtin_amdgcn_mfma_f64_4x4x4f64(zr[k], C[k].x, re[k][g], 0, 0, 0);
+                        im[k][g] = __builtin_amdgcn_mfma_f64_4x4x4f64(zr[k], C[k].y, im[k][g], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int k = 0; k < NCH; ++k) {
+                        re[k][g] = __builtin_amdgcn_mfma_f64_4x4x4f64(zi[k], -C[k].y, re[k][g], 0, 0, 0);
+                        im[k][g] = __builtin_amdgcn_mfma_f64_4x4x4f64(zi[k], C[k].x, im[k][g], 0, 0, 0);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!row_ok) return;
+    const int ri = rg * WR + w;
+    float2 *const vis32 = reinterpret_cast<float2 *>(a.vis32);
+    double2 *const vis64 = reinterpret_cast<double2 *>(a.vis64);
+    const size_t fstride = (size_t)a.nbl * 4;
+#pragma unroll
+    for (int g = 0; g < CG; ++g) {
+        const int cj = cg * NC + 16 * g + (lane >> 2);
+        if (cj >= a.n_col) continue;
+        if (part != nullptr) {
+            double2 *o = part + (((size_t)slice * a.nchan + f0) * a.n_row + ri) * a.n_col * 4 + (size_t)cj * 4 + se;
+#pragma unroll
+            for (int k = 0; k < NCH; ++k)
+                if (k < cnt) o[(size_t)k * a.n_row * a.n_col * 4] = make_double2(re[k][g], im[k][g]);
+        } else {
+            bool flip;
+            const size_t o = rect_entry(a, ri, cj, se, flip) + (size_t)f0 * a.nbl * 4;
+            // Every channel's entries are read before the first is written.
+            float2 t[NCH];
+            double2 d[NCH];
+#pragma unroll
+            for (int k = 0; k < NCH; ++k) {
+                t[k] = k < cnt ? vis32[o + k * fstride] : make_float2(0.0f, 0.0f);
+                d[k] = k < cnt && vis64 != nullptr ? vis64[o + k * fstride] : make_double2(0.0, 0.0);
+            }
+#pragma unroll
+            for (int k = 0; k < NCH; ++k) {
+                if (k >= cnt) break;
+                const double vi = flip ? -im[k][g] : im[k][g];
+                vis32[o + k * fstride] = make_float2(t[k].x + (float)re[k][g], t[k].y + (float)vi);
+                if (vis64 != nullptr) vis64[o + k * fstride] = make_double2(d[k].x + re[k][g], d[k].y + vi);
+            }
+        }
+    }
+}
+
+// The slices' sums, added in order to the visibilities: one thread per (channel, row, column, entry).
+__global__ void k_rect_finish(const RectArgs a, int slices, const double2 *__restrict__ part) {
+    const size_t n = (size_t)a.nchan * a.n_row * a.n_col * 4;
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double re = 0.0, im = 0.0;
+#pragma unroll 4
+    for (int s = 0; s < slices; ++s) {
+        const double2 v = part[s * n + i];
+        re += v.x;
+        im += v.y;
+    }
+    const int se = (int)(i & 3), cj = (int)((i >> 2) % a.n_col);
+    const size_t rf = (i >> 2) / a.n_col;
+    const int ri = (int)(rf % a.n_row), f = (int)(rf / a.n_row);
+    bool flip;
+    const size_t o = rect_entry(a, ri, cj, se, flip) + (size_t)f * a.nbl * 4;
+    if (flip) im = -im;
+    float2 &t = reinterpret_cast<float2 *>(a.vis32)[o];
+    t = make_float2(t.x + (float)re, t.y + (float)im);
+    if (a.vis64 != nullptr) {
+        double2 &d = reinterpret_cast<double2 *>(a.vis64)[o];
+        d = make_double2(d.x + re, d.y + im);
+    }
+}
+
+// FP32 (phases in FP64), k_direct_rect: a block owns 4 row tiles (one per wave) and 64 column tiles
+// (one per lane) for one channel chunk. Every lane of a wave shares its row's class, so C arrives
+// through scalar loads as in k_direct_tiled.
 constexpr int kRC = 16;  // components per LDS stage
 constexpr int kRT = 4 + 64;  // tile slots per block: 4 rows, then 64 columns
-// Gaussians here take 6 channels per lane. Measured per C5 timestep (256 tiles, 384 channels),
-// FP64: 48.1 ms with 4, 42.4 ms with 6 (151 VGPRs, 3 waves per SIMD); FP32: 28.3 ms with 4,
-// 26.8 ms with 6.
+// Channels per lane. 256 tiles, 384 channels: Gaussians 28.3 ms with 4, 26.8 ms with 6.
 constexpr int kRectNchGaussian = 6;
-// Points: the full-form J_r S J_0^H of a row is 64 bytes per channel of scalar loads, so wider
-// chunks cost more scalar registers and waits than they share. Measured per C5 FP64 timestep:
-// 138.1 ms with 4 channels per lane, 137.0 ms with 6, 149.9 ms with 8.
-constexpr int kRectNchPoint = 4;
 
-template <int KIND, int NCH, class T>
+template <int KIND, int NCH>
 __global__ __launch_bounds__(256) void k_direct_rect(const RectArgs a) {
-    using V4 = typename Vec4<T>::type;
+    using T = float;
+    using V4 = float4;
     __shared__ V4 s_ph[kRC][kRT];
     __shared__ double s_uvw[kRT][3];
     const int nrg = (a.n_row + 3) / 4, ncg = (a.n_col + 63) / 64;
@@ -1024,7 +1231,7 @@ __global__ __launch_bounds__(256) void k_direct_rect(const RectArgs a) {
     const double DF = freqs[f0 + 1] - F0;
     const double f0c = F0 / SM_VEL_C;
     const double dfc = DF / SM_VEL_C;
-    const T *__restrict__ coh = pick<T>(a.coh_cls, a.coh_cls32) + (size_t)cls * a.ncomp * a.nchan_pad * 8;
+    const T *__restrict__ coh = a.coh_cls32 + (size_t)cls * a.ncomp * a.nchan_pad * 8;
     const double4 *__restrict__ lmn4 = a.lmn;
     const double4 *__restrict__ shape = a.shape;
 
@@ -1138,24 +1345,46 @@ __global__ __launch_bounds__(256) void k_direct_rect(const RectArgs a) {
     }
 }
 
-hipError_t launch_direct_rect(Kind kind, const RectArgs &a, hipStream_t stream) {
-    if (a.ncomp <= 0 || a.n_row <= 0 || a.n_col <= 0 || a.nchan <= 0) return hipSuccess;
-    const int nch = kind == KIND_GAUSSIAN ? kRectNchGaussian : kRectNchPoint;
-    const long total = (long)((a.n_row + 3) / 4) * ((a.n_col + 63) / 64) * chunk_count(a.chunks, nch, a.nchan);
-    if (a.coh_cls32 != nullptr) {
-        if (kind == KIND_GAUSSIAN)
-            hipLaunchKernelGGL((k_direct_rect<KIND_GAUSSIAN, kRectNchGaussian, float>), dim3((unsigned)total),
-                               dim3(256), 0, stream, a);
-        else
-            hipLaunchKernelGGL((k_direct_rect<KIND_POINT, kRectNchPoint, float>), dim3((unsigned)total), dim3(256), 0,
-                               stream, a);
-    } else if (kind == KIND_GAUSSIAN) {
-        hipLaunchKernelGGL((k_direct_rect<KIND_GAUSSIAN, kRectNchGaussian, double>), dim3((unsigned)total),
-                           dim3(256), 0, stream, a);
-    } else {
-        hipLaunchKernelGGL((k_direct_rect<KIND_POINT, kRectNchPoint, double>), dim3((unsigned)total), dim3(256), 0,
-                           stream, a);
+template <int KIND, bool NARROW>
+static hipError_t launch_rect(const RectArgs &a, DevBuf *part, hipStream_t stream) {
+    constexpr int WR = kRectWR;
+    const int per_slice = ((a.n_row + WR - 1) / WR) * ((a.n_col + 16 * kRectCG - 1) / (16 * kRectCG)) *
+                          chunk_count(a.chunks, kRectNch, a.nchan);
+    // Slices of at least 512 components: as many as fill whole rounds of the blocks that the 256 CUs hold
+    // (two waves a SIMD), few for the traffic of their sums. No room for those: one.
+    constexpr int kSlots = 2 * 256 * 4 / WR;
+    int slices = 1;
+    double t_best = 0.0;
+    for (int s = 1; s == 1 || (s <= 16 && s <= a.ncomp / 512); ++s) {
+        const double t = (double)((per_slice * (long)s + kSlots - 1) / kSlots) / s + 0.02 * s * per_slice / kSlots;
+        if (s == 1 || t < t_best) {
+            slices = s;
+            t_best = t;
+        }
     }
+    const size_t n = (size_t)a.nchan * a.n_row * a.n_col * 4;
+    if (slices > 1 && (part == nullptr || part->reserve(sizeof(double2) * n * slices) != hipSuccess)) {
+        (void)hipGetLastError();
+        slices = 1;
+    }
+    double2 *p = slices > 1 ? part->as<double2>() : nullptr;
+    const int slice_len = ((a.ncomp + slices - 1) / slices + kRectC - 1) / kRectC * kRectC;
+    hipLaunchKernelGGL((k_rect_mfma<KIND, NARROW>), dim3((unsigned)(per_slice * slices)), dim3(64 * WR), 0, stream, a,
+                       per_slice, slice_len, p);
+    if (p != nullptr)
+        hipLaunchKernelGGL(k_rect_finish, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a, slices, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_direct_rect(Kind kind, const RectArgs &a, DevBuf *part, hipStream_t stream) {
+    if (a.ncomp <= 0 || a.n_row <= 0 || a.n_col <= 0 || a.nchan <= 0) return hipSuccess;
+    if (a.coh_cls32 == nullptr)
+        return kind == KIND_GAUSSIAN ? (a.narrow ? launch_rect<KIND_GAUSSIAN, true>(a, part, stream)
+                                                 : launch_rect<KIND_GAUSSIAN, false>(a, part, stream))
+                                     : launch_rect<KIND_POINT, true>(a, part, stream);
+    if (kind != KIND_GAUSSIAN) return hipErrorInvalidValue;  // FP32 points take the MFMA point path
+    const long total = (long)((a.n_row + 3) / 4) * ((a.n_col + 63) / 64) * chunk_count(a.chunks, kRectNchGaussian, a.nchan);
+    hipLaunchKernelGGL((k_direct_rect<KIND_GAUSSIAN, kRectNchGaussian>), dim3((unsigned)total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

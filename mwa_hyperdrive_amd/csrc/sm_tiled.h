@@ -68,9 +68,8 @@ struct ShapeletChanArgs {
     const float *sbf32 = nullptr;      // [SM_SBF_N][SM_SBF_L]
 };
 
-// Pairs of a tile outside beam class 0 (rows) with a class-0 tile (columns): one wave per
-// row tile and 64 column tiles, so the row's class, and with it the coherency
-// J_r S J_0^H, is wave-uniform.
+// Pairs of a tile outside beam class 0 (rows) with a class-0 tile (columns): the coherency
+// J_r S J_0^H depends on the row's class alone.
 struct RectArgs {
     int n_row, n_col, nbl, ntiles_bl, nchan, nchan_pad, ncomp;
     const int *row_tiles;     // [n_row] array tiles outside class 0
@@ -81,10 +80,12 @@ struct RectArgs {
     const double4 *lmn;
     const double4 *shape;
     const double *coh_cls;    // [nclass][ncomp][nchan_pad][8], J_r S J_0^H
-    const float *coh_cls32 = nullptr;  // the same in FP32 (FP32 arithmetic); null: FP64 kernels
+    // The same in FP32 (Gaussians in FP32 arithmetic); null: FP64 kernels.
+    const float *coh_cls32 = nullptr;
     JonesF32 *vis32;
     JonesF64 *vis64;
     ChunkTabs chunks;  // channel chunks; the fixed chunks must then be evenly spaced
+    bool narrow = false;  // as TiledArgs::narrow
 };
 
 // Pairs of two tiles with their own beam rows (tiles outside beam class 0): a block owns a
@@ -116,7 +117,8 @@ std::vector<int4> tile_pairs(int ntiles);
 // accum (nullable) backs the component split, which a grid of fewer than about 2048 blocks
 // takes (few tiles outside beam class 0); without it every block runs all components.
 hipError_t launch_pair_jones(Kind kind, const PairJonesArgs &a, DevBuf *accum, hipStream_t stream);
-hipError_t launch_direct_rect(Kind kind, const RectArgs &a, hipStream_t stream);
+// part (nullable) backs slices of the components, which few row tiles take.
+hipError_t launch_direct_rect(Kind kind, const RectArgs &a, DevBuf *part, hipStream_t stream);
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a, hipStream_t stream);
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream);
 hipError_t launch_tile_uvw_from_baselines(int ntiles, const UVW *d_uvw, double *d_out, hipStream_t stream);
