@@ -11,9 +11,9 @@
 // paired so that 240 of 256 pairs are wanted ones. k_direct_tiled is the precision path's FP32
 // form for Gaussians, which keeps the products on the vector ALUs.
 //
-// k_shapelets (shapelets, one beam or none, FP64): the coefficient sums are formed once per run of
-// channels within a cell of the basis table. k_shapelet_chan_tiles (per-tile beams) and
-// k_shapelet_chan32: one wave per baseline, one or two channels per lane; the basis-table positions x_pos = k f + 5000 of neighbouring
+// k_shapelets (shapelets, FP64): the coefficient sums are formed once per run of channels within a
+// cell of the basis table. k_shapelet_chan_tiles32 (per-tile beams) and k_shapelet_chan32, FP32: one
+// wave per baseline, one or two channels per lane; the basis-table positions x_pos = k f + 5000 of neighbouring
 // channels fall in the same or adjacent table cells, so each coefficient's table reads coalesce
 // across the wave instead of touching 64 unrelated cache lines.
 #include "sm_internal.h"
@@ -1397,8 +1397,11 @@ __device__ __forceinline__ double readlane_f64(double v, int lane) {
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-template <bool PER_TILE, class T>
-__device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
+// Per-tile beams, FP32: one wave per baseline, one channel per lane. Held to 96 VGPRs (5 waves per
+// SIMD, a few spilled values) instead of 118 (4 waves): 256 tiles and 384 channels 66.2 -> 57.8 ms.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_shapelet_chan_tiles32(
+    const ShapeletChanArgs a) {
+    using T = float;
     const int nbx = (a.nbl + 3) / 4;
     const int total = nbx * a.ngroups;
     int b = blockIdx.x;
@@ -1418,21 +1421,18 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
     int uf = 0;
     int cls = -1;
     bool herm = false;
-    if (PER_TILE) {
-        rows = a.beam.bl_rows[bl];
-        uf = a.beam.freq_map[f];
-        if (a.beam.coh_cls != nullptr) {
-            if (rows.y == a.beam.row0) {
-                cls = a.beam.class_of_row[rows.x];
-            } else if (rows.x == a.beam.row0) {
-                cls = a.beam.class_of_row[rows.y];
-                herm = true;
-            }
+    rows = a.beam.bl_rows[bl];
+    uf = a.beam.freq_map[f];
+    if (a.beam.coh_cls != nullptr) {
+        if (rows.y == a.beam.row0) {
+            cls = a.beam.class_of_row[rows.x];
+        } else if (rows.x == a.beam.row0) {
+            cls = a.beam.class_of_row[rows.y];
+            herm = true;
         }
     }
     const PackedCoeff *__restrict__ packed = a.packed;
-    const T *__restrict__ sbf = pick<T>(a.sbf, a.sbf32);
-    const T *__restrict__ coh_t = pick<T>(a.coh, a.coh32);
+    const T *__restrict__ sbf = a.sbf32;
     // Per-wave windows of the basis table (kRows rows x kWin cells per axis).
     __shared__ T wx_lds[4][kRows][kWin], wy_lds[4][kRows][kWin];
     const int wv = threadIdx.x >> 6;
@@ -1446,22 +1446,8 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
     // The wave's baseline is uniform; the next component's coefficient range is loaded one
     // iteration ahead.
     const int blu = __builtin_amdgcn_readfirstlane(bl);
-    // Shapelet UVs: formed here from the baseline's tile XYZs and each component's (HA, Dec)
-    // when those are given, so the [component][baseline] table is not re-read by every channel
-    // group; else read from bl_uv. The per-tile kernel reads bl_uv: it has no registers to spare
-    // (measured on the 256-tile case: more spills, 104 -> 110 ms per timestep).
-    const bool uv_here = !PER_TILE && a.hadec != nullptr;
-    double x1 = 0, y1 = 0, z1 = 0, x2 = 0, y2 = 0, z2 = 0;
-    if (uv_here) {
-        const int2 t = a.bl_tiles[blu];
-        x1 = a.xyz[3 * t.x];
-        y1 = a.xyz[3 * t.x + 1];
-        z1 = a.xyz[3 * t.x + 2];
-        x2 = a.xyz[3 * t.y];
-        y2 = a.xyz[3 * t.y + 1];
-        z2 = a.xyz[3 * t.y + 2];
-    }
-    const double4 *__restrict__ hd4 = reinterpret_cast<const double4 *>(a.hadec);
+    // Shapelet UVs are read from bl_uv: forming them here takes registers that it does not have (256
+    // tiles: more spills, 104 -> 110 ms per timestep).
     // The phase dot product, the UV in the component's frame (xk, yk) and the table window are
     // the same on every lane of the wave: lane l forms those of component 64 q + l once per
     // batch q of 64 components, and each component reads them from that lane. The window is
@@ -1472,8 +1458,7 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
         const int cl = min((q << 6) + lane, a.ncomp - 1);
         const double4 l = a.lmn[cl];
         const double4 sh = a.shape[cl];
-        const double2 suv =
-            uv_here ? shapelet_uv(hd4[cl], x1, y1, z1, x2, y2, z2) : a.bl_uv[(size_t)cl * a.nbl + blu];
+        const double2 suv = a.bl_uv[(size_t)cl * a.nbl + blu];
         th_lane = uvw.u * l.x + uvw.v * l.y + uvw.w * l.z;
         const double xk = (suv.x * sh.x + suv.y * sh.y) * sh.z;
         const double yk = (suv.x * sh.y - suv.y * sh.x) * sh.w;
@@ -1510,8 +1495,6 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
         const T wx = (T)(x_pos - fx), wy = (T)(y_pos - fy);
         T er, ei;
         const int xw = wxp >> 16, yw = wyp >> 16;
-        T cpre[8];
-        const T *s_c = coh_t + ((size_t)c * a.nchan_pad + f) * 8;
         if (xw <= kWin && yw <= kWin && pr4.w <= kRows) {
             // Stage rows 0 .. pr4.w - 1 of both windows in this wave's LDS, then interpolate
             // from LDS: one 16-byte read per axis per coefficient instead of two gathers.
@@ -1557,10 +1540,6 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             const int jx = ix - bx0, jy = iy - by0;
-            if (!PER_TILE) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) cpre[e] = s_c[e];
-            }
             T part[2];
 #pragma unroll
             for (int pt = 0; pt < 2; ++pt) {
@@ -1609,18 +1588,14 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
             }
             er = part[0];
             ei = part[1];
-            if (!PER_TILE) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) cpre[e] = s_c[e];
-            }
         }
         const T pr = zr * er - zi * ei;
         const T pi = zr * ei + zi * er;
         T cj[8];
-        if (PER_TILE && cls >= 0) {
-            class_coh(pick<T>(a.beam.coh_cls, a.coh_cls32) + (((size_t)cls * a.ncomp + c) * a.nchan_pad + f) * 8,
+        if (cls >= 0) {
+            class_coh(a.coh_cls32 + (((size_t)cls * a.ncomp + c) * a.nchan_pad + f) * 8,
                       herm, cj);
-        } else if (PER_TILE) {
+        } else {
             // J_p S J_q^H of the instrumental flux S (FP64 table) and the two tiles' beams.
             const double *s = a.coh + ((size_t)c * a.nchan_pad + f) * 8;
             double sv[8], j1[8], j2[8], cd[8];
@@ -1631,9 +1606,6 @@ __device__ __forceinline__ void shapelet_chan(const ShapeletChanArgs &a) {
             sandwich_t(j1, sv, j2, cd);
 #pragma unroll
             for (int e = 0; e < 8; ++e) cj[e] = (T)cd[e];
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) cj[e] = cpre[e];
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1730,7 +1702,7 @@ __global__ __launch_bounds__(256) void k_shapelet_chan32(const ShapeletChanArgs 
         z2 = a.xyz[3 * t.y + 2];
     }
     const double4 *__restrict__ hd4 = reinterpret_cast<const double4 *>(a.hadec);
-    // As in shapelet_chan: the wave-uniform per-component values, formed by lane l for
+    // As in k_shapelet_chan_tiles32: the wave-uniform per-component values, formed by lane l for
     // component 64 q + l and read back by lane.
     double th_lane = 0.0, xk_lane = 0.0, yk_lane = 0.0;
     int wx_lane = 0, wy_lane = 0;
@@ -1794,7 +1766,7 @@ __global__ __launch_bounds__(256) void k_shapelet_chan32(const ShapeletChanArgs 
         if (near && xw + 1 <= kWinPair && yw + 1 <= kWinPair && pr4.w <= kRows) {
             const int bx0 = wxp & 0xffff, by0 = wyp & 0xffff;
             const int xs = xw + 1, ys = yw + 1;  // staged cells per axis
-            // As in shapelet_chan: lane -> (row lane >> lw, cell lane & (2^lw - 1)). A lane past
+            // As in k_shapelet_chan_tiles32: lane -> (row lane >> lw, cell lane & (2^lw - 1)). A lane past
             // the window or past row pr4.w - 1 reads an in-bounds cell that is never written; the
             // last cell is at most SM_SBF_L, in the row or at the next row's first cell, and the
             // difference it enters is only multiplied by a zero weight when outside the row.
@@ -1930,21 +1902,18 @@ __global__ __launch_bounds__(256) void k_shapelet_chan32(const ShapeletChanArgs 
     }
 }
 
-// Per-tile beams: held to 128 VGPRs (4 waves per SIMD, a few spilled values) instead of the
-// 164 the compiler picks (3 waves). Measured on the 256-tile, 384-channel case: 129 -> 111 ms
-// per timestep.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_shapelet_chan_tiles(
-    const ShapeletChanArgs a) {
-    shapelet_chan<true, double>(a);
-}
-// FP32 per-tile beams: held to 96 VGPRs (5 waves per SIMD, a few spilled values) instead of 118
-// (4 waves). Measured on C5: 66.2 -> 57.8 ms per timestep.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_shapelet_chan_tiles32(
-    const ShapeletChanArgs a) {
-    shapelet_chan<true, float>(a);
+// J_p S J_q^H of component c at channel f, from the flux table (S) and the beams of rows p and q.
+__device__ __forceinline__ void own_beam_coh(const ShapeletChanArgs &a, int2 rows, int c, int f, double o[8]) {
+    double sv[8], j1[8], j2[8];
+    load_jones_t(reinterpret_cast<const JonesF64 *>(a.coh + ((size_t)c * a.nchan_pad + f) * 8), sv);
+    const size_t col = (size_t)a.beam.freq_map[f] * a.beam.n_dir + a.beam.dir_offset + c;
+    load_jones_t(&a.beam.jones[(size_t)rows.x * a.beam.n_ufreq * a.beam.n_dir + col], j1);
+    load_jones_t(&a.beam.jones[(size_t)rows.y * a.beam.n_ufreq * a.beam.n_dir + col], j2);
+    sandwich_t(j1, sv, j2, o);
 }
 
-// Shapelets with one beam on both sides (Hermitian coherencies) or none. One lane per channel (SL
+// Shapelets in FP64, with one beam on both sides (Hermitian coherencies) or none, or per-tile beams
+// (PT: the class's coherency or J_p S J_q^H, 8 values). One lane per channel (SL
 // slots of 64 / LB channels), LB baselines per wave.
 //
 // A component's basis-table positions x(f) = xk f + 5000 and y(f) are linear in frequency and the
@@ -1970,7 +1939,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 // 13.5 ms on 1400 components, 128 tiles and 384 channels of 80 kHz, 4.9 ms are coefficient sums
 // and 2.9 ms phasors. Summing the coefficients per channel, from table windows staged in LDS, took
 // 21.7 ms there, and 4.0 against 0.9 ms on 24 channels of 40 kHz. Slower in step 1: windows staged
-// in LDS (22 ms), the basis functions by their recurrence in registers (15.6 ms).
+// in LDS (22 ms), the basis functions by their recurrence in registers (15.6 ms). Per-tile beams (500
+// components, 256 tiles within 3 km, 96 channels of 80 kHz, so about three channels a run): 26.7 ms
+// summing per channel, 24.4 ms here (24.8 ms with the registers for three waves and no spills).
 constexpr int kShItems = 32;  // (component, baseline) pairs whose values are formed at a time
 constexpr int kShSeg = 64;    // segment quadratics per wave
 constexpr int kShCoef = 128;  // staged coefficients per wave
@@ -1994,7 +1965,7 @@ struct __attribute__((packed, aligned(8))) CellPair {
     double v, next;
 };
 
-template <int SL, int LB, int WPS>
+template <int SL, int LB, int WPS, bool PT>
 __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a) {
     constexpr int LPB = 64 / LB, SPAN = SL * LPB, VC = kShItems / LB;
     __shared__ ShVal s_val[4][kShItems];
@@ -2015,6 +1986,17 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
     if (bl0 >= a.nbl) return;                           // whole wave; no barriers below
     const int bsub = lane / LPB;  // this lane's baseline as a channel
     const int ch0 = group * SPAN + (lane & (LPB - 1));
+    // Per-tile beams: the beam rows of the lane's baseline, and its class if one of them is class 0's.
+    int2 rows = make_int2(0, 0);
+    int cls = -1;
+    bool herm = false;
+    if (PT) {
+        rows = a.beam.bl_rows[min(bl0 + bsub, a.nbl - 1)];
+        if (a.beam.coh_cls != nullptr) {
+            herm = rows.y != a.beam.row0;
+            if (!herm || rows.x == a.beam.row0) cls = a.beam.class_of_row[herm ? rows.y : rows.x];
+        }
+    }
     double freq[SL], tk[SL];
 #pragma unroll
     for (int k = 0; k < SL; ++k) freq[k] = a.freqs[min(ch0 + k * LPB, a.nchan - 1)];
@@ -2198,9 +2180,17 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
             for (int i = i0; i < i1; i += LB) {
                 const int c = c0 + i / LB;
                 const ShVal &v = s_val[wv][i + bsub];
-                double cq[SL][4];
+                double cq[SL][PT ? 8 : 4];
 #pragma unroll
                 for (int k = 0; k < SL; ++k) {
+                    if (PT) {
+                        const int f = min(ch0 + k * LPB, a.nchan - 1);
+                        if (cls >= 0)
+                            class_coh(a.beam.coh_cls + (((size_t)cls * a.ncomp + c) * a.nchan_pad + f) * 8, herm, cq[k]);
+                        else
+                            own_beam_coh(a, rows, c, f, cq[k]);
+                        continue;
+                    }
                     const double *q = coh + ((size_t)c * 2 * a.nchan_pad + min(ch0 + k * LPB, a.nchan - 1)) * 2;
                     cq[k][0] = q[0];
                     cq[k][1] = q[1];
@@ -2268,8 +2258,14 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
                     const double pi = zr[k] * ei[k] + zi[k] * er[k];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        acc[k][2 * e] = fma(cq[k][e], pr, acc[k][2 * e]);
-                        acc[k][2 * e + 1] = fma(cq[k][e], pi, acc[k][2 * e + 1]);
+                        const double cr = cq[k][PT ? 2 * e : e];
+                        acc[k][2 * e] = fma(cr, pr, acc[k][2 * e]);
+                        acc[k][2 * e + 1] = fma(cr, pi, acc[k][2 * e + 1]);
+                        if (PT) {
+                            const double ci = cq[k][PT ? 2 * e + 1 : 0];
+                            acc[k][2 * e] = fma(-ci, pi, acc[k][2 * e]);
+                            acc[k][2 * e + 1] = fma(ci, pr, acc[k][2 * e + 1]);
+                        }
                     }
                 }
             }
@@ -2286,12 +2282,14 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
         double v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = acc[k][e];
-        // XX, XY = A + i B, YX = A - i B, YY.
-        const double ar = v[2], ai = v[3], br = v[4], bi = v[5];
-        v[2] = ar - bi;
-        v[3] = ai + br;
-        v[4] = ar + bi;
-        v[5] = ai - br;
+        if (!PT) {
+            // XX, XY = A + i B, YX = A - i B, YY.
+            const double ar = v[2], ai = v[3], br = v[4], bi = v[5];
+            v[2] = ar - bi;
+            v[3] = ai + br;
+            v[4] = ar + bi;
+            v[5] = ai - br;
+        }
         const size_t o = (size_t)f * a.nbl + bl;
         float *v32 = reinterpret_cast<float *>(&a.vis32[o]);
 #pragma unroll
@@ -2304,10 +2302,10 @@ __global__ __launch_bounds__(256, WPS) void k_shapelets(const ShapeletChanArgs a
     }
 }
 
-template <int SL, int LB, int WPS>
+template <int SL, int LB, int WPS, bool PT>
 static hipError_t launch_shapelets_form(const ShapeletChanArgs &a, hipStream_t stream) {
     const long total = (long)((a.nbl + 4 * LB - 1) / (4 * LB)) * ((a.nchan + SL * 64 / LB - 1) / (SL * 64 / LB));
-    hipLaunchKernelGGL((k_shapelets<SL, LB, WPS>), dim3((unsigned)total), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((k_shapelets<SL, LB, WPS, PT>), dim3((unsigned)total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
@@ -2322,14 +2320,14 @@ static hipError_t launch_shapelets_form(const ShapeletChanArgs &a, hipStream_t s
 //   384 x 80 kHz         5.36   4.82   4.82   7.30
 //   384 x 160 kHz        7.73   8.27   7.33   10.06
 // The weights are straight lines through these and nine more points, per group, in ms.
-static hipError_t launch_shapelets(const ShapeletChanArgs &a, hipStream_t stream) {
+template <bool PT> static hipError_t launch_shapelets(const ShapeletChanArgs &a, hipStream_t stream) {
     const double khz = 1e-3 * a.step;
     const double w32 = ((a.nchan + 31) / 32) * (0.275 + 0.0021 * khz);
     const int g64 = (a.nchan + 63) / 64;
     const double w64 = g64 * (0.30 + 0.0064 * khz), w64one = g64 * (0.42 + 0.0047 * khz);
-    if (w64 < w32 && w64 < w64one) return launch_shapelets_form<2, 2, 3>(a, stream);
-    if (w64one < w32) return launch_shapelets_form<1, 1, 4>(a, stream);
-    return launch_shapelets_form<1, 2, 4>(a, stream);
+    if (w64 < w32 && w64 < w64one) return launch_shapelets_form<2, 2, 3, PT>(a, stream);
+    if (w64one < w32) return launch_shapelets_form<1, 1, 4, PT>(a, stream);
+    return launch_shapelets_form<1, 2, 4, PT>(a, stream);
 }
 
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream) {
@@ -2337,10 +2335,10 @@ hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStr
     const bool f32 = a.coh32 != nullptr;
     if (f32 && (a.sbf32 == nullptr || (per_tile && a.beam.coh_cls != nullptr && a.coh_cls32 == nullptr)))
         return hipErrorInvalidValue;
-    if (!per_tile && !f32) return launch_shapelets(a, stream);
+    if (!f32) return per_tile ? launch_shapelets<true>(a, stream) : launch_shapelets<false>(a, stream);
     // Per-tile beams: a.ngroups groups of 64 channels; FP32 shared beam: groups of 128 channels.
     const int total = ((a.nbl + 3) / 4) * (per_tile ? a.ngroups : (a.nchan + 127) / 128);
-    hipLaunchKernelGGL(!per_tile ? k_shapelet_chan32 : (f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles), dim3(total), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(per_tile ? k_shapelet_chan_tiles32 : k_shapelet_chan32, dim3(total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
