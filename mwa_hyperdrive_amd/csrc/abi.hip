@@ -147,7 +147,24 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const bool shared_shapelet =
         ctx.d_bl_subset == nullptr && g_direct_variant != 1 && kind == KIND_SHAPELET && !per_tile;
     const bool hermitian = shared_tiled || shared_shapelet;
-    const bool f32 = ctx.fp32 && kind != KIND_POINT && ctx.d_bl_subset == nullptr && g_direct_variant == 0;
+    // FP32 arithmetic (the precision path). Where that path's caller takes FP32 visibilities alone, an FP64
+    // kernel stands in wherever it is the faster one (us a timestep, FP32 and FP64):
+    // - tile-pair Gaussians of at most one FP32 block a CU, which then runs all components in one chain:
+    //   64 tiles, 48 channels, 1000 components (64 blocks) 636 and 275; 101 tiles, 93 channels, 700
+    //   components (400 blocks) 581 and 653, and FP32 by 10 to 15% above;
+    // - row-by-column Gaussians: 128 tiles, 12 of them with their own beams, 96 channels, 2000
+    //   components 3324 and 2227; 256 tiles, 26 such 6481 and 6214;
+    // - shared-beam shapelets, unless few channels fall in one table cell: 200 components, 128 tiles,
+    //   96 channels of 10 kHz 1664 and 969; 100 components, 256 tiles within 3 km, 93 of 80 kHz 4529 and 4401;
+    //   128 tiles within 3 km, 96 of 160 kHz 3130 and 3691 (256 tiles, 48 of 160 kHz, which fill less
+    //   than half of an FP32 wave's 128 channels: 4423 and 3913).
+    const bool fp32_path = ctx.fp32 && kind != KIND_POINT && ctx.d_bl_subset == nullptr && g_direct_variant == 0;
+    const bool either = fp32_path && vis64 == nullptr;
+    const int last128 = ctx.nchan % 128;
+    const bool few_per_cell = ctx.step > 80e3 && (last128 == 0 || last128 > 64);
+    auto small_grid = [&](int npairs) { return (long)npairs * chunk_count(ctx.chunks, 6, ctx.nchan) <= 256; };
+    const bool f32 =
+        fp32_path && !(either && ((shared_shapelet && !few_per_cell) || (shared_tiled && small_grid(ctx.npairs))));
     const bool planes = shared_shapelet && !(f32 && ctx.d_sbf32 != nullptr);
     e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, ctx.beam, !per_tile, coh.as<double>(),
                          stream, planes ? COH_HERMITIAN_PLANES : (hermitian ? COH_HERMITIAN : COH_FULL));
@@ -217,7 +234,8 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         b0.uniform_row = ctx.class_row0;
         e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, b0, true, coh0.as<double>(), stream,
                              COH_HERMITIAN);
-        if (e == hipSuccess && f32) e = to_f32(scratch.coh0_32, coh_n / 2, coh0.as<double>(), stream);
+        const bool pairs32 = f32 && !(either && small_grid(ctx.g0_npairs));
+        if (e == hipSuccess && pairs32) e = to_f32(scratch.coh0_32, coh_n / 2, coh0.as<double>(), stream);
         if (e != hipSuccess) return e;
         TiledArgs t;
         t.ntiles = ctx.g0_n;
@@ -233,7 +251,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.lmn = in.lmn;
         t.shape = in.shape;
         t.coh = coh0.as<double>();
-        if (f32) t.coh32 = scratch.coh0_32.as<float>();
+        if (pairs32) t.coh32 = scratch.coh0_32.as<float>();
         t.vis32 = vis32;
         t.vis64 = vis64;
         t.tile_map = ctx.d_g0_tiles;
@@ -255,7 +273,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         if (rect) {
             e = launch_class_coherency(ctx.nclass, n, ctx.nchan, ctx.nchan_pad, coh.as<double>(), ctx.beam,
                                        ctx.d_class_row, ccls.as<double>(), stream);
-            if (e == hipSuccess && f32) e = to_f32(scratch.ccls32, (size_t)ctx.nclass * coh_n, ccls.as<double>(), stream);
+            if (e == hipSuccess && f32 && !either) e = to_f32(scratch.ccls32, (size_t)ctx.nclass * coh_n, ccls.as<double>(), stream);
             if (e == hipSuccess) {
                 RectArgs r;
                 r.n_row = ctx.n_other;
@@ -273,7 +291,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
                 r.lmn = in.lmn;
                 r.shape = in.shape;
                 r.coh_cls = ccls.as<double>();
-                if (f32) r.coh_cls32 = scratch.ccls32.as<float>();
+                if (f32 && !either) r.coh_cls32 = scratch.ccls32.as<float>();
                 r.vis32 = vis32;
                 r.vis64 = vis64;
                 r.chunks = ctx.chunks;
