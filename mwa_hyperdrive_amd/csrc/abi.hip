@@ -259,8 +259,9 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.chunks = ctx.chunks;
         t.narrow = ctx.narrow;
         t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
+        t.part_limit = ctx.part_limit;
         if (ev0 != nullptr) (void)hipEventRecord(ev0, stream);
-        e = launch_direct_tiled(kind, t, stream);
+        e = launch_direct_tiled(kind, t, &scratch.accum, stream);
         // Pairs of a class-r tile with a class-0 tile. With a table of J_r S J_0^H for every
         // class (when it fits, g_class_table_limit): one launch of the row-by-column kernel.
         // Otherwise one shared coherency per segment and the shared-beam form of the
@@ -378,7 +379,8 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.chunks = ctx.chunks;
         t.narrow = ctx.narrow;
         t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
-        e = launch_direct_tiled(kind, t, stream);
+        t.part_limit = ctx.part_limit;
+        e = launch_direct_tiled(kind, t, &scratch.accum, stream);
     } else if (g_direct_variant != 1 && kind == KIND_SHAPELET) {
         ShapeletChanArgs s;
         s.nbl = ctx.nbl;
@@ -543,13 +545,39 @@ const char *gather_shape(Kind kind, int n_pl, const GaussianParams *pl, int n_cp
 
 using namespace sm;
 
-// The body of sm_model_points_f64 / sm_model_points_noalloc over the work buffers in st.
+// Work memory of a points call: the seven buffers that the shared body reserves, in its order.
+struct PointsWork {
+    size_t want[7], total = 0;
+};
+static size_t round_up256(size_t b) { return ((b < 256 ? 256 : b) + 255) / 256 * 256; }
+static PointsWork points_work(int n, const Addresses *a, const void *d_uvws, const void *d_beam_jones) {
+    const size_t nchan_pad = (size_t)pad_channels(a->num_freqs), nbl = (size_t)a->num_baselines;
+    const size_t ntiles = (size_t)llround((1.0 + std::sqrt(1.0 + 8.0 * (double)nbl)) / 2.0);
+    const size_t groups = (ntiles + 15) / 16;
+    const size_t npairs = groups * (groups - 1) / 2 + (groups + 1) / 2;
+    PointsWork w{{
+        sizeof(double) * nchan_pad,                          // padded frequencies
+        d_uvws != nullptr ? sizeof(double) * 3 * ntiles : 0,  // tile UVWs
+        d_uvws != nullptr ? sizeof(int4) * npairs : 0,       // tile-group pairs
+        d_beam_jones != nullptr ? sizeof(int) * ntiles : 0,  // beam row per tile
+        d_beam_jones != nullptr ? sizeof(int2) * nbl : 0,    // beam rows per baseline
+        sizeof(double4) * (size_t)n,                         // LMN
+        sizeof(double) * 8 * (size_t)n * nchan_pad,          // coherency table
+    }};
+    for (size_t b : w.want) w.total += b > 0 ? round_up256(b) : 0;
+    return w;
+}
+
+// The body of sm_model_points_f64 / sm_model_points_noalloc over the work buffers in st. Both keep
+// component slices to what the fixed array has left, so that they agree bit for bit.
 static const char *model_points_with(AbiState &st, const Points *p, const Addresses *a, const UVW *d_uvws,
                                      const JonesF64 *d_beam_jones, JonesF32 *d_vis_fb, JonesF64 *d_vis_fb_f64) {
     const int n = p->num_power_laws + p->num_curved_power_laws + p->num_lists;
     ModelCtx ctx;
     if (const char *err = abi_ctx(st, a, d_uvws, d_beam_jones, n, ctx)) return err;
     if (ctx.nbl == 0 || ctx.nchan == 0) return nullptr;
+    const size_t work = points_work(n, a, d_uvws, d_beam_jones).total;
+    ctx.part_limit = work < SM_NOALLOC_SCRATCH_BYTES ? SM_NOALLOC_SCRATCH_BYTES - work : 0;
     if (const char *err = gather_lmn(p->num_power_laws, p->power_law_lmns, p->num_curved_power_laws,
                                      p->curved_power_law_lmns, p->num_lists, p->list_lmns, st.lmn))
         return err;
@@ -598,8 +626,6 @@ const char *noalloc_scratch(void **out) {
     return nullptr;
 }
 
-size_t round_up256(size_t b) { return ((b < 256 ? 256 : b) + 255) / 256 * 256; }
-
 }  // namespace
 
 extern "C" const char *sm_model_points_noalloc(const Points *p, const Addresses *a, const UVW *d_uvws,
@@ -612,21 +638,9 @@ extern "C" const char *sm_model_points_noalloc(const Points *p, const Addresses 
     const long long nbl = a->num_baselines;
     const int ntiles = (int)llround((1.0 + std::sqrt(1.0 + 8.0 * (double)nbl)) / 2.0);
     if ((long long)ntiles * (ntiles - 1) / 2 != nbl) return "num_baselines is not a triangular number";
-    const size_t nchan_pad = (size_t)pad_channels(a->num_freqs);
-    const size_t groups = (size_t)(ntiles + 15) / 16;
-    const size_t npairs = groups * (groups - 1) / 2 + (groups + 1) / 2;
-    // Every buffer the shared body reserves, in the order it reserves them.
-    const size_t want[7] = {
-        sizeof(double) * nchan_pad,                                  // padded frequencies
-        d_uvws != nullptr ? sizeof(double) * 3 * (size_t)ntiles : 0,  // tile UVWs
-        d_uvws != nullptr ? sizeof(int4) * npairs : 0,               // tile-group pairs
-        d_beam_jones != nullptr ? sizeof(int) * (size_t)ntiles : 0,  // beam row per tile
-        d_beam_jones != nullptr ? sizeof(int2) * (size_t)nbl : 0,    // beam rows per baseline
-        sizeof(double4) * (size_t)n,                                 // LMN
-        sizeof(double) * 8 * (size_t)n * nchan_pad,                  // coherency table
-    };
-    size_t total = 0;
-    for (size_t w : want) total += w > 0 ? round_up256(w) : 0;
+    const PointsWork work = points_work(n, a, d_uvws, d_beam_jones);
+    const size_t(&want)[7] = work.want;
+    const size_t total = work.total;
     if (total > (size_t)SM_NOALLOC_SCRATCH_BYTES)
         return "sm_model_points_noalloc: this call needs more work memory than the fixed scratch array "
                "holds (SM_NOALLOC_SCRATCH_BYTES; about 64 B per component and padded channel)";
@@ -643,10 +657,10 @@ extern "C" const char *sm_model_points_noalloc(const Points *p, const Addresses 
         bufs[i]->borrow(static_cast<unsigned char *>(base) + off, round_up256(want[i]));
         off += round_up256(want[i]);
     }
+    st.scratch.accum.borrow(static_cast<unsigned char *>(base) + off, (size_t)SM_NOALLOC_SCRATCH_BYTES - off);
     // Buffers the point path never reserves: borrowed with no capacity, so that any use
     // fails with an error instead of allocating.
-    for (DevBuf *b : {&st.shape, &st.bl_uv, &st.coeffs, &st.coeff_range, &st.sbf, &st.accum, &st.scratch.accum,
-                      &st.scratch.cls, &st.scratch.prange, &st.scratch.packed, &st.scratch.coh0, &st.scratch.cseg,
+    for (DevBuf *b : {&st.shape, &st.bl_uv, &st.coeffs, &st.coeff_range, &st.sbf, &st.accum, &st.scratch.cls, &st.scratch.prange, &st.scratch.packed, &st.scratch.coh0, &st.scratch.cseg,
                       &st.scratch.ccls})
         b->borrow(nullptr, 0);
     return model_points_with(st, p, a, d_uvws, d_beam_jones, d_vis_fb, d_vis_fb_f64);

@@ -343,7 +343,7 @@ __device__ __forceinline__ void gaussian_envelopes(double4 sh, double bu, double
 // channels. WR waves split the rows (NG each); WC waves split the components (each takes every
 // WC-th group of four of a stage), their sums meeting in LDS at the end. A chunk's coherencies are
 // read NCH wide whatever its count (TiledArgs::coh); what the extra channels accumulate is dropped.
-template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW>
+template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW, bool SLICED>
 __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs a) {
     constexpr int R = NG * WR, SUB = kTG / R, NT = 64 * WR * WC;
     static_assert(kCT % (4 * WC) == 0, "a stage is whole groups of four components per wave");
@@ -361,9 +361,14 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
     __shared__ double s_w[32];
     __shared__ double2 s_sc[64];
     __shared__ double s_exp[64];
-    const int total = a.npairs * a.nchunks * SUB;
+    const int per_slice = a.npairs * a.nchunks * SUB;
+    const int total = per_slice * (SLICED ? a.slices : 1);
     int b = blockIdx.x;
     if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
+    const int slice = SLICED ? b / per_slice : 0;  // of the components
+    b -= slice * per_slice;
+    const int c_begin = slice * a.slice_len;
+    const int c_end = SLICED ? min(a.ncomp, c_begin + a.slice_len) : a.ncomp;
     const int chunk = b / (a.npairs * SUB);
     int f0, cnt;
     chunk_range<NCH>(a.chunks, chunk, a.nchan, f0, cnt);
@@ -414,8 +419,8 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
 #pragma unroll
         for (int g = 0; g < NG; ++g) acc[k][g][0] = acc[k][g][1] = 0.0;
 
-    for (int c0 = 0; c0 < a.ncomp; c0 += kCT) {
-        const int nc = a.ncomp - c0 < kCT ? a.ncomp - c0 : kCT;
+    for (int c0 = c_begin; c0 < c_end; c0 += kCT) {
+        const int nc = min(kCT, c_end - c0);
         const int nc4 = (nc + 3) & ~3;  // components past the last are staged as 0
         for (int e = tid; e < nc4 * (NCH * 2); e += NT) {
             const int cc = e / (NCH * 2), i = e % (NCH * 2);
@@ -472,6 +477,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
     // entries of several channels are read before the first is written, or each would wait for its
     // own: 2 points on 384 channels 114 -> 58 us, with 16 separate spans per wave instruction before.
     const int sc = lane >> 2, se = lane & 3;
+    const size_t fstride = 4 * (SLICED ? (size_t)a.ntiles * (a.ntiles - 1) / 2 : (size_t)a.nbl);
     auto entry = [&](int g, size_t &o) {  // the lane's entry of row g at channel f0; whether there is one
         const int r = row0 + wr * NG + g;
         int p, q;
@@ -490,27 +496,43 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
             valid = r > sc && pr.z >= 0 && q < a.ntiles;
         }
         if (!valid) p = 0, q = 1;
-        if (a.tile_map != nullptr) {
+        if (!SLICED && a.tile_map != nullptr) {
             p = a.tile_map[p];
             q = a.tile_map[q];
         }
-        const size_t nt = a.tile_map != nullptr ? (size_t)a.ntiles_bl : (size_t)a.ntiles;
+        const size_t nt = !SLICED && a.tile_map != nullptr ? (size_t)a.ntiles_bl : (size_t)a.ntiles;
         const size_t bl = (size_t)p * nt - (size_t)p * (p + 1) / 2 + (size_t)(q - p - 1);
-        o = ((size_t)f0 * a.nbl + bl) * 4 + se;
+        o = (f0 * (fstride / 4) + bl) * 4 + se;
         return valid;
     };
     float2 *const vis32 = reinterpret_cast<float2 *>(a.vis32);
     double2 *const vis64 = reinterpret_cast<double2 *>(a.vis64);
-    const size_t fstride = (size_t)a.nbl * 4;
-    auto add = [&](bool on, size_t o, float2 t, double2 d, double re, double im) {
+    auto value = [&](double re, double im) {
         const double ore = __shfl_xor(re, 3), oim = __shfl_xor(im, 3);
-        const double vr = se == 1 ? re - oim : (se == 2 ? ore + im : re);
-        const double vi = se == 1 ? im + ore : (se == 2 ? oim - re : im);
+        return make_double2(se == 1 ? re - oim : (se == 2 ? ore + im : re), se == 1 ? im + ore : (se == 2 ? oim - re : im));
+    };
+    auto add = [&](bool on, size_t o, float2 t, double2 d, double re, double im) {
+        const double2 v = value(re, im);
+        const double vr = v.x, vi = v.y;
         if (!on) return;
         vis32[o] = make_float2(t.x + (float)vr, t.y + (float)vi);
         if (vis64 != nullptr) vis64[o] = make_double2(d.x + vr, d.y + vi);
     };
-    if (WC == 1) {
+    if (SLICED) {
+        static_assert(!SLICED || WC == 1, "one wave has a component's sums");
+        // This slice's sums; k_tiles_finish adds the slices to the visibilities.
+        double2 *const out = a.part + (size_t)slice * a.nchan * fstride;
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            size_t o;
+            const bool valid = entry(g, o);
+#pragma unroll
+            for (int k = 0; k < NCH; ++k) {
+                const double2 v = value(acc[k][g][0], acc[k][g][1]);
+                if (valid && k < cnt) out[o + k * fstride] = v;
+            }
+        }
+    } else if (WC == 1) {
         constexpr int KB = 8;  // channels read at a time
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
@@ -568,6 +590,36 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
     }
 }
 
+// The component slices' sums, added in order to the visibilities: one thread per (channel, baseline,
+// entry), baselines numbered over the kernel's tiles.
+__global__ void k_tiles_finish(const TiledArgs a) {
+    const size_t npl = (size_t)a.ntiles * (a.ntiles - 1) / 2, n = a.nchan * npl * 4;
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double re = 0.0, im = 0.0;
+#pragma unroll 4
+    for (int s = 0; s < a.slices; ++s) {
+        const double2 v = a.part[s * n + i];
+        re += v.x;
+        im += v.y;
+    }
+    size_t o = i;
+    if (a.tile_map != nullptr) {
+        const size_t f = i / (npl * 4);
+        int p, q;
+        triangle_pair((int)(i / 4 - f * npl), a.ntiles, p, q);
+        p = a.tile_map[p];
+        q = a.tile_map[q];
+        o = (f * a.nbl + (size_t)p * a.ntiles_bl - (size_t)p * (p + 1) / 2 + (size_t)(q - p - 1)) * 4 + (i & 3);
+    }
+    float2 &t = reinterpret_cast<float2 *>(a.vis32)[o];
+    t = make_float2(t.x + (float)re, t.y + (float)im);
+    if (a.vis64 != nullptr) {
+        double2 &d = reinterpret_cast<double2 *>(a.vis64)[o];
+        d = make_double2(d.x + re, d.y + im);
+    }
+}
+
 // Tile-group pairs: off-diagonal (0, g0, g1) with g0 < g1, then diagonal groups paired from
 // both ends (1, g, G-1-g), the middle one alone (1, g, -1) when G is odd.
 std::vector<int4> tile_pairs(int ntiles) {
@@ -580,11 +632,17 @@ std::vector<int4> tile_pairs(int ntiles) {
     return out;
 }
 
-template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW>
+template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW, bool SLICED = false>
 static hipError_t launch_tiles_form(TiledArgs a, hipStream_t stream) {
+    if (WC == 1 && !SLICED && a.part != nullptr)
+        return launch_tiles_form<KIND, NCH, NG, WR, WC, NARROW, WC == 1>(a, stream);
     a.nchunks = chunk_count(a.chunks, NCH, a.nchan);
-    hipLaunchKernelGGL((k_tiles_mfma<KIND, NCH, NG, WR, WC, NARROW>),
-                       dim3((unsigned)(a.npairs * a.nchunks * (kTG / (NG * WR)))), dim3(64 * WR * WC), 0, stream, a);
+    hipLaunchKernelGGL((k_tiles_mfma<KIND, NCH, NG, WR, WC, NARROW, SLICED>),
+                       dim3((unsigned)(a.npairs * a.nchunks * (kTG / (NG * WR)) * a.slices)), dim3(64 * WR * WC), 0, stream, a);
+    if (a.part != nullptr) {
+        const size_t n = (size_t)a.nchan * a.ntiles * (a.ntiles - 1) * 2;
+        hipLaunchKernelGGL(k_tiles_finish, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, a);
+    }
     return hipGetLastError();
 }
 
@@ -597,7 +655,14 @@ static hipError_t launch_tiles_form(TiledArgs a, hipStream_t stream) {
 // against 38 and 59 us. Splitting the components over eight waves costs 1.5 times the widest form's
 // time on a full chip, but its blocks are 4 rows high: 90 points on 2 channels take 13 us, 4 wide,
 // against 32 us.
-template <int KIND, bool NARROW> static hipError_t launch_tiles(const TiledArgs &a, hipStream_t stream) {
+// A form whose waves hold whole components (all but the last two) may also run slices of the components,
+// of at least 128, in blocks of their own: their FP64 sums are written, read and added to the
+// visibilities (at about 4 TB/s), after one more launch. 128 tiles, 27 of 32 channels: 5600 points 1012 ->
+// 673 us, 2000 Gaussians 561 -> 402 us; calls of 10000 points for 32 tiles and 32 channels 728 -> 175 us,
+// 20000 for 48 tiles and 2 channels 1418 -> 270 us. The estimate's line between k blocks a CU is
+// straight from one (`single`) to the most it holds (`full`).
+template <int KIND, bool NARROW>
+static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t stream) {
     constexpr bool g = KIND == KIND_GAUSSIAN;
     struct Form {
         int nch, sub, resident;
@@ -608,19 +673,39 @@ template <int KIND, bool NARROW> static hipError_t launch_tiles(const TiledArgs 
                            {8, 2, 768, 9.0, g ? 0.47 : 0.27, g ? 0.235 : 0.15},
                            {8, 4, 256, 5.9, g ? 0.109 : 0.0704, g ? 0.109 : 0.0704},
                            {4, 4, 512, 4.8, g ? 0.168 : 0.0780, g ? 0.07 : 0.05}};
-    int best = -1;
-    double t_best = 0.0;
-    for (int i = 0; i < 5; ++i) {
-        if (i == 0 && !a.even16) continue;
-        const Form &f = forms[i];
-        const double r = (double)a.npairs * f.sub * chunk_count(a.chunks, f.nch, a.nchan) / f.resident;
-        const double rounds = r <= 1.0 ? r : 0.5 * (r + ceil(r));
-        const double t = fmax(r, 1.0) * f.fixed + a.ncomp * fmax(f.single, f.full * rounds);
-        if (best < 0 || t < t_best) {
-            best = i;
-            t_best = t;
+    const size_t n = (size_t)a_in.nchan * a_in.ntiles * (a_in.ntiles - 1) * 2;  // entries of a slice's sums
+    int best = -1, slices = 1;
+    auto choose = [&](int most) {
+        best = -1;
+        double t_best = 0.0;
+        for (int i = 0; i < 5; ++i) {
+            if (i == 0 && !a_in.even16) continue;
+            const Form &f = forms[i];
+            for (int s = 1; s == 1 || (i < 3 && s <= most && s <= a_in.ncomp / 128); ++s) {
+                const double blocks = (double)a_in.npairs * f.sub * chunk_count(a_in.chunks, f.nch, a_in.nchan) * s;
+                const double r = blocks / f.resident, m = f.resident / 256, k = fmin(ceil(blocks / 256), m);
+                const double per_comp = r > 1.0 ? f.full * 0.5 * (r + ceil(r))
+                                                : f.single + (m > 1.0 ? (f.full - f.single) * (k - 1.0) / (m - 1.0) : 0.0);
+                double t = fmax(r, 1.0) * f.fixed + (double)a_in.ncomp / s * per_comp;
+                if (s > 1) t += 5.0 + n * s * 32.0 / 4e6;
+                if (best < 0 || t < t_best) {
+                    best = i;
+                    slices = s;
+                    t_best = t;
+                }
+            }
         }
+    };
+    choose(part != nullptr ? (int)std::min<size_t>(16, a_in.part_limit / (sizeof(double2) * std::max<size_t>(n, 1))) : 1);
+    TiledArgs a = a_in;
+    a.part = nullptr;
+    if (slices > 1 && part->reserve(sizeof(double2) * n * slices) != hipSuccess) {
+        (void)hipGetLastError();  // no room for the slices' sums
+        choose(1);
     }
+    a.slices = slices;
+    if (slices > 1) a.part = part->as<double2>();
+    a.slice_len = ((a.ncomp + slices - 1) / slices + kCT - 1) / kCT * kCT;
     switch (best) {
     case 0: return launch_tiles_form<KIND, 16, 2, 4, 1, NARROW>(a, stream);
     case 1: return launch_tiles_form<KIND, 8, 4, 4, 1, NARROW>(a, stream);
@@ -630,7 +715,7 @@ template <int KIND, bool NARROW> static hipError_t launch_tiles(const TiledArgs 
     }
 }
 
-hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a_in, hipStream_t stream) {
+hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a_in, DevBuf *part, hipStream_t stream) {
     if (a_in.ncomp <= 0 || a_in.nbl <= 0 || a_in.nchan <= 0) return hipSuccess;
     TiledArgs a = a_in;
     if (a.coh32 != nullptr) {
@@ -640,9 +725,9 @@ hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a_in, hipStream_t str
                            dim3(256), 0, stream, a);
         return hipGetLastError();
     }
-    return kind == KIND_GAUSSIAN ? (a.narrow ? launch_tiles<KIND_GAUSSIAN, true>(a, stream)
-                                             : launch_tiles<KIND_GAUSSIAN, false>(a, stream))
-                                 : launch_tiles<KIND_POINT, true>(a, stream);
+    return kind == KIND_GAUSSIAN ? (a.narrow ? launch_tiles<KIND_GAUSSIAN, true>(a, part, stream)
+                                             : launch_tiles<KIND_GAUSSIAN, false>(a, part, stream))
+                                 : launch_tiles<KIND_POINT, true>(a, part, stream);
 }
 
 // ------------------------------------------------------------------ pairs with own beams

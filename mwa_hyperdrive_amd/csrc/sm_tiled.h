@@ -1,6 +1,7 @@
 // Arguments of the tiled point/Gaussian kernel and the channel-per-lane shapelet kernel.
 #pragma once
 
+#include <cstdint>
 #include <vector>
 
 #include "sm_internal.h"
@@ -36,6 +37,11 @@ struct TiledArgs {
     bool narrow = false;
     // Chunks of 16 channels are evenly spaced too (always with chunk tables).
     bool even16 = false;
+    // Set by the launcher: slices of slice_len components, whose sums go to part [slice][channel]
+    // [baseline of the kernel's tiles][4] when there are several.
+    int slices = 1, slice_len = 0;
+    double2 *part = nullptr;
+    size_t part_limit = SIZE_MAX;  // bytes that part may take
 };
 
 struct ShapeletChanArgs {
@@ -119,7 +125,8 @@ std::vector<int4> tile_pairs(int ntiles);
 hipError_t launch_pair_jones(Kind kind, const PairJonesArgs &a, DevBuf *accum, hipStream_t stream);
 // part (nullable) backs slices of the components, which few row tiles take.
 hipError_t launch_direct_rect(Kind kind, const RectArgs &a, DevBuf *part, hipStream_t stream);
-hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a, hipStream_t stream);
+// part (nullable) backs slices of the components, which few blocks of many components take.
+hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a, DevBuf *part, hipStream_t stream);
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream);
 hipError_t launch_tile_uvw_from_baselines(int ntiles, const UVW *d_uvw, double *d_out, hipStream_t stream);
 // FP64 -> FP32 copy of n values (coherency tables, basis table).

@@ -73,3 +73,11 @@ def test_envelope_forms_agree_with_the_baseline_kernel():
         finally:
             _lib.call("sm_set_direct_variant", 0)
         assert rel_err(got, want) <= 1e-12
+
+
+# Few blocks of many components take slices of the components (at least 128 each), the last one
+# shorter or of a ragged stage.
+@pytest.mark.parametrize("gaussian", [False, True], ids=["point", "gaussian"])
+@pytest.mark.parametrize("nt,nchan,ncomp", [(2, 1, 257), (17, 9, 1500), (33, 17, 1025), (49, 2, 2099), (65, 28, 700)])
+def test_component_slices_vs_oracle(nt, nchan, ncomp, gaussian):
+    check(nt, 167e6 + 40e3 * np.arange(nchan), sky(np.random.default_rng(ncomp), ncomp, gaussian))

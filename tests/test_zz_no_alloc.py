@@ -81,3 +81,13 @@ def test_noalloc_rejects_calls_beyond_the_scratch_array():
                   p(case["d_beam"]), p(v32), None)
     torch.cuda.synchronize()
     assert float(v32.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("nt,nchan,n_each", [(33, 24, 400), (5, 3, 900), (128, 40, 250), (128, 16, 4000)])
+def test_noalloc_matches_on_component_slices(nt, nchan, n_each):
+    """Sizes whose components are split into slices where the array has room for their sums."""
+    case = _case(6, nt, nchan, n_each, False)
+    want32, want64 = _run("sm_model_points_f64", case)
+    got32, got64 = _run("sm_model_points_noalloc", case)
+    np.testing.assert_array_equal(got64, want64)
+    np.testing.assert_array_equal(got32, want32)
