@@ -128,19 +128,6 @@ void cross_uvws(const std::vector<double> &xyz, int nt, double ha, double dec, s
         }
 }
 
-// HADec::to_azel (ERFA hd2ae formulation), returns (az, za).
-void azza(double ha, double dec, double lat, double &az, double &za) {
-    const double s_ha = std::sin(ha), c_ha = std::cos(ha), s_dec = std::sin(dec), c_dec = std::cos(dec);
-    const double s_lat = std::sin(lat), c_lat = std::cos(lat);
-    const double x = -c_ha * c_dec * s_lat + s_dec * c_lat;
-    const double y = -s_ha * c_dec;
-    const double z = c_ha * c_dec * c_lat + s_dec * s_lat;
-    const double r = std::hypot(x, y);
-    const double a = r != 0.0 ? std::atan2(y, x) : 0.0;
-    az = a < 0.0 ? a + kTau : a;
-    za = 1.5707963267948966 - std::atan2(z, r);
-}
-
 // Hermite-function table B_n(x_j), x_j = j/100 - 50 (src/model/make_shapelet_basis_values.py),
 // by the normalised recurrence B_{n+1} = sqrt(2/(n+1)) x B_n - sqrt(n/(n+1)) B_{n-1}.
 std::vector<double> shapelet_table() {
@@ -173,7 +160,7 @@ struct HostType {
 
 struct DevType {
     DevBuf lmn, shape, pl_fds, pl_sis, cpl_fds, cpl_sis, cpl_qs, list_fds, coeffs, ranges;
-    DevBuf bl_uv, hadec, az, za, beam, coh;
+    DevBuf bl_uv, hadec, radec, az, za, beam, coh;
     HostType h;
 };
 
@@ -373,6 +360,7 @@ const char *set_components(SmModeller *m, const SmComponent *const *comps, int n
         SM_TRY(upload(d.list_fds, h.list_fds));
         SM_TRY(upload(d.coeffs, h.coeffs));
         SM_TRY(upload(d.ranges, h.ranges));
+        if (m->beam_type != SM_BEAM_NONE) SM_TRY(upload(d.radec, h.radec));
         d.h = std::move(h);
     }
     return nullptr;
@@ -411,10 +399,9 @@ const char *prepare_beam(SmModeller *m, DevType &d, double lst, double latitude,
     b.dir_offset = 0;
     b.uniform_row = 0;
     if (m->beam_type == SM_BEAM_NONE || n == 0) return nullptr;
-    std::vector<double> az(n), za(n);
-    for (int i = 0; i < n; ++i) azza(lst - d.h.radec[i].ra, d.h.radec[i].dec, latitude, az[i], za[i]);
-    SM_TRY(upload(d.az, az));
-    SM_TRY(upload(d.za, za));
+    SM_TRY(d.az.reserve(sizeof(double) * n));
+    SM_TRY(d.za.reserve(sizeof(double) * n));
+    SM_TRY(launch_azza(n, d.radec.as<RADec>(), lst, latitude, d.az.as<double>(), d.za.as<double>(), 0));
     SM_TRY(d.beam.reserve(sizeof(JonesF64) * (size_t)m->n_utile * m->n_ufreq * n));
     if (m->surrogate != nullptr) {
         std::vector<uint32_t> dl;

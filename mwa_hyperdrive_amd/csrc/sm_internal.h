@@ -206,6 +206,9 @@ hipError_t launch_shapelet_bl_uv(int ncomp, int ntiles, int nbl, const double *d
 hipError_t launch_repack_shapelet_uv(int nbl, int n_pl, int n_cpl, int n_list, const ShapeletUV *pl,
                                      const ShapeletUV *cpl, const ShapeletUV *list, double2 *d_bl_uv,
                                      hipStream_t stream);
+// (az, za) of each component at the LST and latitude.
+hipError_t launch_azza(int n, const RADec *d_radec, double lst, double latitude, double *d_az, double *d_za,
+                       hipStream_t stream);
 hipError_t launch_analytic_beam(int n_tiles, const unsigned *d_delays, const double *d_gains, int n_freqs,
                                 const double *d_freqs, int n_dirs, const double *d_az, const double *d_za,
                                 JonesF64 *d_out, hipStream_t stream);
