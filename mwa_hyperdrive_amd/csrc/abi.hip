@@ -149,9 +149,10 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const bool hermitian = shared_tiled || shared_shapelet;
     // FP32 arithmetic (the precision path). Where that path's caller takes FP32 visibilities alone, an FP64
     // kernel stands in wherever it is the faster one (us a timestep, FP32 and FP64):
-    // - tile-pair Gaussians of at most one FP32 block a CU, which then runs all components in one chain:
-    //   64 tiles, 48 channels, 1000 components (64 blocks) 636 and 275; 101 tiles, 93 channels, 700
-    //   components (400 blocks) 581 and 653, and FP32 by 10 to 15% above;
+    // - tile-pair Gaussians of at most 400 FP32 blocks, which leave CUs idle or with one block where
+    //   the FP64 kernel takes slices of the components: 64 blocks (64 tiles, 48 channels, 1000
+    //   components) 635 and 248, 256 blocks (128, 48, 2000) 1244 and 832, 400 (101, 93, 700) 587
+    //   and 552, but 512 (128, 96, 2000) 1308 and 1450, 2048 (256, 96, 2000) 3594 and 4146;
     // - row-by-column Gaussians: 128 tiles, 12 of them with their own beams, 96 channels, 2000
     //   components 3324 and 2227; 256 tiles, 26 such 6481 and 6214;
     // - shared-beam shapelets, unless few channels fall in one table cell: 200 components, 128 tiles,
@@ -162,7 +163,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const bool either = fp32_path && vis64 == nullptr;
     const int last128 = ctx.nchan % 128;
     const bool few_per_cell = ctx.step > 80e3 && (last128 == 0 || last128 > 64);
-    auto small_grid = [&](int npairs) { return (long)npairs * chunk_count(ctx.chunks, 6, ctx.nchan) <= 256; };
+    auto small_grid = [&](int npairs) { return (long)npairs * chunk_count(ctx.chunks, 6, ctx.nchan) <= 400; };
     const bool f32 =
         fp32_path && !(either && ((shared_shapelet && !few_per_cell) || (shared_tiled && small_grid(ctx.npairs))));
     const bool planes = shared_shapelet && !(f32 && ctx.d_sbf32 != nullptr);
