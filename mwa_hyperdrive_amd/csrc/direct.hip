@@ -26,13 +26,18 @@ namespace sm {
 // coh[c][f] = J S J^H (one shared beam row) or S; S from the power-law / curved-power-law
 // parameters at 150 MHz or the list table (src/gpu/model.cu:16-28,137-167). The Hermitian forms
 // hold 4 values per entry instead of 8, Re XX, Re XY, Im XY, Re YY (J S J^H with the same J on both
-// sides is Hermitian, as S is).
-__global__ void k_coherency(int ncomp, int nchan, int nchan_pad, const double *__restrict__ freqs, FluxBuckets fb,
+// sides is Hermitian, as S is). A block takes 16 components by 16 channels, so that the table (channels
+// adjacent) and the beam (components adjacent) are both touched in runs (8000
+// components, 768 channels 196 -> 157 us).
+constexpr int kCohC = 16, kCohF = 16;
+
+__global__ __launch_bounds__(kCohC *kCohF) void k_coherency(int ncomp, int nchan, int nchan_pad, const double *__restrict__ freqs, FluxBuckets fb,
                             BeamDesc beam, int apply_beam, int form, double *__restrict__ coh) {
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (size_t)ncomp * nchan_pad) return;
-    const int c = (int)(idx / nchan_pad);
-    const int f = (int)(idx % nchan_pad);
+    const int ngroups = (nchan_pad + kCohF - 1) / kCohF;
+    const int c = (int)(blockIdx.x / ngroups) * kCohC + (int)threadIdx.x / kCohF;
+    const int f = (int)(blockIdx.x % ngroups) * kCohF + (int)threadIdx.x % kCohF;
+    if (c >= ncomp || f >= nchan_pad) return;
+    const size_t idx = (size_t)c * nchan_pad + f;
     double *out = coh + idx * (form == COH_FULL ? 8 : 4);
     double *out2 = out + 2;  // the second half of the Hermitian form
     if (form == COH_HERMITIAN_PLANES) {
@@ -163,10 +168,9 @@ hipError_t launch_class_coherency(int nclass, int ncomp, int nchan, int nchan_pa
 hipError_t launch_coherency(int ncomp, int nchan, int nchan_pad, const double *d_freqs, FluxBuckets fb,
                             BeamDesc beam, bool apply_beam, double *d_coh, hipStream_t stream, CohForm form) {
     if (ncomp <= 0) return hipSuccess;
-    const size_t n = (size_t)ncomp * nchan_pad;
-    const unsigned blocks = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL(k_coherency, dim3(blocks), dim3(256), 0, stream, ncomp, nchan, nchan_pad, d_freqs, fb, beam,
-                       apply_beam ? 1 : 0, (int)form, d_coh);
+    const unsigned blocks = (unsigned)(((ncomp + kCohC - 1) / kCohC) * ((nchan_pad + kCohF - 1) / kCohF));
+    hipLaunchKernelGGL(k_coherency, dim3(blocks), dim3(kCohC * kCohF), 0, stream, ncomp, nchan, nchan_pad, d_freqs,
+                       fb, beam, apply_beam ? 1 : 0, (int)form, d_coh);
     return hipGetLastError();
 }
 
