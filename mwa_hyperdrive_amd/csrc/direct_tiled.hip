@@ -12,7 +12,7 @@
 // form for Gaussians, which keeps the products on the vector ALUs.
 //
 // k_shapelets (shapelets, FP64): the coefficient sums are formed once per run of channels within a
-// cell of the basis table. k_shapelet_chan_tiles32 (per-tile beams) and k_shapelet_chan32, FP32: one
+// cell of the basis table. k_shapelet_chan_tiles(32) (per-tile beams) and k_shapelet_chan32 (FP32): one
 // wave per baseline, one or two channels per lane; the basis-table positions x_pos = k f + 5000 of neighbouring
 // channels fall in the same or adjacent table cells, so each coefficient's table reads coalesce
 // across the wave instead of touching 64 unrelated cache lines.
@@ -1482,11 +1482,8 @@ __device__ __forceinline__ double readlane_f64(double v, int lane) {
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// Per-tile beams, FP32: one wave per baseline, one channel per lane. Held to 96 VGPRs (5 waves per
-// SIMD, a few spilled values) instead of 118 (4 waves): 256 tiles and 384 channels 66.2 -> 57.8 ms.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_shapelet_chan_tiles32(
-    const ShapeletChanArgs a) {
-    using T = float;
+// Per-tile beams: one wave per baseline, one channel per lane, the coefficients summed per channel.
+template <class T> __device__ __forceinline__ void shapelet_chan_tiles(const ShapeletChanArgs &a) {
     const int nbx = (a.nbl + 3) / 4;
     const int total = nbx * a.ngroups;
     int b = blockIdx.x;
@@ -1517,7 +1514,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         }
     }
     const PackedCoeff *__restrict__ packed = a.packed;
-    const T *__restrict__ sbf = a.sbf32;
+    const T *__restrict__ sbf = pick<T>(a.sbf, a.sbf32);
     // Per-wave windows of the basis table (kRows rows x kWin cells per axis).
     __shared__ T wx_lds[4][kRows][kWin], wy_lds[4][kRows][kWin];
     const int wv = threadIdx.x >> 6;
@@ -1678,7 +1675,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         const T pi = zr * ei + zi * er;
         T cj[8];
         if (cls >= 0) {
-            class_coh(a.coh_cls32 + (((size_t)cls * a.ncomp + c) * a.nchan_pad + f) * 8,
+            class_coh(pick<T>(a.beam.coh_cls, a.coh_cls32) + (((size_t)cls * a.ncomp + c) * a.nchan_pad + f) * 8,
                       herm, cj);
         } else {
             // J_p S J_q^H of the instrumental flux S (FP64 table) and the two tiles' beams.
@@ -1711,6 +1708,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 #pragma unroll
         for (int e = 0; e < 8; ++e) v64[e] += (double)two_level_sum(acc[0][e], tot[0][e]);
     }
+}
+
+// Held to 128 VGPRs in FP64 (4 waves per SIMD, a few spilled values) instead of 164 (3 waves), and to 96
+// in FP32 (5 waves) instead of 118: 256 tiles and 384 channels 129 -> 111 ms and 66.2 -> 57.8 ms.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_shapelet_chan_tiles(
+    const ShapeletChanArgs a) {
+    shapelet_chan_tiles<double>(a);
+}
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_shapelet_chan_tiles32(
+    const ShapeletChanArgs a) {
+    shapelet_chan_tiles<float>(a);
 }
 
 // Shared beam, FP32: one wave per baseline and 128 channels, two adjacent channels per lane
@@ -2420,10 +2428,15 @@ hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStr
     const bool f32 = a.coh32 != nullptr;
     if (f32 && (a.sbf32 == nullptr || (per_tile && a.beam.coh_cls != nullptr && a.coh_cls32 == nullptr)))
         return hipErrorInvalidValue;
-    if (!f32) return per_tile ? launch_shapelets<true>(a, stream) : launch_shapelets<false>(a, stream);
+    // Per-tile beams in FP64: runs of a table cell hold few channels of a wide step on long baselines, where
+    // the sums per channel are cheaper if the channels fill their 64 lanes. 500 components, 256 tiles
+    // within 3 km, 80 kHz: 384 channels 80 ms per channel and 91 ms per run, 96 channels (a group and a
+    // half) 26.7 and 24.4 ms.
+    const bool per_channel = per_tile && a.step >= 80e3 && (a.nchan % 64 == 0 || a.nchan % 64 > 32);
+    if (!f32 && !per_channel) return per_tile ? launch_shapelets<true>(a, stream) : launch_shapelets<false>(a, stream);
     // Per-tile beams: a.ngroups groups of 64 channels; FP32 shared beam: groups of 128 channels.
     const int total = ((a.nbl + 3) / 4) * (per_tile ? a.ngroups : (a.nchan + 127) / 128);
-    hipLaunchKernelGGL(per_tile ? k_shapelet_chan_tiles32 : k_shapelet_chan32, dim3(total), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(!per_tile ? k_shapelet_chan32 : (f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles), dim3(total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

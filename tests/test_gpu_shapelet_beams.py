@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("limit", [-1, 0], ids=["class-table", "no-table"])
 @pytest.mark.parametrize("nt,dead,nchan,ncomp,df", [(2, 1, 1, 1, 40e3), (5, 2, 33, 17, 40e3), (6, 5, 65, 9, 1.28e6),
-                                                    (7, 3, 129, 35, 10e3), (9, 4, 70, 18, 160e3)])
+                                                    (7, 3, 129, 35, 10e3), (9, 4, 70, 18, 160e3), (4, 2, 97, 9, 80e3),
+                                                    (4, 2, 96, 9, 80e3)])
 def test_per_tile_beams_vs_oracle(nt, dead, nchan, ncomp, df, limit):
     rng = np.random.default_rng(nt)
     ra, dec = synthetic.cap_positions(rng, ncomp, 10.0)
