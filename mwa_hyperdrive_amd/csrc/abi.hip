@@ -153,8 +153,9 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     //   the FP64 kernel takes slices of the components: 64 blocks (64 tiles, 48 channels, 1000
     //   components) 635 and 248, 256 blocks (128, 48, 2000) 1244 and 832, 400 (101, 93, 700) 587
     //   and 552, but 512 (128, 96, 2000) 1308 and 1450, 2048 (256, 96, 2000) 3594 and 4146;
-    // - row-by-column Gaussians: 128 tiles, 12 of them with their own beams, 96 channels, 2000
-    //   components 3324 and 2227; 256 tiles, 26 such 6481 and 6214;
+    // - row-by-column Gaussians of at most one round of FP32 blocks (three a CU): 128 tiles, 12 of them
+    //   with their own beams, 96 channels, 2000 components (96 blocks) 3324 and 2227; 256 tiles, 26 such,
+    //   10000 components, the kernel alone: 96 channels (448 blocks) 8820 and 7540, 384 (1792) 25750 and 29400;
     // - shared-beam shapelets, unless few channels fall in one table cell: 200 components, 128 tiles,
     //   96 channels of 10 kHz 1664 and 969; 100 components, 256 tiles within 3 km, 93 of 80 kHz 4529 and 4401;
     //   128 tiles within 3 km, 96 of 160 kHz 3130 and 3691 (256 tiles, 48 of 160 kHz, which fill less
@@ -270,12 +271,15 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         DevBuf &cseg = scratch.cseg, &ccls = scratch.ccls;
         const int nseg = 2 * (ctx.nclass - 1);
         const size_t ccls_bytes = (size_t)ctx.nclass * n * ctx.nchan_pad * 8 * sizeof(double);
+        const bool rect32 = f32 && !(either && (long)((ctx.n_other + 3) / 4) * ((ctx.g0_n + 63) / 64) *
+                                                       chunk_count(ctx.chunks, 6, ctx.nchan) <= 768);
         const bool rect = e == hipSuccess && ctx.n_other > 0 && ctx.d_other_tiles != nullptr && ctx.nclass > 1 &&
                           reserve_class_table(ccls, ccls_bytes);
         if (rect) {
             e = launch_class_coherency(ctx.nclass, n, ctx.nchan, ctx.nchan_pad, coh.as<double>(), ctx.beam,
                                        ctx.d_class_row, ccls.as<double>(), stream);
-            if (e == hipSuccess && f32 && !either) e = to_f32(scratch.ccls32, (size_t)ctx.nclass * coh_n, ccls.as<double>(), stream);
+            if (e == hipSuccess && rect32)
+                e = to_f32(scratch.ccls32, (size_t)ctx.nclass * coh_n, ccls.as<double>(), stream);
             if (e == hipSuccess) {
                 RectArgs r;
                 r.n_row = ctx.n_other;
@@ -293,7 +297,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
                 r.lmn = in.lmn;
                 r.shape = in.shape;
                 r.coh_cls = ccls.as<double>();
-                if (f32 && !either) r.coh_cls32 = scratch.ccls32.as<float>();
+                if (rect32) r.coh_cls32 = scratch.ccls32.as<float>();
                 r.vis32 = vis32;
                 r.vis64 = vis64;
                 r.chunks = ctx.chunks;
