@@ -665,8 +665,8 @@ extern "C" const char *sm_model_points_noalloc(const Points *p, const Addresses 
     st.scratch.accum.borrow(static_cast<unsigned char *>(base) + off, (size_t)SM_NOALLOC_SCRATCH_BYTES - off);
     // Buffers the point path never reserves: borrowed with no capacity, so that any use
     // fails with an error instead of allocating.
-    for (DevBuf *b : {&st.shape, &st.bl_uv, &st.coeffs, &st.coeff_range, &st.sbf, &st.accum, &st.scratch.cls, &st.scratch.prange, &st.scratch.packed, &st.scratch.coh0, &st.scratch.cseg,
-                      &st.scratch.ccls})
+    for (DevBuf *b : {&st.shape, &st.bl_uv, &st.coeffs, &st.coeff_range, &st.sbf, &st.accum, &st.scratch.cls,
+                      &st.scratch.prange, &st.scratch.packed, &st.scratch.coh0, &st.scratch.cseg, &st.scratch.ccls})
         b->borrow(nullptr, 0);
     return model_points_with(st, p, a, d_uvws, d_beam_jones, d_vis_fb, d_vis_fb_f64);
 }

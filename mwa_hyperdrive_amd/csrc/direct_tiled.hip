@@ -11,10 +11,12 @@
 // paired so that 240 of 256 pairs are wanted ones. k_direct_tiled is the precision path's FP32
 // form for Gaussians, which keeps the products on the vector ALUs.
 //
+// k_rect_mfma does the same for pairs of a tile with its own beam and one of the shared beam.
+//
 // k_shapelets (shapelets, FP64): the coefficient sums are formed once per run of channels within a
-// cell of the basis table. k_shapelet_chan_tiles(32) (per-tile beams) and k_shapelet_chan32 (FP32): one
-// wave per baseline, one or two channels per lane; the basis-table positions x_pos = k f + 5000 of neighbouring
-// channels fall in the same or adjacent table cells, so each coefficient's table reads coalesce
+// cell of the basis table. k_shapelet_chan_tiles(32) (per-tile beams) and k_shapelet_chan32 (FP32):
+// one wave per baseline, one or two channels per lane; the table positions x_pos = k f + 5000 of
+// neighbouring channels fall in the same or adjacent table cells, so each coefficient's table reads coalesce
 // across the wave instead of touching 64 unrelated cache lines.
 #include "sm_internal.h"
 #include "sm_jones.h"
@@ -1104,8 +1106,8 @@ __global__ __launch_bounds__(64 * kRectWR, 2) void k_rect_mfma(const RectArgs a,
     const int nrg = (a.n_row + WR - 1) / WR, ncg = (a.n_col + NC - 1) / NC;
     // Consecutive blocks of one XCD (blockIdx modulo 8) take the column groups of the same rows,
     // channels and components, which share their C in its L2.
-    const int total = gridDim.x / 8 * 8;
-    const int vb = (int)blockIdx.x < total ? (int)(blockIdx.x & 7) * (total >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    const int bid = blockIdx.x, per = gridDim.x >> 3;
+    const int vb = bid < per * 8 ? (bid & 7) * per + (bid >> 3) : bid;
     const int slice = vb / per_slice, b = vb - slice * per_slice;
     const int chunk = b / (nrg * ncg), rem = b - chunk * (nrg * ncg);
     const int rg = rem / ncg, cg = rem - rg * ncg;
@@ -2436,7 +2438,8 @@ hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStr
     if (!f32 && !per_channel) return per_tile ? launch_shapelets<true>(a, stream) : launch_shapelets<false>(a, stream);
     // Per-tile beams: a.ngroups groups of 64 channels; FP32 shared beam: groups of 128 channels.
     const int total = ((a.nbl + 3) / 4) * (per_tile ? a.ngroups : (a.nchan + 127) / 128);
-    hipLaunchKernelGGL(!per_tile ? k_shapelet_chan32 : (f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles), dim3(total), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(!per_tile ? k_shapelet_chan32 : (f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles),
+                       dim3(total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
