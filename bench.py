@@ -40,15 +40,12 @@ PEAK_HBM_GBS = 8000.0
 # Algorithmic FP64 work of the point tile-pair kernel per comp.vis: the 4 Jones entries'
 # coherency x phasor accumulations, which with one beam on both sides take the Hermitian form
 # (XX and YY real, YX = conj(XY): Re XX, Re XY, Im XY and Re YY times the complex phasor, 8
-# FMAs = 16), the phasor's advance across the chunk's channels (6), the tile-phasor product at
-# the chunk's first channel shared by its 4 channels (1.5), and the tile phasors themselves,
-# shared by 256 baselines (under 0.5). The reference kernel's per comp.vis J S J^H (112 FLOP)
+# FMAs = 16), the phasor's advance across the chunk's channels (a two-term recurrence, 2 FMAs = 4),
+# the tile-phasor products at the chunk's middle channel and one channel step, shared by its 16
+# channels (about 1), and the tile phasors themselves (under 0.5). The reference kernel's per comp.vis J S J^H (112 FLOP)
 # and per-baseline sincos are not part of this algorithm: J S J^H is formed once per
 # (component, channel) and the phase factorises over antennas.
-FLOP_PER_COMPVIS_POINT = 24.0
-# The same terms in the full complex form (4 complex multiply-adds = 32 instead of 16), as the
-# shapelet kernel computes them.
-FLOP_PER_COMPVIS_POINT_FULL = 40.0
+FLOP_PER_COMPVIS_POINT = 21.0
 
 
 def cpu_model_name() -> str:
@@ -138,24 +135,18 @@ def host_entry_c2(obs, timesteps: int = 2) -> dict:
             "vis_bytes_each_way": vis.nbytes, "timesteps": timesteps}
 
 
-FLOP_PER_COMPVIS_GAUSSIAN = FLOP_PER_COMPVIS_POINT + 21.0  # (kx, ky) 6, quadratic form 5, x K 1, exp 1, scale 8
+# The envelope's product (2) and advance (2), and its quadratic form and three exponentials, shared by
+# 16 channels (1).
+FLOP_PER_COMPVIS_GAUSSIAN = FLOP_PER_COMPVIS_POINT + 5.0
+# The accumulation (16), the phasor's advance (4) and its product with the envelope (6), the envelope's
+# two quadratics in frequency (8) and the position of its run (6). The coefficient sums, once per run
+# of channels in a table cell, are not counted.
+FLOP_PER_COMPVIS_SHAPELET = 40.0
 KERNEL_NAMES = {
-    "points": "k_direct_tiled<point> (FP64 tile-pair phasor kernel)",
-    "gaussians": "k_direct_tiled<gaussian> (FP64 tile-pair phasor kernel)",
-    "shapelets": "k_shapelet_chan (FP64 shapelet kernel, two channels per lane)",
+    "points": "k_tiles_mfma<point> (FP64 tile-pair kernel on the 4x4x4 matrix instruction)",
+    "gaussians": "k_tiles_mfma<gaussian> (FP64 tile-pair kernel on the 4x4x4 matrix instruction)",
+    "shapelets": "k_shapelets (FP64 shapelet kernel, coefficient sums per run of channels)",
 }
-
-
-def shapelet_flop(obs) -> float:
-    """Executed FP64 work per shapelet comp.vis: the point terms, 34 for the rotation,
-    positions and complex envelope, and 9 per coefficient (two table interpolations, the
-    product and the complex accumulation), at the sky's mean coefficient count."""
-    from mwa_hyperdrive_amd.srclist import Shapelet
-
-    counts = [len(c.comp_type.coeffs) for src in obs.srclist.values() for c in src.components
-              if isinstance(c.comp_type, Shapelet)]
-    mean = sum(counts) / len(counts) if counts else 0.0
-    return FLOP_PER_COMPVIS_POINT_FULL + 34.0 + 9.0 * mean
 
 
 def split_precision() -> dict:
@@ -509,7 +500,7 @@ def main() -> int:
     per_kernel = {}
     for ty, key, flop in (("points", "num_points", FLOP_PER_COMPVIS_POINT),
                           ("gaussians", "num_gaussians", FLOP_PER_COMPVIS_GAUSSIAN),
-                          ("shapelets", "num_shapelets", shapelet_flop(obs))):
+                          ("shapelets", "num_shapelets", FLOP_PER_COMPVIS_SHAPELET)):
         ms = info[f"kernel_ms_{ty}"] / launches_per_type
         fl = flop * info[key] * nbf
         per_kernel[ty] = {"avg_launch_ms": ms, "flop_per_comp_vis": flop,
