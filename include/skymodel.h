@@ -185,6 +185,14 @@ const char *sm_synchronize(void);
  * kernels everywhere. Process-wide; used to compare the two. */
 const char *sm_set_direct_variant(int32_t variant);
 
+/* Which form of the FP64 tile-pair kernel, and how many slices of the components, a timestep of a
+ * modeller takes for its points or Gaussians where num_tiles tiles share a beam: 0 = 16 channels wide,
+ * 1 = 8 channels and 16 rows of tiles a block, 2 = 8 channels and 8 rows, 3 and 4 = 8 and 4 channels
+ * with the components over eight waves. Sizes only, no device; used to test every form. No
+ * counterpart in the reference. */
+const char *sm_tiles_form(int32_t gaussian, int32_t num_tiles, int32_t num_freqs, const double *freqs,
+                          int32_t num_comps, int32_t *form, int32_t *slices);
+
 /* Limit in bytes on the per-beam-row-class coherency tables the per-tile-beam paths build
  * (J_r S J_0^H for every class; 64 B per class, component and padded channel). Above it, or
  * when the allocation fails, those paths form the coherency per baseline segment instead,

@@ -884,6 +884,25 @@ extern "C" const char *sm_set_class_table_limit(int64_t bytes) {
     return nullptr;
 }
 
+extern "C" const char *sm_tiles_form(int32_t gaussian, int32_t num_tiles, int32_t num_freqs, const double *freqs,
+                                     int32_t num_comps, int32_t *form, int32_t *slices) {
+    if (freqs == nullptr || form == nullptr || slices == nullptr) return "null argument";
+    if (num_tiles < 2 || num_freqs < 1 || num_comps < 1) return "no pairs of tiles, channels or components";
+    const std::vector<int2> c4 = even_chunks(freqs, num_freqs, 4), c6 = even_chunks(freqs, num_freqs, 6),
+                            c8 = even_chunks(freqs, num_freqs, 8), c16 = even_chunks(freqs, num_freqs, 16);
+    TiledArgs a{};
+    a.chunks = {c4.data(), (int)c4.size(), c6.data(), (int)c6.size(), c8.data(), (int)c8.size(), c16.data(), (int)c16.size()};
+    a.ntiles = num_tiles;
+    a.npairs = (int)tile_pairs(num_tiles).size();
+    a.nchan = num_freqs;
+    a.ncomp = num_comps;
+    a.even16 = true;
+    const TilesChoice t = choose_tiles_form(gaussian != 0, a, true);
+    *form = t.form;
+    *slices = t.slices;
+    return nullptr;
+}
+
 extern "C" const char *sm_set_direct_variant(int32_t variant) {
     if (variant < 0 || variant > 1) return "variant must be 0 (fastest) or 1 (baseline per lane)";
     sm::g_direct_variant = variant;

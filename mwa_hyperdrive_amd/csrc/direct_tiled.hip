@@ -663,9 +663,7 @@ static hipError_t launch_tiles_form(TiledArgs a, hipStream_t stream) {
 // 673 us, 2000 Gaussians 561 -> 402 us; calls of 10000 points for 32 tiles and 32 channels 728 -> 175 us,
 // 20000 for 48 tiles and 2 channels 1418 -> 270 us. The estimate's line between k blocks a CU is
 // straight from one (`single`) to the most it holds (`full`).
-template <int KIND, bool NARROW>
-static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t stream) {
-    constexpr bool g = KIND == KIND_GAUSSIAN;
+TilesChoice choose_tiles_form(bool g, const TiledArgs &a, bool may_slice) {
     struct Form {
         int nch, sub, resident;
         double fixed, full, single;  // us: per round; per component and round; per component, one block a CU
@@ -675,40 +673,40 @@ static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t 
                            {8, 2, 768, 9.0, g ? 0.47 : 0.27, g ? 0.235 : 0.15},
                            {8, 4, 256, 5.9, g ? 0.109 : 0.0704, g ? 0.109 : 0.0704},
                            {4, 4, 512, 4.8, g ? 0.168 : 0.0780, g ? 0.07 : 0.05}};
-    const size_t n = (size_t)a_in.nchan * a_in.ntiles * (a_in.ntiles - 1) * 2;  // entries of a slice's sums
-    int best = -1, slices = 1;
-    auto choose = [&](int most) {
-        best = -1;
-        double t_best = 0.0;
-        for (int i = 0; i < 5; ++i) {
-            if (i == 0 && !a_in.even16) continue;
-            const Form &f = forms[i];
-            for (int s = 1; s == 1 || (i < 3 && s <= most && s <= a_in.ncomp / 128); ++s) {
-                const double blocks = (double)a_in.npairs * f.sub * chunk_count(a_in.chunks, f.nch, a_in.nchan) * s;
-                const double r = blocks / f.resident, m = f.resident / 256, k = fmin(ceil(blocks / 256), m);
-                const double per_comp = r > 1.0 ? f.full * 0.5 * (r + ceil(r))
-                                                : f.single + (m > 1.0 ? (f.full - f.single) * (k - 1.0) / (m - 1.0) : 0.0);
-                double t = fmax(r, 1.0) * f.fixed + (double)a_in.ncomp / s * per_comp;
-                if (s > 1) t += 5.0 + n * s * 32.0 / 4e6;
-                if (best < 0 || t < t_best) {
-                    best = i;
-                    slices = s;
-                    t_best = t;
-                }
-            }
+    const size_t n = (size_t)a.nchan * a.ntiles * (a.ntiles - 1) * 2;  // entries of a slice's sums
+    const int most = may_slice ? (int)std::min<size_t>(16, a.part_limit / (sizeof(double2) * std::max<size_t>(n, 1))) : 1;
+    TilesChoice best{-1, 1, 0.0};
+    for (int i = 0; i < 5; ++i) {
+        if (i == 0 && !a.even16) continue;
+        const Form &f = forms[i];
+        for (int s = 1; s == 1 || (i < 3 && s <= most && s <= a.ncomp / 128); ++s) {
+            const double blocks = (double)a.npairs * f.sub * chunk_count(a.chunks, f.nch, a.nchan) * s;
+            const double r = blocks / f.resident, m = f.resident / 256, k = fmin(ceil(blocks / 256), m);
+            const double per_comp = r > 1.0 ? f.full * 0.5 * (r + ceil(r))
+                                            : f.single + (m > 1.0 ? (f.full - f.single) * (k - 1.0) / (m - 1.0) : 0.0);
+            double t = fmax(r, 1.0) * f.fixed + (double)a.ncomp / s * per_comp;
+            if (s > 1) t += 5.0 + n * s * 32.0 / 4e6;
+            if (best.form < 0 || t < best.us) best = TilesChoice{i, s, t};
         }
-    };
-    choose(part != nullptr ? (int)std::min<size_t>(16, a_in.part_limit / (sizeof(double2) * std::max<size_t>(n, 1))) : 1);
+    }
+    return best;
+}
+
+template <int KIND, bool NARROW>
+static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t stream) {
+    constexpr bool g = KIND == KIND_GAUSSIAN;
+    TilesChoice best = choose_tiles_form(g, a_in, part != nullptr);
     TiledArgs a = a_in;
     a.part = nullptr;
-    if (slices > 1 && part->reserve(sizeof(double2) * n * slices) != hipSuccess) {
+    const size_t n = (size_t)a.nchan * a.ntiles * (a.ntiles - 1) * 2;
+    if (best.slices > 1 && part->reserve(sizeof(double2) * n * best.slices) != hipSuccess) {
         (void)hipGetLastError();  // no room for the slices' sums
-        choose(1);
+        best = choose_tiles_form(g, a, false);
     }
-    a.slices = slices;
-    if (slices > 1) a.part = part->as<double2>();
-    a.slice_len = ((a.ncomp + slices - 1) / slices + kCT - 1) / kCT * kCT;
-    switch (best) {
+    a.slices = best.slices;
+    if (a.slices > 1) a.part = part->as<double2>();
+    a.slice_len = ((a.ncomp + a.slices - 1) / a.slices + kCT - 1) / kCT * kCT;
+    switch (best.form) {
     case 0: return launch_tiles_form<KIND, 16, 2, 4, 1, NARROW>(a, stream);
     case 1: return launch_tiles_form<KIND, 8, 4, 4, 1, NARROW>(a, stream);
     case 2: return launch_tiles_form<KIND, 8, 2, 4, 1, NARROW>(a, stream);

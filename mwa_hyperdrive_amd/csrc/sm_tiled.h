@@ -125,6 +125,13 @@ std::vector<int4> tile_pairs(int ntiles);
 hipError_t launch_pair_jones(Kind kind, const PairJonesArgs &a, DevBuf *accum, hipStream_t stream);
 // part (nullable) backs slices of the components, which few row tiles take.
 hipError_t launch_direct_rect(Kind kind, const RectArgs &a, DevBuf *part, hipStream_t stream);
+// The FP64 tile-pair kernel's form (0 .. 4: 16 channels wide, 8 with 16 rows a block, 8 with 8 rows, 8
+// and 4 with the components over eight waves), slices of the components and estimated time. Host only.
+struct TilesChoice {
+    int form, slices;
+    double us;
+};
+TilesChoice choose_tiles_form(bool gaussian, const TiledArgs &a, bool may_slice);
 // part (nullable) backs slices of the components, which few blocks of many components take.
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a, DevBuf *part, hipStream_t stream);
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream);
