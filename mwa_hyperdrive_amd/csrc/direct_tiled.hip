@@ -283,12 +283,28 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
 // l / 16, and accumulates e = l % 4 of baseline l / 4: a wave's stores are contiguous. The vector
 // ALUs only form z.
 
+// Lane `lane`'s value of v (every lane active), as a wave-uniform value.
+__device__ __forceinline__ double readlane_f64(double v, int lane) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), lane);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// A frequency over c in two doubles, kept in scalar registers (the same on every lane).
+__device__ __forceinline__ TwoDouble over_c(double f) {
+    const TwoDouble q = two_quotient(f, SM_VEL_C);
+    return {readlane_f64(q.hi, 0), readlane_f64(q.lo, 0)};
+}
+
 // z of the chunk's channels from the middle one outwards in both directions: evenly spaced
 // channels obey z_{k+1} = 2 cos(delta) z_k - z_{k-1}, one FMA per part, and starting in the middle
 // keeps the recurrence's error growth to (NCH / 2)^2 roundings. (a0, b0) are the tiles' phasors at
-// channel NCH / 2 - 1, (a1, b1) at one channel step's frequency: the step's small phase carries a
-// small rounding. Two neighbouring channels' phasors instead would have their independent phase
-// roundings, 1e-12 at 1e4 rad, extrapolated over the chunk.
+// channel NCH / 2 - 1, (a1, b1) at one channel step's frequency. Neither phase may be rounded to one
+// double (table_sincos_product): a run of two channels across a gap of the band starts NCH / 2 - 1 gaps
+// above its first channel, where such a rounding is several times the first channel's, and the step's
+// is carried back as often (100 and 300 MHz, tiles within 3 km: rms error of z 1.5e-12 with rounded
+// phases, 1.9e-13 without, as on any other band; most of that is theta's own rounding).
 template <int NCH>
 __device__ __forceinline__ void chunk_phasors(double2 a0, double2 a1, double2 b0, double2 b1, double (&zr)[NCH],
                                               double (&zi)[NCH]) {
@@ -339,14 +355,15 @@ __device__ __forceinline__ void gaussian_envelopes(double4 sh, double bu, double
 // FMAs of the recurrence. At 128 tiles, 768 channels: 5600 points 18.0 -> 13.7 ms (MFMA 53% and
 // other VALU 34% of the cycles, at 2.05 GHz), 2000 Gaussians 12.9 -> 7.8 ms (their exponentials
 // through table_exp: 10.1 -> 8.6 ms). Two waves per SIMD: the accumulators take 128 VGPRs. Four
-// waves of half the accumulators spill and run slower (15.5 and 23.7 ms).
+// waves of half the accumulators spill and run slower (15.5 and 23.7 ms). Points in the 4-channel form
+// are held to 128 VGPRs, two blocks a CU.
 //
 // A block owns R = NG * WR rows of one 16 x 16 tile-pair block and one chunk of at most NCH
 // channels. WR waves split the rows (NG each); WC waves split the components (each takes every
 // WC-th group of four of a stage), their sums meeting in LDS at the end. A chunk's coherencies are
 // read NCH wide whatever its count (TiledArgs::coh); what the extra channels accumulate is dropped.
 template <int KIND, int NCH, int NG, int WR, int WC, bool NARROW, bool SLICED>
-__global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs a) {
+__global__ __launch_bounds__(64 * WR * WC, KIND == KIND_POINT && NCH == 4 ? 4 : 2) void k_tiles_mfma(const TiledArgs a) {
     constexpr int R = NG * WR, SUB = kTG / R, NT = 64 * WR * WC;
     static_assert(kCT % (4 * WC) == 0, "a stage is whole groups of four components per wave");
     constexpr int KR = WC > 1 ? WC / NG : 1;  // channels reduced at a time (WC > 1)
@@ -408,7 +425,7 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
     const double F0 = freqs[f0];
     const double DF = freqs[f0 + 1] - F0;
     constexpr int m = NCH / 2 - 1;
-    const double fm0 = (F0 + m * DF) / SM_VEL_C, fm1 = DF / SM_VEL_C;
+    const TwoDouble fm0 = over_c(F0 + m * DF), fm1 = over_c(DF);
     const double4 *__restrict__ lmn4 = a.lmn;
     const double4 *__restrict__ shape = a.shape;
     const double *__restrict__ coh = a.coh + (size_t)f0 * 4;
@@ -439,8 +456,8 @@ __global__ __launch_bounds__(64 * WR * WC, 2) void k_tiles_mfma(const TiledArgs 
                 const double4 l = lmn4[c0 + cc];
                 const double2 uv = s_uv[slot];
                 const double th = uv.x * l.x + uv.y * l.y + s_w[slot] * l.z;
-                table_sincos(th * fm0, reinterpret_cast<const double *>(s_sc), s0, c0_);
-                table_sincos(th * fm1, reinterpret_cast<const double *>(s_sc), s1, c1);
+                table_sincos_product(th, fm0, reinterpret_cast<const double *>(s_sc), s0, c0_);
+                table_sincos_product(th, fm1, reinterpret_cast<const double *>(s_sc), s1, c1);
             }
             L.st.p0[cc][slot] = make_double2(c0_, s0);
             L.st.p1[cc][slot] = make_double2(c1, s1);
@@ -1128,7 +1145,7 @@ __global__ __launch_bounds__(64 * kRectWR, 2) void k_rect_mfma(const RectArgs a,
     const bool row_ok = w < rows;
     const int cq = 4 * (lane & 3) + ((lane >> 2) & 3), ck = lane >> 4, se = lane & 3;
     const double F0 = a.freqs[f0], DF = a.freqs[f0 + 1] - F0;
-    const double fm0 = (F0 + (NCH / 2 - 1) * DF) / SM_VEL_C, fm1 = DF / SM_VEL_C;
+    const TwoDouble fm0 = over_c(F0 + (NCH / 2 - 1) * DF), fm1 = over_c(DF);
     const double qmin = -800.0 / (F0 * F0), q0 = F0 * F0, q1 = DF * (2.0 * F0 + DF), q2 = 2.0 * DF * DF;
     const double4 *__restrict__ lmn4 = a.lmn;
     const double4 *__restrict__ shape = a.shape;
@@ -1165,8 +1182,8 @@ __global__ __launch_bounds__(64 * kRectWR, 2) void k_rect_mfma(const RectArgs a,
                 const double4 l = lmn4[c0 + cc];
                 const double2 uv = s_uv[slot];
                 const double th = uv.x * l.x + uv.y * l.y + s_w[slot] * l.z;
-                table_sincos(th * fm0, reinterpret_cast<const double *>(s_sc), s0, c0_);
-                table_sincos(th * fm1, reinterpret_cast<const double *>(s_sc), s1, c1);
+                table_sincos_product(th, fm0, reinterpret_cast<const double *>(s_sc), s0, c0_);
+                table_sincos_product(th, fm1, reinterpret_cast<const double *>(s_sc), s1, c1);
             }
             s_p0[cc][slot] = make_double2(c0_, s0);
             s_p1[cc][slot] = make_double2(c1, s1);
@@ -1474,14 +1491,6 @@ hipError_t launch_direct_rect(Kind kind, const RectArgs &a, DevBuf *part, hipStr
 }
 
 // ------------------------------------------------------------------ shapelets
-// Lane `lane`'s value of v (every lane active), as a wave-uniform value.
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, lane);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), lane);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
 // Per-tile beams: one wave per baseline, one channel per lane, the coefficients summed per channel.
 template <class T> __device__ __forceinline__ void shapelet_chan_tiles(const ShapeletChanArgs &a) {
     const int nbx = (a.nbl + 3) / 4;

@@ -99,11 +99,14 @@ SM_HD inline void fast_sincos(double x, double &s, double &c) {
 // and the Taylor series of sin r to r^9 and of cos r to r^8 leave remainders below 3e-20 at
 // |r| = pi/64. The reduction is fast_sincos's with a two-part pi/32 (P1 = pi/32 rounded to
 // double, P2 = the rest rounded to double, 32/pi rounded to double, all from a 300-bit pi).
-// Nine polynomial terms instead of twenty and no quadrant selection, for one table read.
-SM_HD inline void table_sincos(double x, const double *tab, double &s, double &c) {
-    const double k = rint(x * 10.185916357881302);
-    double r = fma(-k, 0.09817477042468103, x);
-    r = fma(-k, 3.827021247335479e-18, r);
+// Nine polynomial terms instead of twenty and no quadrant selection, for one table read. In two
+// steps: k and r of x, and sin and cos from them.
+SM_HD inline double table_reduce(double x, double &k) {
+    k = rint(x * 10.185916357881302);
+    return fma(-k, 3.827021247335479e-18, fma(-k, 0.09817477042468103, x));
+}
+
+SM_HD inline void table_reduced_sincos(double k, double r, const double *tab, double &s, double &c) {
     const double r2 = r * r;
     // coefficients (-1)^n / (2n+1)! and (-1)^n / (2n)!
     double ps = 2.7557319223985893e-06;
@@ -120,6 +123,33 @@ SM_HD inline void table_sincos(double x, const double *tab, double &s, double &c
     const double S = tab[2 * i], C = tab[2 * i + 1];
     s = fma(S, cr, C * sr);
     c = fma(C, cr, -(S * sr));
+}
+
+SM_HD inline void table_sincos(double x, const double *tab, double &s, double &c) {
+    double k;
+    const double r = table_reduce(x, k);
+    table_reduced_sincos(k, r, tab, s, c);
+}
+
+// A factor in two doubles, hi + lo.
+struct TwoDouble {
+    double hi, lo;
+};
+
+// a / b in two doubles (exact to about 2^-105 of it).
+SM_HD inline TwoDouble two_quotient(double a, double b) {
+    const double hi = a / b;
+    return {hi, fma(-hi, b, a) / b};
+}
+
+// sin and cos of x y with neither the product nor y rounded to one double: a phase of 1e4 rad
+// rounded to one is off by up to 9e-13. Three instructions more than table_sincos(x * y.hi).
+SM_HD inline void table_sincos_product(double x, TwoDouble y, const double *tab, double &s, double &c) {
+    const double p = x * y.hi;
+    const double lo = fma(x, y.lo, fma(x, y.hi, -p));
+    double k;
+    const double r = table_reduce(p, k);
+    table_reduced_sincos(k, r + lo, tab, s, c);
 }
 
 // 2^(j / 64) for j = 0 .. 63, each rounded to nearest from a 60-digit evaluation.
