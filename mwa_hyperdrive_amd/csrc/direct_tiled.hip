@@ -665,44 +665,53 @@ static hipError_t launch_tiles_form(TiledArgs a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Which form: the one with the smallest estimated time, from its blocks in units of what the 256
-// CUs hold at once (r), the time to start and end a block, and the time per component when the chip
-// is full and when a CU holds one block; all measured on 128 tiles. Two row groups of 16 channels
-// share a Gaussian's exponentials and a phasor's set-up over the most channels (768 channels, 5600
-// points 13.7 ms, 2000 Gaussians 7.8 ms; four row groups of 8 channels 13.7 and 8.3 ms). Two row
-// groups of 8 channels fill the chip sooner: 128 points and Gaussians on 32 channels 25 and 38 us,
-// against 38 and 59 us. Splitting the components over eight waves costs 1.5 times the widest form's
-// time on a full chip, but its blocks are 4 rows high: 90 points on 2 channels take 13 us, 4 wide,
-// against 32 us.
+// Components of a slice: whole stages.
+static int slice_length(int ncomp, int slices) { return ((ncomp + slices - 1) / slices + kCT - 1) / kCT * kCT; }
+
+// Which form: the one with the smallest estimated time. With k = ceil(blocks / 256) blocks for the CU
+// with the most, n components take start + start_block k + n (comp + comp_block k) us, whether a CU holds
+// one, two or three at once; the constants are fits to the kernel times of every form and slice count at
+// 381 sizes (9 to 256 tiles, 1 to 768 channels, 4 to 6000 components, points and Gaussians), each form's
+// within 6% rms. The form taken is 0.5% slower than the fastest on average, and more than 10% slower at 5
+// sizes of 762. Two row groups of 16 channels share a Gaussian's exponentials and a phasor's set-up over the
+// most channels (768 channels, 5600 points 13.7 ms, 2000 Gaussians 7.8 ms; four row groups of 8 channels
+// 13.7 and 8.3 ms). Two row groups of 8 channels fill the chip sooner: 100 points and Gaussians on 24
+// channels and 128 tiles 28 and 37 us, against 38 and 53 us. Splitting the components over eight waves
+// costs 1.5 times the widest form's time on a full chip, but its blocks are 4 rows high: 32 tiles, 64
+// channels, 100 points 16 us, 4 wide, against 39 us.
 // A form whose waves hold whole components (all but the last two) may also run slices of the components,
 // of at least 128, in blocks of their own: their FP64 sums are written, read and added to the
-// visibilities (at about 4 TB/s), after one more launch. 128 tiles, 27 of 32 channels: 5600 points 1012 ->
-// 673 us, 2000 Gaussians 561 -> 402 us; calls of 10000 points for 32 tiles and 32 channels 728 -> 175 us,
-// 20000 for 48 tiles and 2 channels 1418 -> 270 us. The estimate's line between k blocks a CU is
-// straight from one (`single`) to the most it holds (`full`).
+// visibilities, after one more launch (5 us; 4 TB/s, or 12 TB/s for sums that fit the last-level cache).
+// 128 tiles, 27 of 32 channels: 5600 points 1012 -> 673 us, 2000 Gaussians 561 -> 402 us; calls of 10000
+// points for 32 tiles and 32 channels 728 -> 175 us, 20000 for 48 tiles and 2 channels 1418 -> 270 us.
 TilesChoice choose_tiles_form(bool g, const TiledArgs &a, bool may_slice) {
     struct Form {
-        int nch, sub, resident;
-        double fixed, full, single;  // us: per round; per component and round; per component, one block a CU
+        int nch, sub;
+        double start, start_block, comp, comp_block;
     };
-    const Form forms[5] = {{16, 2, 512, 12.0, g ? 0.554 : 0.348, g ? 0.39 : 0.24},
-                           {8, 1, 512, 12.0, g ? 0.591 : 0.349, g ? 0.41 : 0.24},
-                           {8, 2, 768, 9.0, g ? 0.47 : 0.27, g ? 0.235 : 0.15},
-                           {8, 4, 256, 5.9, g ? 0.109 : 0.0704, g ? 0.109 : 0.0704},
-                           {4, 4, 512, 4.8, g ? 0.168 : 0.0780, g ? 0.07 : 0.05}};
+    static const Form kPoint[5] = {{16, 2, 7.2, 5.7, 0.088, 0.167},
+                                   {8, 1, 7.8, 5.4, 0.080, 0.173},
+                                   {8, 2, 6.2, 2.4, 0.070, 0.092},
+                                   {8, 4, 3.8, 6.1, 0.008, 0.077},
+                                   {4, 4, 5.6, 2.4, 0.024, 0.044}};
+    static const Form kGaussian[5] = {{16, 2, 7.8, 6.7, 0.120, 0.272},
+                                      {8, 1, 8.2, 6.5, 0.106, 0.308},
+                                      {8, 2, 5.3, 3.3, 0.078, 0.167},
+                                      {8, 4, 3.8, 6.8, 0.008, 0.119},
+                                      {4, 4, 4.2, 4.5, 0.005, 0.0936}};
     const size_t n = (size_t)a.nchan * a.ntiles * (a.ntiles - 1) * 2;  // entries of a slice's sums
     const int most = may_slice ? (int)std::min<size_t>(16, a.part_limit / (sizeof(double2) * std::max<size_t>(n, 1))) : 1;
     TilesChoice best{-1, 1, 0.0};
     for (int i = 0; i < 5; ++i) {
         if (i == 0 && !a.even16) continue;
-        const Form &f = forms[i];
+        const Form &f = g ? kGaussian[i] : kPoint[i];
         for (int s = 1; s == 1 || (i < 3 && s <= most && s <= a.ncomp / 128); ++s) {
-            const double blocks = (double)a.npairs * f.sub * chunk_count(a.chunks, f.nch, a.nchan) * s;
-            const double r = blocks / f.resident, m = f.resident / 256, k = fmin(ceil(blocks / 256), m);
-            const double per_comp = r > 1.0 ? f.full * 0.5 * (r + ceil(r))
-                                            : f.single + (m > 1.0 ? (f.full - f.single) * (k - 1.0) / (m - 1.0) : 0.0);
-            double t = fmax(r, 1.0) * f.fixed + (double)a.ncomp / s * per_comp;
-            if (s > 1) t += 5.0 + n * s * 32.0 / 4e6;
+            const int len = s > 1 ? slice_length(a.ncomp, s) : a.ncomp;
+            if ((a.ncomp + len - 1) / len != s) continue;  // the last slices would be empty
+            const double k = ceil((double)a.npairs * f.sub * chunk_count(a.chunks, f.nch, a.nchan) * s / 256.0);
+            double t = f.start + f.start_block * k + len * (f.comp + f.comp_block * k);
+            const double bytes = (double)sizeof(double2) * n * s;
+            if (s > 1) t += 5.0 + 2.0 * bytes / (bytes <= 2e8 ? 12e6 : 4e6);
             if (best.form < 0 || t < best.us) best = TilesChoice{i, s, t};
         }
     }
@@ -722,7 +731,7 @@ static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t 
     }
     a.slices = best.slices;
     if (a.slices > 1) a.part = part->as<double2>();
-    a.slice_len = ((a.ncomp + a.slices - 1) / a.slices + kCT - 1) / kCT * kCT;
+    a.slice_len = slice_length(a.ncomp, a.slices);
     switch (best.form) {
     case 0: return launch_tiles_form<KIND, 16, 2, 4, 1, NARROW>(a, stream);
     case 1: return launch_tiles_form<KIND, 8, 4, 4, 1, NARROW>(a, stream);
