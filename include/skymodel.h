@@ -186,11 +186,12 @@ const char *sm_synchronize(void);
 const char *sm_set_direct_variant(int32_t variant);
 
 /* Which form of the FP64 tile-pair kernel, and how many slices of the components, a timestep of a
- * modeller takes for its points or Gaussians where num_tiles tiles share a beam: 0 = 16 channels wide,
- * 1 = 8 channels and 16 rows of tiles a block, 2 = 8 channels and 8 rows, 3 and 4 = 8 and 4 channels
- * with the components over eight waves. Sizes only, no device; used to test every form. No
- * counterpart in the reference. */
-const char *sm_tiles_form(int32_t gaussian, int32_t num_tiles, int32_t num_freqs, const double *freqs,
+ * modeller takes where num_tiles tiles share a beam, for its points (kind 0), its Gaussians (1) or its
+ * Gaussians on the split-precision path with FP32 visibilities alone (2): 0 = 16 channels wide, 1 = 8
+ * channels and 16 rows of tiles a block, 2 = 8 channels and 8 rows, 3 and 4 = 8 and 4 channels with the
+ * components over eight waves, -1 = the FP32 kernel. Sizes only, no device; used to test every form.
+ * No counterpart in the reference. */
+const char *sm_tiles_form(int32_t kind, int32_t num_tiles, int32_t num_freqs, const double *freqs,
                           int32_t num_comps, int32_t *form, int32_t *slices);
 
 /* Limit in bytes on the per-beam-row-class coherency tables the per-tile-beam paths build

@@ -149,12 +149,10 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const bool hermitian = shared_tiled || shared_shapelet;
     // FP32 arithmetic (the precision path). Where that path's caller takes FP32 visibilities alone, an FP64
     // kernel stands in wherever it is the faster one (us a timestep, FP32 and FP64):
-    // - tile-pair Gaussians of at most 400 FP32 blocks, which leave CUs idle or with one block where
-    //   the FP64 kernel takes slices of the components: 64 blocks (64 tiles, 48 channels, 1000
-    //   components) 635 and 248, 256 blocks (128, 48, 2000) 1244 and 832, 400 (101, 93, 700) 587
-    //   and 552, but 512 (128, 96, 2000) 1308 and 1450, 2048 (256, 96, 2000) 3594 and 4146;
-    // - row-by-column Gaussians of at most one round of FP32 blocks (three a CU): 128 tiles, 12 of them
-    //   with their own beams, 96 channels, 2000 components (96 blocks) 3324 and 2227; 256 tiles, 26 such,
+    // - tile-pair Gaussians by the estimates of both kernels (fp64_gaussians_faster);
+    // - row-by-column Gaussians of fewer than 700 FP32 blocks: 128 tiles, 12 of them with their own beams,
+    //   96 channels, 2000 components (96 blocks) 3324 and 2227; 1000 components of every kind of pair, 192
+    //   blocks 2137 and 1942, 384 3166 and 3083, 448 to 672 within 1%, 768 5415 and 5572; 256 tiles, 26 such,
     //   10000 components, the kernel alone: 96 channels (448 blocks) 8820 and 7540, 384 (1792) 25750 and 29400;
     // - shared-beam shapelets, unless few channels fall in one table cell: 200 components, 128 tiles,
     //   96 channels of 10 kHz 1664 and 969; 100 components, 256 tiles within 3 km, 93 of 80 kHz 4529 and 4401;
@@ -164,9 +162,19 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const bool either = fp32_path && vis64 == nullptr;
     const int last128 = ctx.nchan % 128;
     const bool few_per_cell = ctx.step > 80e3 && (last128 == 0 || last128 > 64);
-    auto small_grid = [&](int npairs) { return (long)npairs * chunk_count(ctx.chunks, 6, ctx.nchan) <= 400; };
+    auto fp64_pairs = [&](int ntiles, int npairs) {
+        TiledArgs t{};
+        t.ntiles = ntiles;
+        t.npairs = npairs;
+        t.nchan = ctx.nchan;
+        t.ncomp = n;
+        t.chunks = ctx.chunks;
+        t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
+        t.part_limit = ctx.part_limit;
+        return fp64_gaussians_faster(t);
+    };
     const bool f32 =
-        fp32_path && !(either && ((shared_shapelet && !few_per_cell) || (shared_tiled && small_grid(ctx.npairs))));
+        fp32_path && !(either && ((shared_shapelet && !few_per_cell) || (shared_tiled && fp64_pairs(ctx.ntiles, ctx.npairs))));
     const bool planes = shared_shapelet && !(f32 && ctx.d_sbf32 != nullptr);
     e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, ctx.beam, !per_tile, coh.as<double>(),
                          stream, planes ? COH_HERMITIAN_PLANES : (hermitian ? COH_HERMITIAN : COH_FULL));
@@ -236,7 +244,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         b0.uniform_row = ctx.class_row0;
         e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, b0, true, coh0.as<double>(), stream,
                              COH_HERMITIAN);
-        const bool pairs32 = f32 && !(either && small_grid(ctx.g0_npairs));
+        const bool pairs32 = f32 && !(either && fp64_pairs(ctx.g0_n, ctx.g0_npairs));
         if (e == hipSuccess && pairs32) e = to_f32(scratch.coh0_32, coh_n / 2, coh0.as<double>(), stream);
         if (e != hipSuccess) return e;
         TiledArgs t;
@@ -272,7 +280,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         const int nseg = 2 * (ctx.nclass - 1);
         const size_t ccls_bytes = (size_t)ctx.nclass * n * ctx.nchan_pad * 8 * sizeof(double);
         const bool rect32 = f32 && !(either && (long)((ctx.n_other + 3) / 4) * ((ctx.g0_n + 63) / 64) *
-                                                       chunk_count(ctx.chunks, 6, ctx.nchan) <= 768);
+                                                       chunk_count(ctx.chunks, 6, ctx.nchan) < 700);
         const bool rect = e == hipSuccess && ctx.n_other > 0 && ctx.d_other_tiles != nullptr && ctx.nclass > 1 &&
                           reserve_class_table(ccls, ccls_bytes);
         if (rect) {
@@ -884,9 +892,10 @@ extern "C" const char *sm_set_class_table_limit(int64_t bytes) {
     return nullptr;
 }
 
-extern "C" const char *sm_tiles_form(int32_t gaussian, int32_t num_tiles, int32_t num_freqs, const double *freqs,
+extern "C" const char *sm_tiles_form(int32_t kind, int32_t num_tiles, int32_t num_freqs, const double *freqs,
                                      int32_t num_comps, int32_t *form, int32_t *slices) {
     if (freqs == nullptr || form == nullptr || slices == nullptr) return "null argument";
+    if (kind < 0 || kind > 2) return "kind must be 0, 1 or 2";
     if (num_tiles < 2 || num_freqs < 1 || num_comps < 1) return "no pairs of tiles, channels or components";
     const std::vector<int2> c4 = even_chunks(freqs, num_freqs, 4), c6 = even_chunks(freqs, num_freqs, 6),
                             c8 = even_chunks(freqs, num_freqs, 8), c16 = even_chunks(freqs, num_freqs, 16);
@@ -897,9 +906,10 @@ extern "C" const char *sm_tiles_form(int32_t gaussian, int32_t num_tiles, int32_
     a.nchan = num_freqs;
     a.ncomp = num_comps;
     a.even16 = true;
-    const TilesChoice t = choose_tiles_form(gaussian != 0, a, true);
-    *form = t.form;
-    *slices = t.slices;
+    const TilesChoice t = choose_tiles_form(kind != 0, a, true);
+    const bool fp32 = kind == 2 && !fp64_gaussians_faster(a);
+    *form = fp32 ? -1 : t.form;
+    *slices = fp32 ? 1 : t.slices;
     return nullptr;
 }
 

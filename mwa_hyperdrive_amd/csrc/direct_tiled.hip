@@ -718,6 +718,18 @@ TilesChoice choose_tiles_form(bool g, const TiledArgs &a, bool may_slice) {
     return best;
 }
 
+// The FP32 kernel's blocks are three to a CU and take n components in n (0.53, 0.55, 0.64) us for one, two
+// and three of them, 0.09 less behind a full round (32 to 256 tiles, 256 to 2048 blocks); the estimates of
+// both kernels are within 7%, so that 8% decide. us a timestep, FP32 and FP64: 128 tiles, 72 channels, 200 Gaussians 183 and 201, 1000
+// 619 and 578; 96 channels, 1000 628 and 639, 5000 2752 and 2530; 256 tiles, 36 channels, 5000 3245 and
+// 4400.
+bool fp64_gaussians_faster(const TiledArgs &a) {
+    const int k = (a.npairs * chunk_count(a.chunks, kTiledNchGaussian, a.nchan) + 255) / 256;
+    const double rest = k % 3 == 0 ? 0.0 : (k % 3 == 1 ? 0.53 : 0.55) - (k > 3 ? 0.09 : 0.0);
+    const double us32 = 15.0 + a.ncomp * (0.64 * (k / 3) + rest);
+    return choose_tiles_form(true, a, true).us < 0.92 * us32;
+}
+
 template <int KIND, bool NARROW>
 static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t stream) {
     constexpr bool g = KIND == KIND_GAUSSIAN;

@@ -132,6 +132,8 @@ struct TilesChoice {
     double us;
 };
 TilesChoice choose_tiles_form(bool gaussian, const TiledArgs &a, bool may_slice);
+// Whether a's Gaussians take less time on the FP64 tile-pair kernel than on the FP32 one. Host only.
+bool fp64_gaussians_faster(const TiledArgs &a);
 // part (nullable) backs slices of the components, which few blocks of many components take.
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a, DevBuf *part, hipStream_t stream);
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream);

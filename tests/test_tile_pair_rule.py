@@ -1,5 +1,6 @@
-"""The rule that picks the FP64 tile-pair kernel's form, against measured kernel times (us, 40 kHz
-channels, MI355X): what it picks is within 10% of the fastest of the forms measured."""
+"""The rules that pick the FP64 tile-pair kernel's form, and on the precision path the FP32 or the FP64
+kernel, against measured times (us, 40 kHz channels, MI355X): what they pick is within 10% of the
+fastest measured."""
 
 import pytest
 
@@ -50,3 +51,21 @@ def check(gaussian, size, measured):
     below, above = max(s for s in times if s <= slices), min((s for s in times if s >= slices), default=None)
     assert above is not None, f"{slices} slices of form {form}: more than the most measured"
     assert max(times[below], times[above]) <= 1.1 * min(t for v in measured.values() for t in v.values())
+
+
+# (tiles, channels, components): timesteps of Gaussians alone on the FP32 and on the FP64 kernel.
+PRECISION = {
+    (64, 192, 200): (159.0, 148.1), (64, 192, 5000): (2713.2, 1426.1), (64, 384, 200): (185.3, 211.9),
+    (101, 96, 200): (170.2, 195.3), (101, 96, 5000): (2661.9, 2072.8), (128, 48, 1000): (564.5, 368.7),
+    (128, 72, 200): (183.0, 206.9), (128, 72, 1000): (619.0, 555.0), (128, 132, 200): (218.6, 291.6),
+    (128, 132, 5000): (3193.1, 3668.5), (200, 48, 1000): (699.7, 804.7), (256, 18, 200): (197.2, 222.0),
+    (256, 18, 1000): (627.6, 719.7), (256, 36, 1000): (774.5, 1090.3), (256, 36, 5000): (3244.7, 4540.8),
+    (32, 768, 1000): (604.6, 375.4),
+}
+
+
+@pytest.mark.parametrize("size", PRECISION)
+def test_precision_path_gaussians(size):
+    nt, nchan, ncomp = size
+    fp32 = form_of(2, nt, band(nchan, 40e3), ncomp)[0] < 0
+    assert PRECISION[size][0 if fp32 else 1] <= 1.1 * min(PRECISION[size])
