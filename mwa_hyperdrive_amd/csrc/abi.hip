@@ -154,14 +154,14 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     //   96 channels, 2000 components (96 blocks) 3324 and 2227; 1000 components of every kind of pair, 192
     //   blocks 2137 and 1942, 384 3166 and 3083, 448 to 672 within 1%, 768 5415 and 5572; 256 tiles, 26 such,
     //   10000 components, the kernel alone: 96 channels (448 blocks) 8820 and 7540, 384 (1792) 25750 and 29400;
-    // - shared-beam shapelets, unless few channels fall in one table cell: 200 components, 128 tiles,
-    //   96 channels of 10 kHz 1664 and 969; 100 components, 256 tiles within 3 km, 93 of 80 kHz 4529 and 4401;
-    //   128 tiles within 3 km, 96 of 160 kHz 3130 and 3691 (256 tiles, 48 of 160 kHz, which fill less
-    //   than half of an FP32 wave's 128 channels: 4423 and 3913).
+    // - shared-beam shapelets, unless a group of 64 channels crosses more than 20 table edges and there are
+    //   several: 200 components, 128 tiles within 3 km, 192 channels of 160 kHz (28 edges) 6280 and 6370, 64
+    //   tiles 1760 and 2180, but 64 channels 2690 and 2540, 384 of 80 kHz (14 edges) 7310 and 7200; within
+    //   1.5 km 96 of 160 kHz (14 edges) 2470 and 2350, 24 of 1.28 MHz 3460 and 1740.
     const bool fp32_path = ctx.fp32 && kind != KIND_POINT && ctx.d_bl_subset == nullptr && g_direct_variant == 0;
     const bool either = fp32_path && vis64 == nullptr;
-    const int last128 = ctx.nchan % 128;
-    const bool few_per_cell = ctx.step > 80e3 && (last128 == 0 || last128 > 64);
+    const double edges_per_hz = ctx.edges_per_hz > 0.0 ? ctx.edges_per_hz : kTypicalEdgesPerHz;
+    const bool many_edges = ctx.nchan > 64 && edges_per_hz * ctx.step * 64 > 20.0;
     auto fp64_pairs = [&](int ntiles, int npairs) {
         TiledArgs t{};
         t.ntiles = ntiles;
@@ -174,7 +174,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         return fp64_gaussians_faster(t);
     };
     const bool f32 =
-        fp32_path && !(either && ((shared_shapelet && !few_per_cell) || (shared_tiled && fp64_pairs(ctx.ntiles, ctx.npairs))));
+        fp32_path && !(either && ((shared_shapelet && !many_edges) || (shared_tiled && fp64_pairs(ctx.ntiles, ctx.npairs))));
     const bool planes = shared_shapelet && !(f32 && ctx.d_sbf32 != nullptr);
     e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, ctx.beam, !per_tile, coh.as<double>(),
                          stream, planes ? COH_HERMITIAN_PLANES : (hermitian ? COH_HERMITIAN : COH_FULL));
@@ -402,6 +402,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         s.ncomp = n;
         s.ngroups = (ctx.nchan + 63) / 64;
         s.step = ctx.step;
+        s.edges_per_hz = edges_per_hz;
         s.freqs = ctx.d_freqs_pad;
         s.uvw = ctx.d_uvw;
         s.lmn = in.lmn;
@@ -778,6 +779,14 @@ extern "C" const char *sm_model_shapelets_f64(const Shapelets *s, const Addresse
     in.coeff_range = st.coeff_range.as<int2>();
     in.coeffs = st.coeffs.as<ShapeletCoeff>();
     in.coeff_count = (int)off;
+    // Per-tile beams: which kernel depends on the table edges crossed, asked of the device where the band
+    // may cross several and the kernel is long enough (50 us, against 15 us for the answer).
+    if (d_beam_jones != nullptr && ctx.beam.uniform_row < 0 && ctx.step * ctx.nchan > 1e6 &&
+        (double)n * ctx.nbl * ((ctx.nchan + 63) / 64) > 5e4) {
+        SM_TRY(st.accum.reserve(sizeof(double)));
+        SM_TRY(launch_shapelet_edges(n, ctx.nbl, in.shape, in.bl_uv, st.accum.as<double>(), 0));
+        SM_TRY(hipMemcpy(&ctx.edges_per_hz, st.accum.ptr, sizeof(double), hipMemcpyDeviceToHost));
+    }
     SM_TRY(run_type(KIND_SHAPELET, in, ctx, st.coh, st.scratch, d_vis_fb, d_vis_fb_f64, 0, nullptr, nullptr));
     SM_TRY(hipStreamSynchronize(0));
     return nullptr;
@@ -910,6 +919,14 @@ extern "C" const char *sm_tiles_form(int32_t kind, int32_t num_tiles, int32_t nu
     const bool fp32 = kind == 2 && !fp64_gaussians_faster(a);
     *form = fp32 ? -1 : t.form;
     *slices = fp32 ? 1 : t.slices;
+    return nullptr;
+}
+
+extern "C" const char *sm_shapelet_form(int32_t per_tile, int32_t num_freqs, double step, double edges_per_hz,
+                                        int32_t *form) {
+    if (form == nullptr) return "null argument";
+    if (num_freqs < 1) return "no channels";
+    *form = choose_shapelet_form(per_tile != 0, num_freqs, step, edges_per_hz);
     return nullptr;
 }
 

@@ -2432,25 +2432,70 @@ static hipError_t launch_shapelets_form(const ShapeletChanArgs &a, hipStream_t s
     return hipGetLastError();
 }
 
-// The forms by channel count and step: fewer, wider groups share the phasors' start and the
-// component's values among more channels; narrow ones hold fewer segments, the cost that grows
-// with the step. Measured with 128 tiles within 1.5 km and 200 components (ms, FP64; FP32 within
-// 3%), as <slots, baselines per wave>:
-//   channels x step     <1,2>  <2,2>  <1,1>   one wave per baseline, adjacent channels
-//   32 x 40 kHz          0.59   0.73   0.73   2.19
-//   96 x 20 kHz          1.22   1.11   1.28   2.29
-//   384 x 20 kHz         4.05   2.81   3.30   5.85
-//   384 x 80 kHz         5.36   4.82   4.82   7.30
-//   384 x 160 kHz        7.73   8.27   7.33   10.06
-// The weights are straight lines through these and nine more points, per group, in ms.
-template <bool PT> static hipError_t launch_shapelets(const ShapeletChanArgs &a, hipStream_t stream) {
-    const double khz = 1e-3 * a.step;
-    const double w32 = ((a.nchan + 31) / 32) * (0.275 + 0.0021 * khz);
-    const int g64 = (a.nchan + 63) / 64;
-    const double w64 = g64 * (0.30 + 0.0064 * khz), w64one = g64 * (0.42 + 0.0047 * khz);
-    if (w64 < w32 && w64 < w64one) return launch_shapelets_form<2, 2, 3, PT>(a, stream);
-    if (w64one < w32) return launch_shapelets_form<1, 1, 4, PT>(a, stream);
-    return launch_shapelets_form<1, 2, 4, PT>(a, stream);
+// The forms: fewer, wider groups share the phasors' start and the component's values among more
+// channels; narrow ones hold fewer segments, the cost that grows with the table edges that a component
+// crosses over a group's channels. Per-tile beams have a fourth, k_shapelet_chan_tiles, whose sums per
+// channel cost the same wherever the edges lie. Each takes a time per group that is linear in those edges
+// up to where most components leave the segments for the direct sums; the lines are fits, within 12%, to
+// 200 components of 0.5 to 5 arcmin, 128 tiles within 0.5, 1.5 and 3 km, and 4 to 384 channels of 20 kHz
+// to 1.28 MHz. The form taken is within 5% of the fastest at 77 of these 78 sizes (10% at the other). ms,
+// forms 0 to 3, per-tile beams:
+//   384 x 80 kHz, 500 m   4.6 4.9 5.5 7.7     24 x 80 kHz, 1500 m      0.93 0.79 0.62 1.36
+//   384 x 80 kHz, 1500 m  6.6 6.3 6.7 7.8     12 x 1.28 MHz, 500 m     1.29 1.00 0.94 1.35
+//   384 x 80 kHz, 3000 m  10.5 9.3 9.4 7.9    12 x 1.28 MHz, 1500 m    3.11 2.20 1.68 1.48
+int choose_shapelet_form(bool per_tile, int nchan, double step, double edges_per_hz) {
+    struct Line {
+        int span;  // channels of a group
+        double at0, edge, most;
+    };
+    static const Line kShared[3] = {{64, 0.29, 0.092, 45.0}, {64, 0.37, 0.071, 36.0}, {32, 0.25, 0.069, 20.0}};
+    static const Line kOwn[4] = {{64, 0.56, 0.099, 45.0}, {64, 0.62, 0.075, 37.0}, {32, 0.395, 0.069, 21.0},
+                                 {64, 1.29, 0.0132, 60.0}};
+    int best = 0;
+    double t_best = 0.0;
+    for (int i = 0; i < (per_tile ? 4 : 3); ++i) {
+        const Line &f = per_tile ? kOwn[i] : kShared[i];
+        const double edges = edges_per_hz * step * std::min(nchan, f.span);
+        const double t = ((nchan + f.span - 1) / f.span) * (f.at0 + f.edge * fmin(edges, f.most));
+        if (i == 0 || t < t_best) {
+            best = i;
+            t_best = t;
+        }
+    }
+    return best;
+}
+
+template <bool PT> static hipError_t launch_shapelets(int form, const ShapeletChanArgs &a, hipStream_t stream) {
+    switch (form) {
+    case 0: return launch_shapelets_form<2, 2, 3, PT>(a, stream);
+    case 1: return launch_shapelets_form<1, 1, 4, PT>(a, stream);
+    default: return launch_shapelets_form<1, 2, 4, PT>(a, stream);
+    }
+}
+
+// Mean table edges per Hz that a shapelet crosses, over up to 4096 of the (component, baseline) pairs.
+__global__ __launch_bounds__(256) void k_shapelet_edges(size_t n, int nbl, const double4 *__restrict__ shape,
+                                                        const double2 *__restrict__ bl_uv, double *out) {
+    __shared__ double part[4];
+    const size_t samples = n < 4096 ? n : 4096;
+    double sum = 0.0;
+    for (size_t i = threadIdx.x; i < samples; i += 256) {
+        const size_t at = i * n / samples;
+        const double4 sh = shape[at / nbl];
+        const double2 uv = bl_uv[at];
+        sum += fabs((uv.x * sh.x + uv.y * sh.y) * sh.z) + fabs((uv.x * sh.y - uv.y * sh.x) * sh.w);
+    }
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) *out = (part[0] + part[1] + part[2] + part[3]) / samples;
+}
+
+hipError_t launch_shapelet_edges(int ncomp, int nbl, const double4 *d_shape, const double2 *d_bl_uv, double *d_out,
+                                 hipStream_t stream) {
+    if (ncomp <= 0 || nbl <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_shapelet_edges, dim3(1), dim3(256), 0, stream, (size_t)ncomp * nbl, nbl, d_shape, d_bl_uv, d_out);
+    return hipGetLastError();
 }
 
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream) {
@@ -2458,12 +2503,8 @@ hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStr
     const bool f32 = a.coh32 != nullptr;
     if (f32 && (a.sbf32 == nullptr || (per_tile && a.beam.coh_cls != nullptr && a.coh_cls32 == nullptr)))
         return hipErrorInvalidValue;
-    // Per-tile beams in FP64: runs of a table cell hold few channels of a wide step on long baselines, where
-    // the sums per channel are cheaper if the channels fill their 64 lanes. 500 components, 256 tiles
-    // within 3 km, 80 kHz: 384 channels 80 ms per channel and 91 ms per run, 96 channels (a group and a
-    // half) 26.7 and 24.4 ms.
-    const bool per_channel = per_tile && a.step >= 80e3 && (a.nchan % 64 == 0 || a.nchan % 64 > 32);
-    if (!f32 && !per_channel) return per_tile ? launch_shapelets<true>(a, stream) : launch_shapelets<false>(a, stream);
+    const int form = choose_shapelet_form(per_tile, a.nchan, a.step, a.edges_per_hz);
+    if (!f32 && form < 3) return per_tile ? launch_shapelets<true>(form, a, stream) : launch_shapelets<false>(form, a, stream);
     // Per-tile beams: a.ngroups groups of 64 channels; FP32 shared beam: groups of 128 channels.
     const int total = ((a.nbl + 3) / 4) * (per_tile ? a.ngroups : (a.nchan + 127) / 128);
     hipLaunchKernelGGL(!per_tile ? k_shapelet_chan32 : (f32 ? k_shapelet_chan_tiles32 : k_shapelet_chan_tiles),

@@ -198,6 +198,8 @@ struct SmModeller {
     std::vector<int> freq_map;
     std::vector<double> ufreqs;
     bool even = false, narrow = false;
+    double rms_baseline = 0.0;  // [m]
+    double edges_per_hz = 0.0;  // ModelCtx::edges_per_hz of the shapelets set
     // device
     DevBuf d_freqs, d_xyz, d_bl_tiles, d_bl_rows, d_tile_rows, d_freq_map, d_ufreqs, d_delays, d_gains, d_sbf;
     DevBuf d_udelays, d_ugains;  // the unique tiles' delays [n_utile][16] and gains [n_utile][32]
@@ -348,6 +350,11 @@ const char *set_components(SmModeller *m, const SmComponent *const *comps, int n
             for (int f = 0; f < m->nchan; ++f)
                 for (int i = 0; i < h.n_list; ++i)
                     h.list_fds[(size_t)f * h.n_list + i] = inst_stokes(estimate_at_freq(*lists[i], m->freqs[f]));
+        }
+        if (ty == SM_SHAPELET) {
+            double axes = 0.0;  // mean of |x| + |y| cells per metre and Hz; 2/pi: a baseline's mean projection
+            for (const double4 &sh : h.shape) axes += (std::fabs(sh.z) + std::fabs(sh.w)) / (double)h.shape.size();
+            m->edges_per_hz = 0.6366 * m->rms_baseline * axes;
         }
         DevType &d = m->types[ty];
         SM_TRY(upload(d.lmn, h.lmn));
@@ -528,6 +535,12 @@ extern "C" const char *sm_new(const SmObsParams *p, const SmComponent *comps, co
             bl_tiles[b] = make_int2(i, j);
             bl_rows[b] = make_int2(m->tile_rows[i], m->tile_rows[j]);
         }
+    double mean[3] = {0.0, 0.0, 0.0}, sq = 0.0;
+    for (int i = 0; i < 3 * m->nt; ++i) {
+        mean[i % 3] += m->xyz[i] / m->nt;
+        sq += m->xyz[i] * m->xyz[i] / m->nt;
+    }
+    m->rms_baseline = std::sqrt(std::max(0.0, 2.0 * (sq - mean[0] * mean[0] - mean[1] * mean[1] - mean[2] * mean[2])));
     auto fail = [m](const char *e) {
         sm_free(m);
         return e;
@@ -792,6 +805,7 @@ static const char *model_timestep_device(SmModeller *m, double lst, double latit
     ctx.even = true;
     ctx.narrow = m->narrow;
     ctx.step = mean_step(m->freqs_pad.data(), m->nchan);
+    ctx.edges_per_hz = m->edges_per_hz;
     ctx.d_uvw = uvw;
     ctx.d_sbf = m->d_sbf.as<double>();
     ctx.d_tile_uvw = tile_uvw;

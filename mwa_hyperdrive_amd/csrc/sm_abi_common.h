@@ -32,6 +32,7 @@ struct ModelCtx {
     bool even16 = false; // fixed chunks of 16 channels are evenly spaced (chunk tables need no such test)
     bool narrow = false; // every channel step at most a thousandth of its frequency (narrow_steps)
     double step = 0.0;   // mean channel spacing [Hz]
+    double edges_per_hz = 0.0;  // ShapeletChanArgs::edges_per_hz, or 0 (unknown)
     const UVW *d_uvw = nullptr;
     const double *d_sbf = nullptr;
     BeamDesc beam{};

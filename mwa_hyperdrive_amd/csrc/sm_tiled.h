@@ -44,10 +44,15 @@ struct TiledArgs {
     size_t part_limit = SIZE_MAX;  // bytes that part may take
 };
 
+// Basis-table edges (of both axes) that a shapelet crosses per Hz on a typical baseline: 5.5 arcmin for the
+// sum of its axes, tiles within 1.5 km.
+constexpr double kTypicalEdgesPerHz = 1.36e-6;
+
 struct ShapeletChanArgs {
     // ngroups: groups of 64 channels of the per-tile kernels (the shared-beam kernels form their own).
     int nbl, nchan, nchan_pad, ncomp, ngroups;
     double step = 0.0;  // mean channel spacing [Hz]
+    double edges_per_hz = kTypicalEdgesPerHz;
     const double *freqs;
     const UVW *uvw;           // [nbl]
     const double4 *lmn;
@@ -136,6 +141,12 @@ TilesChoice choose_tiles_form(bool gaussian, const TiledArgs &a, bool may_slice)
 bool fp64_gaussians_faster(const TiledArgs &a);
 // part (nullable) backs slices of the components, which few blocks of many components take.
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a, DevBuf *part, hipStream_t stream);
+// The form of the FP64 shapelet kernels (0 .. 2: k_shapelets with 2, 1 and 1 channels a lane for 2, 1 and
+// 2 baselines a wave; 3, per-tile beams alone: k_shapelet_chan_tiles). Host only.
+int choose_shapelet_form(bool per_tile, int nchan, double step, double edges_per_hz);
+// ShapeletChanArgs::edges_per_hz of the components' shapes and baseline UVs, to device memory.
+hipError_t launch_shapelet_edges(int ncomp, int nbl, const double4 *d_shape, const double2 *d_bl_uv, double *d_out,
+                                 hipStream_t stream);
 hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStream_t stream);
 hipError_t launch_tile_uvw_from_baselines(int ntiles, const UVW *d_uvw, double *d_out, hipStream_t stream);
 // FP64 -> FP32 copy of n values (coherency tables, basis table).
