@@ -106,8 +106,10 @@ static hipError_t to_f32(DevBuf &buf, size_t n, const double *src, hipStream_t s
 
 // Reserves a per-class coherency table of `bytes` in buf if it is within the limit and the
 // allocation succeeds; false sends the caller to its per-segment path. A failed allocation
-// is cleared from the runtime's last-error state, so it does not surface later.
-static bool reserve_class_table(DevBuf &buf, size_t bytes) {
+// is cleared from the runtime's last-error state, so it does not surface later. The slices' sums of
+// earlier launches (`spare`; freeing them waits for the kernels queued) give way to a table that would
+// not fit beside them.
+static bool reserve_class_table(DevBuf &buf, size_t bytes, DevBuf &spare) {
     if (g_class_table_limit >= 0 && bytes > (size_t)g_class_table_limit) return false;
     if (buf.ptr != nullptr && buf.bytes >= bytes) return true;
     size_t limit;
@@ -122,6 +124,10 @@ static bool reserve_class_table(DevBuf &buf, size_t bytes) {
         // What buf already holds is released before the larger allocation.
         free_b += buf.bytes;
         limit = free_b > (size_t(1) << 30) ? free_b - (size_t(1) << 30) : 0;
+        if (!spare.borrowed && bytes > limit && bytes <= limit + spare.bytes) {
+            limit += spare.bytes;
+            spare.release();
+        }
     }
     if (bytes > limit) return false;
     if (buf.reserve(bytes) != hipSuccess) {
@@ -170,7 +176,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.ncomp = n;
         t.chunks = ctx.chunks;
         t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
-        t.part_limit = ctx.part_limit;
+        t.part_limit = std::min(kSliceBytes, ctx.part_limit);
         return fp64_gaussians_faster(t);
     };
     const bool f32 =
@@ -188,7 +194,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     const size_t cls_bytes = (size_t)ctx.nclass * n * ctx.nchan_pad * 8 * sizeof(double);
     if (kind == KIND_SHAPELET && g_direct_variant != 1 && ctx.d_bl_subset == nullptr && per_tile &&
         ctx.nclass > 0 && ctx.d_class_row != nullptr && ctx.class_row0 >= 0 &&
-        reserve_class_table(scratch.cls, cls_bytes)) {
+        reserve_class_table(scratch.cls, cls_bytes, scratch.accum)) {
         e = launch_class_coherency(ctx.nclass, n, ctx.nchan, ctx.nchan_pad, coh.as<double>(), ctx.beam, ctx.d_class_row,
                                    scratch.cls.as<double>(), stream);
         if (e != hipSuccess) return e;
@@ -269,21 +275,21 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.chunks = ctx.chunks;
         t.narrow = ctx.narrow;
         t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
-        t.part_limit = ctx.part_limit;
-        if (ev0 != nullptr) (void)hipEventRecord(ev0, stream);
-        e = launch_direct_tiled(kind, t, &scratch.accum, stream);
+        t.part_limit = std::min(kSliceBytes, ctx.part_limit);
         // Pairs of a class-r tile with a class-0 tile. With a table of J_r S J_0^H for every
         // class (when it fits, g_class_table_limit): one launch of the row-by-column kernel.
         // Otherwise one shared coherency per segment and the shared-beam form of the
-        // baseline kernel.
+        // baseline kernel. The table is reserved before the tile-pair kernel's slices, which give way to it.
         DevBuf &cseg = scratch.cseg, &ccls = scratch.ccls;
         const int nseg = 2 * (ctx.nclass - 1);
         const size_t ccls_bytes = (size_t)ctx.nclass * n * ctx.nchan_pad * 8 * sizeof(double);
+        const bool rect = ctx.n_other > 0 && ctx.d_other_tiles != nullptr && ctx.nclass > 1 &&
+                          reserve_class_table(ccls, ccls_bytes, scratch.accum);
+        if (ev0 != nullptr) (void)hipEventRecord(ev0, stream);
+        e = launch_direct_tiled(kind, t, &scratch.accum, stream);
         const bool rect32 = f32 && !(either && (long)((ctx.n_other + 3) / 4) * ((ctx.g0_n + 63) / 64) *
                                                        chunk_count(ctx.chunks, 6, ctx.nchan) < 700);
-        const bool rect = e == hipSuccess && ctx.n_other > 0 && ctx.d_other_tiles != nullptr && ctx.nclass > 1 &&
-                          reserve_class_table(ccls, ccls_bytes);
-        if (rect) {
+        if (e == hipSuccess && rect) {
             e = launch_class_coherency(ctx.nclass, n, ctx.nchan, ctx.nchan_pad, coh.as<double>(), ctx.beam,
                                        ctx.d_class_row, ccls.as<double>(), stream);
             if (e == hipSuccess && rect32)
@@ -392,7 +398,7 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.chunks = ctx.chunks;
         t.narrow = ctx.narrow;
         t.even16 = ctx.chunks.c16 != nullptr || ctx.even16;
-        t.part_limit = ctx.part_limit;
+        t.part_limit = std::min(kSliceBytes, ctx.part_limit);
         e = launch_direct_tiled(kind, t, &scratch.accum, stream);
     } else if (g_direct_variant != 1 && kind == KIND_SHAPELET) {
         ShapeletChanArgs s;

@@ -1476,16 +1476,17 @@ static hipError_t launch_rect(const RectArgs &a, DevBuf *part, hipStream_t strea
     // Slices of at least 512 components: as many as fill whole rounds of the blocks that the 256 CUs hold
     // (two waves a SIMD), few for the traffic of their sums. No room for those: one.
     constexpr int kSlots = 2 * 256 * 4 / WR;
+    const size_t n = (size_t)a.nchan * a.n_row * a.n_col * 4;  // entries of a slice's sums
+    const int most = (int)std::min<size_t>(16, kSliceBytes / (sizeof(double2) * n));
     int slices = 1;
     double t_best = 0.0;
-    for (int s = 1; s == 1 || (s <= 16 && s <= a.ncomp / 512); ++s) {
+    for (int s = 1; s == 1 || (s <= most && s <= a.ncomp / 512); ++s) {
         const double t = (double)((per_slice * (long)s + kSlots - 1) / kSlots) / s + 0.02 * s * per_slice / kSlots;
         if (s == 1 || t < t_best) {
             slices = s;
             t_best = t;
         }
     }
-    const size_t n = (size_t)a.nchan * a.n_row * a.n_col * 4;
     if (slices > 1 && (part == nullptr || part->reserve(sizeof(double2) * n * slices) != hipSuccess)) {
         (void)hipGetLastError();
         slices = 1;

@@ -39,7 +39,7 @@ struct ModelCtx {
     const double *d_tile_uvw = nullptr;  // [ntiles][3], enables the tile-pair kernel
     const int4 *d_pairs = nullptr;
     int npairs = 0;
-    size_t part_limit = SIZE_MAX;  // TiledArgs::part_limit
+    size_t part_limit = SIZE_MAX;  // a further bound on TiledArgs::part_limit
     const int *d_bl_subset = nullptr;  // nullable: the direct kernels model only these baselines
     int nsub = 0;
     // Per-tile beams, optional: beam-row classes (class 0 = row class_row[0]); the per-tile

@@ -9,6 +9,11 @@
 
 namespace sm {
 
+// Bytes that the slices' sums of a launch may take: half of what the class tables leave free
+// (reserve_class_table), and beyond what any launch gains from. (An estimate is a few per cent off, and
+// without a bound 1000 tiles, 768 channels and 200000 components would take two slices of 24 GB for 1%.)
+constexpr size_t kSliceBytes = size_t(512) << 20;
+
 struct TiledArgs {
     int ntiles, nbl, nchan, nchan_pad, ncomp, npairs, nchunks;
     const int4 *pairs;        // [npairs] tile-group pairs (see tile_pairs)
@@ -41,7 +46,7 @@ struct TiledArgs {
     // [baseline of the kernel's tiles][4] when there are several.
     int slices = 1, slice_len = 0;
     double2 *part = nullptr;
-    size_t part_limit = SIZE_MAX;  // bytes that part may take
+    size_t part_limit = kSliceBytes;  // bytes that part may take
 };
 
 // Basis-table edges (of both axes) that a shapelet crosses per Hz on a typical baseline: 5.5 arcmin for the

@@ -53,6 +53,15 @@ def check(gaussian, size, measured):
     assert max(times[below], times[above]) <= 1.1 * min(t for v in measured.values() for t in v.values())
 
 
+@pytest.mark.parametrize("size", [(1000, 768, 200000), (1000, 192, 200000), (512, 48, 100000), (256, 192, 50000),
+                                  (256, 48, 10000), (128, 96, 10000)])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_slices_stay_within_their_workspace(kind, size):
+    nt, nchan, ncomp = size
+    _, slices = form_of(kind, nt, band(nchan, 40e3), ncomp)
+    assert slices == 1 or slices * nchan * nt * (nt - 1) // 2 * 64 <= 512 << 20
+
+
 # (tiles, channels, components): timesteps of Gaussians alone on the FP32 and on the FP64 kernel.
 PRECISION = {
     (64, 192, 200): (159.0, 148.1), (64, 192, 5000): (2713.2, 1426.1), (64, 384, 200): (185.3, 211.9),
