@@ -106,10 +106,11 @@ template <class T> __device__ __forceinline__ const T *pick(const double *d, con
 template <> __device__ __forceinline__ const double *pick<double>(const double *d, const float *) { return d; }
 template <> __device__ __forceinline__ const float *pick<float>(const double *, const float *f) { return f; }
 
-template <int KIND, int NCH, class T>
+// The precision path's tile-pair Gaussians: FP32, phases and exponents in FP64.
 __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
-    using V4 = typename Vec4<T>::type;
-    __shared__ V4 s_ph[kCT][32];
+    using T = float;
+    constexpr int NCH = kTiledNchGaussian;
+    __shared__ float4 s_ph[kCT][32];
     __shared__ double s_uvw[32][3];
     const int total = a.npairs * a.nchunks;
     int b = blockIdx.x;
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
     const double DF = freqs[f0 + 1] - F0;
     const double f0c = F0 / SM_VEL_C;
     const double dfc = DF / SM_VEL_C;
-    const T *__restrict__ coh = pick<T>(a.coh, a.coh32);
+    const T *__restrict__ coh = a.coh32;
     const double4 *__restrict__ lmn4 = a.lmn;
     const double4 *__restrict__ shape = a.shape;
 
@@ -185,35 +186,23 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
                 table_sincos(th * f0c, kSinCos32, ps, pc);
                 table_sincos(th * dfc, kSinCos32, qs, qc);
             }
-            V4 ph;
-            ph.x = (T)pc;
-            ph.y = (T)ps;
-            ph.z = (T)qc;
-            ph.w = (T)qs;
-            s_ph[cc][slot] = ph;
+            s_ph[cc][slot] = make_float4((float)pc, (float)ps, (float)qc, (float)qs);
         }
         __syncthreads();
-        // Component cc + 1's tile phasors, coherencies and Gaussian shape are loaded while
-        // component cc's products run. The explicit wait comes first: a scalar load's result
-        // can only be waited for with every outstanding scalar and LDS load, so the next
-        // component's loads are issued after it and are not waited for until the next
-        // iteration.
         for (int cc = 0; cc < nc; ++cc) {
             const int c = c0 + cc;
-            const V4 A = s_ph[cc][sp];
-            const V4 B = s_ph[cc][sq];
+            const float4 A = s_ph[cc][sp];
+            const float4 B = s_ph[cc][sq];
             T zr = A.x * B.x + A.y * B.y;
             T zi = A.y * B.x - A.x * B.y;
             const T rr = A.z * B.z + A.w * B.w;
             const T ri = A.w * B.z - A.z * B.w;
-            T env = T(1), er = T(1), eg = T(1);
-            if (KIND == KIND_GAUSSIAN) {
-                const double4 g = shape[c];
-                const double qf = g.x * (bu * bu) + g.y * (bu * bv) + g.z * (bv * bv);
-                exp_of(qf * (F0 * F0), env);
-                exp_of(qf * (DF * (2.0 * F0 + DF)), er);
-                exp_of(qf * (2.0 * DF * DF), eg);
-            }
+            T env, er, eg;
+            const double4 g = shape[c];
+            const double qf = g.x * (bu * bu) + g.y * (bu * bv) + g.z * (bv * bv);
+            exp_of(qf * (F0 * F0), env);
+            exp_of(qf * (DF * (2.0 * F0 + DF)), er);
+            exp_of(qf * (2.0 * DF * DF), eg);
             // The table is the Hermitian form (Re XX, Re XY, Im XY, Re YY) of J S J^H (see
             // TiledArgs), 32 contiguous bytes per channel. Per visibility: V_XX = sum C_XX z,
             // A = sum Re(C_XY) z, B = sum Im(C_XY) z, V_YY = sum C_YY z (8 FMAs per component
@@ -221,11 +210,7 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
             const T *cc4 = coh + ((size_t)c * a.nchan_pad + f0) * 4;
 #pragma unroll
             for (int k = 0; k < NCH; ++k) {
-                T pr_ = zr, pi_ = zi;
-                if (KIND == KIND_GAUSSIAN) {
-                    pr_ *= env;
-                    pi_ *= env;
-                }
+                const T pr_ = zr * env, pi_ = zi * env;
                 const T cxx = cc4[k * 4], cxyr = cc4[k * 4 + 1], cxyi = cc4[k * 4 + 2], cyy = cc4[k * 4 + 3];
                 acc[k][0] = fma_t(cxx, pr_, acc[k][0]);
                 acc[k][1] = fma_t(cxx, pi_, acc[k][1]);
@@ -238,10 +223,8 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
                 const T nr = zr * rr - zi * ri;
                 zi = zr * ri + zi * rr;
                 zr = nr;
-                if (KIND == KIND_GAUSSIAN) {
-                    env *= er;
-                    er *= eg;
-                }
+                env *= er;
+                er *= eg;
             }
         }
         flush_stage(acc, tot);
@@ -759,8 +742,7 @@ hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a_in, DevBuf *part, h
     if (a.coh32 != nullptr) {
         if (kind != KIND_GAUSSIAN) return hipErrorInvalidValue;  // FP32 points take the MFMA point path
         a.nchunks = chunk_count(a.chunks, kTiledNchGaussian, a.nchan);
-        hipLaunchKernelGGL((k_direct_tiled<KIND_GAUSSIAN, kTiledNchGaussian, float>), dim3(a.npairs * a.nchunks),
-                           dim3(256), 0, stream, a);
+        hipLaunchKernelGGL(k_direct_tiled, dim3(a.npairs * a.nchunks), dim3(256), 0, stream, a);
         return hipGetLastError();
     }
     return kind == KIND_GAUSSIAN ? (a.narrow ? launch_tiles<KIND_GAUSSIAN, true>(a, part, stream)
@@ -1313,11 +1295,10 @@ constexpr int kRT = 4 + 64;  // tile slots per block: 4 rows, then 64 columns
 // Channels per lane. 256 tiles, 384 channels: Gaussians 28.3 ms with 4, 26.8 ms with 6.
 constexpr int kRectNchGaussian = 6;
 
-template <int KIND, int NCH>
 __global__ __launch_bounds__(256) void k_direct_rect(const RectArgs a) {
     using T = float;
-    using V4 = float4;
-    __shared__ V4 s_ph[kRC][kRT];
+    constexpr int NCH = kRectNchGaussian;
+    __shared__ float4 s_ph[kRC][kRT];
     __shared__ double s_uvw[kRT][3];
     const int nrg = (a.n_row + 3) / 4, ncg = (a.n_col + 63) / 64;
     const int b = blockIdx.x;
@@ -1375,39 +1356,28 @@ __global__ __launch_bounds__(256) void k_direct_rect(const RectArgs a) {
                 table_sincos(th * f0c, kSinCos32, ps, pc);
                 table_sincos(th * dfc, kSinCos32, qs, qc);
             }
-            V4 ph;
-            ph.x = (T)pc;
-            ph.y = (T)ps;
-            ph.z = (T)qc;
-            ph.w = (T)qs;
-            s_ph[cc][slot] = ph;
+            s_ph[cc][slot] = make_float4((float)pc, (float)ps, (float)qc, (float)qs);
         }
         __syncthreads();
         if (row_ok) {
             for (int cc = 0; cc < nc; ++cc) {
                 const int c = c0 + cc;
-                const V4 A = s_ph[cc][sp];
-                const V4 B = s_ph[cc][sq];
+                const float4 A = s_ph[cc][sp];
+                const float4 B = s_ph[cc][sq];
                 T zr = A.x * B.x + A.y * B.y;
                 T zi = A.y * B.x - A.x * B.y;
                 const T rr = A.z * B.z + A.w * B.w;
                 const T ri_ = A.w * B.z - A.z * B.w;
-                T env = T(1), er = T(1), eg = T(1);
-                if (KIND == KIND_GAUSSIAN) {
-                    const double4 g = shape[c];
-                    const double qf = g.x * (bu * bu) + g.y * (bu * bv) + g.z * (bv * bv);
-                    exp_of(qf * (F0 * F0), env);
-                    exp_of(qf * (DF * (2.0 * F0 + DF)), er);
-                    exp_of(qf * (2.0 * DF * DF), eg);
-                }
+                T env, er, eg;
+                const double4 g = shape[c];
+                const double qf = g.x * (bu * bu) + g.y * (bu * bv) + g.z * (bv * bv);
+                exp_of(qf * (F0 * F0), env);
+                exp_of(qf * (DF * (2.0 * F0 + DF)), er);
+                exp_of(qf * (2.0 * DF * DF), eg);
                 const T *cc8 = coh + ((size_t)c * a.nchan_pad + f0) * 8;
 #pragma unroll
                 for (int k = 0; k < NCH; ++k) {
-                    T pr_ = zr, pi_ = zi;
-                    if (KIND == KIND_GAUSSIAN) {
-                        pr_ *= env;
-                        pi_ *= env;
-                    }
+                    const T pr_ = zr * env, pi_ = zi * env;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const T cr = cc8[k * 8 + 2 * e], ci = cc8[k * 8 + 2 * e + 1];
@@ -1419,10 +1389,8 @@ __global__ __launch_bounds__(256) void k_direct_rect(const RectArgs a) {
                     const T nr = zr * rr - zi * ri_;
                     zi = zr * ri_ + zi * rr;
                     zr = nr;
-                    if (KIND == KIND_GAUSSIAN) {
-                        env *= er;
-                        er *= eg;
-                    }
+                    env *= er;
+                    er *= eg;
                 }
             }
         }
@@ -1508,7 +1476,7 @@ hipError_t launch_direct_rect(Kind kind, const RectArgs &a, DevBuf *part, hipStr
                                      : launch_rect<KIND_POINT, true>(a, part, stream);
     if (kind != KIND_GAUSSIAN) return hipErrorInvalidValue;  // FP32 points take the MFMA point path
     const long total = (long)((a.n_row + 3) / 4) * ((a.n_col + 63) / 64) * chunk_count(a.chunks, kRectNchGaussian, a.nchan);
-    hipLaunchKernelGGL((k_direct_rect<KIND_GAUSSIAN, kRectNchGaussian>), dim3((unsigned)total), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(k_direct_rect, dim3((unsigned)total), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
