@@ -648,6 +648,23 @@ static hipError_t launch_tiles_form(TiledArgs a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// Whether part holds, or could be made to hold, `bytes` of slice sums.
+static bool reserve_slices(DevBuf *part, size_t bytes) {
+    if (part == nullptr) return false;
+    if (part->ptr == nullptr || part->bytes < bytes) {
+        size_t free_b = 0, total_b = 0;
+        if (!part->borrowed && (hipMemGetInfo(&free_b, &total_b) != hipSuccess || bytes > (free_b + part->bytes) / 8)) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (part->reserve(bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    return true;
+}
+
 // Components of a slice: whole stages.
 static int slice_length(int ncomp, int slices) { return ((ncomp + slices - 1) / slices + kCT - 1) / kCT * kCT; }
 
@@ -720,10 +737,7 @@ static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t 
     TiledArgs a = a_in;
     a.part = nullptr;
     const size_t n = (size_t)a.nchan * a.ntiles * (a.ntiles - 1) * 2;
-    if (best.slices > 1 && part->reserve(sizeof(double2) * n * best.slices) != hipSuccess) {
-        (void)hipGetLastError();  // no room for the slices' sums
-        best = choose_tiles_form(g, a, false);
-    }
+    if (best.slices > 1 && !reserve_slices(part, sizeof(double2) * n * best.slices)) best = choose_tiles_form(g, a, false);
     a.slices = best.slices;
     if (a.slices > 1) a.part = part->as<double2>();
     a.slice_len = slice_length(a.ncomp, a.slices);
@@ -1455,10 +1469,7 @@ static hipError_t launch_rect(const RectArgs &a, DevBuf *part, hipStream_t strea
             t_best = t;
         }
     }
-    if (slices > 1 && (part == nullptr || part->reserve(sizeof(double2) * n * slices) != hipSuccess)) {
-        (void)hipGetLastError();
-        slices = 1;
-    }
+    if (slices > 1 && !reserve_slices(part, sizeof(double2) * n * slices)) slices = 1;
     double2 *p = slices > 1 ? part->as<double2>() : nullptr;
     const int slice_len = ((a.ncomp + slices - 1) / slices + kRectC - 1) / kRectC * kRectC;
     hipLaunchKernelGGL((k_rect_mfma<KIND, NARROW>), dim3((unsigned)(per_slice * slices)), dim3(64 * WR), 0, stream, a,

@@ -9,10 +9,10 @@
 
 namespace sm {
 
-// Bytes that the slices' sums of a launch may take: half of what the class tables leave free
-// (reserve_class_table), and beyond what any launch gains from. (An estimate is a few per cent off, and
-// without a bound 1000 tiles, 768 channels and 200000 components would take two slices of 24 GB for 1%.)
-constexpr size_t kSliceBytes = size_t(512) << 20;
+// Bytes that the slices' sums of a launch may take; they also take no more than an eighth of the device's
+// free memory. (256 tiles, 384 channels, 50000 points take two slices of 650 MB, 396 -> 383 ms; without a
+// bound 1000 tiles, 768 channels and 200000 components would take two of 24 GB for an estimated 1%.)
+constexpr size_t kSliceBytes = size_t(4) << 30;
 
 struct TiledArgs {
     int ntiles, nbl, nchan, nchan_pad, ncomp, npairs, nchunks;
