@@ -718,15 +718,15 @@ TilesChoice choose_tiles_form(bool g, const TiledArgs &a, bool may_slice) {
     return best;
 }
 
-// The FP32 kernel's blocks are three to a CU and take n components in n (0.53, 0.55, 0.64) us for one, two
-// and three of them, 0.09 less behind a full round (32 to 256 tiles, 256 to 2048 blocks); the estimates of
-// both kernels are within 7%, so that 8% decide. us a timestep, FP32 and FP64: 128 tiles, 72 channels, 200 Gaussians 183 and 201, 1000
-// 619 and 578; 96 channels, 1000 628 and 639, 5000 2752 and 2530; 256 tiles, 36 channels, 5000 3245 and
-// 4400.
+// The FP32 kernel's blocks are three to a CU: with x = blocks / 256, n components take n (0.53, 0.55, 0.64)
+// us for up to one, two and three a CU, then n (0.30 + 0.183 x) (32 to 256 tiles, x of 1 to 64, within 8%).
+// The FP64 kernel's estimate is some 5% short at such sizes, so that 8% decide. us a timestep, FP32 and
+// FP64: 128 tiles, 72 channels, 200 Gaussians 183 and 207, 1000 619 and 555; 96 channels, 1000 628 and 639,
+// 5000 2752 and 2542; 230 tiles, 48 channels, 10000 10810 and 8250, 96 channels 15650 and 16180; 256 tiles,
+// 36 channels, 5000 3245 and 4541.
 bool fp64_gaussians_faster(const TiledArgs &a) {
-    const int k = (a.npairs * chunk_count(a.chunks, kTiledNchGaussian, a.nchan) + 255) / 256;
-    const double rest = k % 3 == 0 ? 0.0 : (k % 3 == 1 ? 0.53 : 0.55) - (k > 3 ? 0.09 : 0.0);
-    const double us32 = 15.0 + a.ncomp * (0.64 * (k / 3) + rest);
+    const double x = (double)a.npairs * chunk_count(a.chunks, kTiledNchGaussian, a.nchan) / 256.0;
+    const double us32 = 15.0 + a.ncomp * (x > 3.0 ? 0.30 + 0.183 * x : (x > 2.0 ? 0.64 : (x > 1.0 ? 0.55 : 0.53)));
     return choose_tiles_form(true, a, true).us < 0.92 * us32;
 }
 

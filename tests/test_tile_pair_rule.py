@@ -69,7 +69,9 @@ PRECISION = {
     (128, 72, 200): (183.0, 206.9), (128, 72, 1000): (619.0, 555.0), (128, 132, 200): (218.6, 291.6),
     (128, 132, 5000): (3193.1, 3668.5), (200, 48, 1000): (699.7, 804.7), (256, 18, 200): (197.2, 222.0),
     (256, 18, 1000): (627.6, 719.7), (256, 36, 1000): (774.5, 1090.3), (256, 36, 5000): (3244.7, 4540.8),
-    (32, 768, 1000): (604.6, 375.4),
+    (32, 768, 1000): (604.6, 375.4), (230, 48, 10000): (10809, 8253), (230, 96, 10000): (15647, 17893),
+    (230, 384, 10000): (54030, 64570), (128, 400, 10000): (18424, 19590), (180, 300, 6000): (16588, 19700),
+    (60, 768, 20000): (25728, 19357), (256, 768, 2000): (23302, 28549),
 }
 
 
