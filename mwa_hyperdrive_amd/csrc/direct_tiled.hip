@@ -670,10 +670,10 @@ static int slice_length(int ncomp, int slices) { return ((ncomp + slices - 1) / 
 
 // Which form: the one with the smallest estimated time. With k = ceil(blocks / 256) blocks for the CU
 // with the most, n components take start + start_block k + n (comp + comp_block k) us, whether a CU holds
-// one, two or three at once; the constants are fits to the kernel times of every form and slice count at
-// 381 sizes (9 to 256 tiles, 1 to 768 channels, 4 to 6000 components, points and Gaussians), each form's
-// within 6% rms. The form taken is 0.5% slower than the fastest on average, and more than 10% slower at 5
-// sizes of 762. Two row groups of 16 channels share a Gaussian's exponentials and a phasor's set-up over the
+// one, two or three at once (from 8 on the constant part is one of a block: slices do not divide it); the
+// constants are fits to the kernel times of every form and slice count at 393 sizes (9 to 256 tiles, 1 to
+// 768 channels, 4 to 20000 components, points and Gaussians), each form's within 6% rms. The form taken is
+// 0.6% slower than the fastest on average, and more than 10% slower at 5 sizes of 786. Two row groups of 16 channels share a Gaussian's exponentials and a phasor's set-up over the
 // most channels (768 channels, 5600 points 13.7 ms, 2000 Gaussians 7.8 ms; four row groups of 8 channels
 // 13.7 and 8.3 ms). Two row groups of 8 channels fill the chip sooner: 100 points and Gaussians on 24
 // channels and 128 tiles 28 and 37 us, against 38 and 53 us. Splitting the components over eight waves
@@ -709,7 +709,7 @@ TilesChoice choose_tiles_form(bool g, const TiledArgs &a, bool may_slice) {
             const int len = s > 1 ? slice_length(a.ncomp, s) : a.ncomp;
             if ((a.ncomp + len - 1) / len != s) continue;  // the last slices would be empty
             const double k = ceil((double)a.npairs * f.sub * chunk_count(a.chunks, f.nch, a.nchan) * s / 256.0);
-            double t = f.start + f.start_block * k + len * (f.comp + f.comp_block * k);
+            double t = f.start + f.start_block * k + len * fmax(f.comp + f.comp_block * k, (f.comp / 8.0 + f.comp_block) * k);
             const double bytes = (double)sizeof(double2) * n * s;
             if (s > 1) t += 5.0 + 2.0 * bytes / (bytes <= 2e8 ? 12e6 : 4e6);
             if (best.form < 0 || t < best.us) best = TilesChoice{i, s, t};
