@@ -154,7 +154,9 @@ typedef struct SmInfo {
  * their range reduction in FP64, operands split into hi + lo halves of `dtype`, products on
  * MFMA with FP32 accumulation promoted to FP64 every 1024 components. Gaussians and
  * shapelets run in FP32 with their phases, phase reductions, exponents and table positions in
- * FP64. With per-tile beams, every baseline with a tile of the most common beam row takes the
+ * FP64. With d_vis_fb_f64 null, types and sizes for which an FP64 kernel is the faster one take
+ * that, so that FP32 visibilities asked for alone may differ (by FP32 rounding, towards the FP64
+ * path's) from those asked for beside FP64 ones. With per-tile beams, every baseline with a tile of the most common beam row takes the
  * MFMA path (row coherency J_r S J_0^H), and the points of pairs of two tiles of other rows
  * the own-beam pair kernel in FP32 with FP64 phases. */
 enum { SM_MFMA_FP16 = 0, SM_MFMA_BF16 = 1 };
@@ -179,10 +181,9 @@ const char *sm_get_info(SmModeller *m, SmInfo *info);
 const char *sm_set_timing(SmModeller *m, int32_t enabled);
 const char *sm_synchronize(void);
 /* Kernel choice for the direct path: 0 (default) picks the fastest kernel for the case
- * (tile-pair phasor kernel for points and Gaussians with evenly spaced channels and one
- * shared beam, channel-per-lane kernels for shapelets, two channels per lane with a shared
- * beam); 1 forces the baseline-per-lane
- * kernels everywhere. Process-wide; used to compare the two. */
+ * (matrix kernels for points and Gaussians with evenly spaced channels, shapelets by runs of
+ * channels in a cell of the basis table or one channel per lane); 1 forces the
+ * baseline-per-lane kernels everywhere. Process-wide; used to compare the two. */
 const char *sm_set_direct_variant(int32_t variant);
 
 /* Which form of the FP64 tile-pair kernel, and how many slices of the components, a timestep of a

@@ -14,10 +14,10 @@
 // k_rect_mfma does the same for pairs of a tile with its own beam and one of the shared beam.
 //
 // k_shapelets (shapelets, FP64): the coefficient sums are formed once per run of channels within a
-// cell of the basis table. k_shapelet_chan_tiles(32) (per-tile beams) and k_shapelet_chan32 (FP32):
-// one wave per baseline, one or two channels per lane; the table positions x_pos = k f + 5000 of
-// neighbouring channels fall in the same or adjacent table cells, so each coefficient's table reads coalesce
-// across the wave instead of touching 64 unrelated cache lines.
+// cell of the basis table. k_shapelet_chan_tiles (per-tile beams whose runs hold few channels),
+// k_shapelet_chan_tiles32 and k_shapelet_chan32 (FP32): one wave per baseline, one or two channels per lane;
+// the table positions x_pos = k f + 5000 of neighbouring channels fall in the same or adjacent table cells, so
+// each coefficient's table reads coalesce across the wave instead of touching 64 unrelated cache lines.
 #include "sm_internal.h"
 #include "sm_jones.h"
 #include "sm_math.h"

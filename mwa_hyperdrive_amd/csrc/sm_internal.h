@@ -63,8 +63,10 @@ struct BeamDesc {
 // Channel chunks of the direct kernels. With tables: runs of at most 4 (c4), 6 (c6), 8 (c8) or
 // 16 (c16) evenly spaced channels, (first channel, count), so that a flagged channel only shortens
 // the runs around it; every chunk is evenly spaced. Null tables: fixed chunks of 4, 6, 8 or 16
-// consecutive channels, evenly spaced or not. A chunk reads up to 8 channels from its first
-// one, inside the padded channel count (pad_channels adds 8).
+// consecutive channels, evenly spaced or not. A chunk of up to 8 reads at most 8 channels from its
+// first one, inside the padded channel count (pad_channels adds 8). The 16-channel kernels read 16,
+// up to 8 past the padded row: into the next component's, so that a table that they read must hold 8
+// more channels after its last row.
 struct ChunkTabs {
     const int2 *c4 = nullptr;
     int n4 = 0;

@@ -22,7 +22,7 @@ struct TiledArgs {
     const double4 *lmn;
     const double4 *shape;
     // The Hermitian form of the coherency table, [ncomp][nchan_pad][4] = (Re XX, Re XY, Im XY,
-    // Re YY) of J S J^H (launch_coherency with `hermitian`). Valid because the same J stands on
+    // Re YY) of J S J^H (launch_coherency's COH_HERMITIAN). Valid because the same J stands on
     // both sides (one shared beam, or class 0's beam for pairs of two class-0 tiles) and S is
     // Hermitian, so XX and YY are real and YX = conj(XY). Kernels read 16 channels from a chunk's
     // first one: the buffer holds at least 8 more channels after the last row.

@@ -161,7 +161,8 @@ hipError_t gemm(int M, int N, int K, const S *A, int lda, const S *B, int ldb, f
 
 // The weight gradient dW = dZ^T H_in reduces over the whole batch into a small matrix: its output
 // tiles alone (16 of 256 x 256) leave most of the chip idle. The batch is split so that about 512
-// blocks run, no slice below 128 rows, and k_sum_slices adds the slices' results, in FP64, together
+// blocks run, into at most one slice per 128 rows begun (of whole K steps of 32 rows, so that the last
+// slices may be short or empty), and k_sum_slices adds the slices' results, in FP64, together
 // with the column sums of dZ. A batch of 8192 on the 4 x 256 network: 1139 -> 44 us a layer (21 with
 // the operands read ahead), the whole gradient 6.55 -> 0.77 ms (0.51), and its error against 64 bits
 // 1.3e-6 -> 1.5e-7 (shorter FP32 sums).
