@@ -912,12 +912,14 @@ extern "C" const char *sm_tiles_form(int32_t kind, int32_t num_tiles, int32_t nu
     if (freqs == nullptr || form == nullptr || slices == nullptr) return "null argument";
     if (kind < 0 || kind > 2) return "kind must be 0, 1 or 2";
     if (num_tiles < 2 || num_freqs < 1 || num_comps < 1) return "no pairs of tiles, channels or components";
+    if (num_tiles > 65536) return "too many tiles";
     const std::vector<int2> c4 = even_chunks(freqs, num_freqs, 4), c6 = even_chunks(freqs, num_freqs, 6),
                             c8 = even_chunks(freqs, num_freqs, 8), c16 = even_chunks(freqs, num_freqs, 16);
     TiledArgs a{};
     a.chunks = {c4.data(), (int)c4.size(), c6.data(), (int)c6.size(), c8.data(), (int)c8.size(), c16.data(), (int)c16.size()};
     a.ntiles = num_tiles;
-    a.npairs = (int)tile_pairs(num_tiles).size();
+    const int groups = (num_tiles + 15) / 16;
+    a.npairs = groups * (groups - 1) / 2 + (groups + 1) / 2;  // tile_pairs
     a.nchan = num_freqs;
     a.ncomp = num_comps;
     a.even16 = true;
