@@ -186,13 +186,13 @@ const char *sm_synchronize(void);
  * baseline-per-lane kernels everywhere. Process-wide; used to compare the two. */
 const char *sm_set_direct_variant(int32_t variant);
 
-/* Which form of the FP64 tile-pair kernel, and how many slices of the components, a timestep of a
- * modeller takes where num_tiles tiles share a beam, for its points (kind 0), its Gaussians (1) or its
- * Gaussians on the split-precision path with FP32 visibilities alone (2): 0 = 16 channels wide, 1 = 8
- * channels and 16 rows of tiles a block, 2 = 8 channels and 8 rows, 3 and 4 = 8 and 4 channels with the
- * components over eight waves, -1 = the FP32 kernel. Sizes only, no device; used to test every form.
- * No counterpart in the reference. */
-const char *sm_tiles_form(int32_t kind, int32_t num_tiles, int32_t num_freqs, const double *freqs,
+/* Which form of the tile-pair kernels, and how many slices of the components, a timestep of a modeller
+ * takes where num_tiles tiles share a beam, with FP64 visibilities (want_f64) or FP32 ones alone, for its
+ * points (kind 0), its Gaussians (1) or its Gaussians on the split-precision path (2): 0 = 16 channels
+ * wide, 1 = 8 channels and 16 rows of tiles a block, 2 = 8 channels and 8 rows, 3 and 4 = 8 and 4
+ * channels with the components over eight waves, 5 = the FP64 vector kernel, -1 = the FP32 one. Sizes
+ * only, no device; used to test every form. No counterpart in the reference. */
+const char *sm_tiles_form(int32_t kind, int32_t want_f64, int32_t num_tiles, int32_t num_freqs, const double *freqs,
                           int32_t num_comps, int32_t *form, int32_t *slices);
 
 /* Which form of the FP64 shapelet kernels a call takes for a channel step [Hz] and a mean number of

@@ -907,8 +907,8 @@ extern "C" const char *sm_set_class_table_limit(int64_t bytes) {
     return nullptr;
 }
 
-extern "C" const char *sm_tiles_form(int32_t kind, int32_t num_tiles, int32_t num_freqs, const double *freqs,
-                                     int32_t num_comps, int32_t *form, int32_t *slices) {
+extern "C" const char *sm_tiles_form(int32_t kind, int32_t want_f64, int32_t num_tiles, int32_t num_freqs,
+                                     const double *freqs, int32_t num_comps, int32_t *form, int32_t *slices) {
     if (freqs == nullptr || form == nullptr || slices == nullptr) return "null argument";
     if (kind < 0 || kind > 2) return "kind must be 0, 1 or 2";
     if (num_tiles < 2 || num_freqs < 1 || num_comps < 1) return "no pairs of tiles, channels or components";
@@ -923,10 +923,12 @@ extern "C" const char *sm_tiles_form(int32_t kind, int32_t num_tiles, int32_t nu
     a.nchan = num_freqs;
     a.ncomp = num_comps;
     a.even16 = true;
+    JonesF64 none{};
+    a.vis64 = want_f64 != 0 ? &none : nullptr;
     const TilesChoice t = choose_tiles_form(kind != 0, a, true);
-    const bool fp32 = kind == 2 && !fp64_gaussians_faster(a);
-    *form = fp32 ? -1 : t.form;
-    *slices = fp32 ? 1 : t.slices;
+    const bool fp32 = kind == 2 && (want_f64 != 0 || !fp64_gaussians_faster(a)), few = few_components(kind != 0, a);
+    *form = fp32 ? -1 : (few ? 5 : t.form);
+    *slices = fp32 || few ? 1 : t.slices;
     return nullptr;
 }
 

@@ -8,8 +8,8 @@
 // evaluates the phasors of its 32 tiles (middle channel and channel step) into LDS (64
 // sincos shared by 256 baselines instead of 512), each lane forms its baseline's phasors from
 // them, and the FP64 matrix cores multiply them by the coherencies. Diagonal tile blocks are
-// paired so that 240 of 256 pairs are wanted ones. k_direct_tiled is the precision path's FP32
-// form for Gaussians, which keeps the products on the vector ALUs.
+// paired so that 240 of 256 pairs are wanted ones. k_direct_tiled keeps the products on the vector
+// ALUs: the precision path's FP32 Gaussians, and few components in FP64.
 //
 // k_rect_mfma does the same for pairs of a tile with its own beam and one of the shared beam.
 //
@@ -30,10 +30,11 @@ constexpr int kWin = 32;  // shapelet table window per wave and axis, cells
 constexpr int kRows = 16; // shapelet table rows staged per wave
 constexpr int kWinPair = 24;  // shapelet table window per wave and axis of the two-channel kernel, cells
 constexpr int kCT = 32;   // components per LDS stage
-// Channels per lane in k_direct_tiled (FP32 Gaussians). Measured per timestep of 256 tiles,
+// Channels per lane in k_direct_tiled. FP32 Gaussians, measured per timestep of 256 tiles,
 // 384 channels and 10 000 Gaussians: 78.4 ms with 4, 76.2 ms with 6 (142 VGPRs), 115.9 ms with 8.
 constexpr int kTiledNchGaussian = 6;
-static_assert(kTiledNchGaussian <= SM_NCH, "the padded channel count covers whole chunks of SM_NCH channels");
+constexpr int kTiledNchPoint = 8;
+static_assert(kTiledNchGaussian <= SM_NCH && kTiledNchPoint <= SM_NCH, "the padded channel count covers whole chunks of SM_NCH channels");
 
 // The kernels below come in two arithmetic types T. double: the FP64 direct kernels. float:
 // the precision path's kernels, in which the phases, their range reduction mod 2 pi, the table
@@ -106,11 +107,15 @@ template <class T> __device__ __forceinline__ const T *pick(const double *d, con
 template <> __device__ __forceinline__ const double *pick<double>(const double *d, const float *) { return d; }
 template <> __device__ __forceinline__ const float *pick<float>(const double *, const float *f) { return f; }
 
-// The precision path's tile-pair Gaussians: FP32, phases and exponents in FP64.
+// Tile pairs on the vector units: a lane per pair, NCH channels. float: the precision path's Gaussians
+// (phases and exponents in FP64). double: few components on many blocks with FP32 visibilities alone, where
+// reading and adding to the visibilities is most of the time: a lane moves all 32 bytes of one, k_tiles_mfma's
+// 8. 128 tiles, 768 channels, 1 and 7 Gaussians 66 and 82 us (5.9 TB/s), on k_tiles_mfma 100 and 108; 384
+// channels, 2 points 39 and 44.
+template <int KIND, int NCH, class T>
 __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
-    using T = float;
-    constexpr int NCH = kTiledNchGaussian;
-    __shared__ float4 s_ph[kCT][32];
+    using V4 = typename Vec4<T>::type;
+    __shared__ V4 s_ph[kCT][32];
     __shared__ double s_uvw[32][3];
     const int total = a.npairs * a.nchunks;
     int b = blockIdx.x;
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
     const double DF = freqs[f0 + 1] - F0;
     const double f0c = F0 / SM_VEL_C;
     const double dfc = DF / SM_VEL_C;
-    const T *__restrict__ coh = a.coh32;
+    const T *__restrict__ coh = pick<T>(a.coh, a.coh32);
     const double4 *__restrict__ lmn4 = a.lmn;
     const double4 *__restrict__ shape = a.shape;
 
@@ -186,23 +191,30 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
                 table_sincos(th * f0c, kSinCos32, ps, pc);
                 table_sincos(th * dfc, kSinCos32, qs, qc);
             }
-            s_ph[cc][slot] = make_float4((float)pc, (float)ps, (float)qc, (float)qs);
+            V4 ph;
+            ph.x = (T)pc;
+            ph.y = (T)ps;
+            ph.z = (T)qc;
+            ph.w = (T)qs;
+            s_ph[cc][slot] = ph;
         }
         __syncthreads();
         for (int cc = 0; cc < nc; ++cc) {
             const int c = c0 + cc;
-            const float4 A = s_ph[cc][sp];
-            const float4 B = s_ph[cc][sq];
+            const V4 A = s_ph[cc][sp];
+            const V4 B = s_ph[cc][sq];
             T zr = A.x * B.x + A.y * B.y;
             T zi = A.y * B.x - A.x * B.y;
             const T rr = A.z * B.z + A.w * B.w;
             const T ri = A.w * B.z - A.z * B.w;
-            T env, er, eg;
-            const double4 g = shape[c];
-            const double qf = g.x * (bu * bu) + g.y * (bu * bv) + g.z * (bv * bv);
-            exp_of(qf * (F0 * F0), env);
-            exp_of(qf * (DF * (2.0 * F0 + DF)), er);
-            exp_of(qf * (2.0 * DF * DF), eg);
+            T env = T(1), er = T(1), eg = T(1);
+            if (KIND == KIND_GAUSSIAN) {
+                const double4 g = shape[c];
+                const double qf = g.x * (bu * bu) + g.y * (bu * bv) + g.z * (bv * bv);
+                exp_of(qf * (F0 * F0), env);
+                exp_of(qf * (DF * (2.0 * F0 + DF)), er);
+                exp_of(qf * (2.0 * DF * DF), eg);
+            }
             // The table is the Hermitian form (Re XX, Re XY, Im XY, Re YY) of J S J^H (see
             // TiledArgs), 32 contiguous bytes per channel. Per visibility: V_XX = sum C_XX z,
             // A = sum Re(C_XY) z, B = sum Im(C_XY) z, V_YY = sum C_YY z (8 FMAs per component
@@ -210,7 +222,11 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
             const T *cc4 = coh + ((size_t)c * a.nchan_pad + f0) * 4;
 #pragma unroll
             for (int k = 0; k < NCH; ++k) {
-                const T pr_ = zr * env, pi_ = zi * env;
+                T pr_ = zr, pi_ = zi;
+                if (KIND == KIND_GAUSSIAN) {
+                    pr_ *= env;
+                    pi_ *= env;
+                }
                 const T cxx = cc4[k * 4], cxyr = cc4[k * 4 + 1], cxyi = cc4[k * 4 + 2], cyy = cc4[k * 4 + 3];
                 acc[k][0] = fma_t(cxx, pr_, acc[k][0]);
                 acc[k][1] = fma_t(cxx, pi_, acc[k][1]);
@@ -223,8 +239,10 @@ __global__ __launch_bounds__(256) void k_direct_tiled(const TiledArgs a) {
                 const T nr = zr * rr - zi * ri;
                 zi = zr * ri + zi * rr;
                 zr = nr;
-                env *= er;
-                er *= eg;
+                if (KIND == KIND_GAUSSIAN) {
+                    env *= er;
+                    er *= eg;
+                }
             }
         }
         flush_stage(acc, tot);
@@ -750,13 +768,31 @@ static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t 
     }
 }
 
+// 60 tiles, 400 channels: 14 Gaussians 29.9 us, on k_tiles_mfma 32.3, but 20 37.9 and 35.8; 20 points 25.7
+// and 27.7, 28 30.1 and 30.8. 128 tiles, 64 channels (352 blocks), 7 Gaussians 18.3 and 16.6; 768 channels,
+// 24 points 111 and 123.
+bool few_components(bool g, const TiledArgs &a) {
+    const long blocks = (long)a.npairs * chunk_count(a.chunks, g ? kTiledNchGaussian : kTiledNchPoint, a.nchan);
+    return a.vis64 == nullptr && blocks >= 400 && a.ncomp <= (g ? 14 : (blocks < 600 ? 20 : 28));
+}
+
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a_in, DevBuf *part, hipStream_t stream) {
     if (a_in.ncomp <= 0 || a_in.nbl <= 0 || a_in.nchan <= 0) return hipSuccess;
     TiledArgs a = a_in;
     if (a.coh32 != nullptr) {
         if (kind != KIND_GAUSSIAN) return hipErrorInvalidValue;  // FP32 points take the MFMA point path
         a.nchunks = chunk_count(a.chunks, kTiledNchGaussian, a.nchan);
-        hipLaunchKernelGGL(k_direct_tiled, dim3(a.npairs * a.nchunks), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((k_direct_tiled<KIND_GAUSSIAN, kTiledNchGaussian, float>), dim3(a.npairs * a.nchunks),
+                           dim3(256), 0, stream, a);
+        return hipGetLastError();
+    }
+    if (few_components(kind == KIND_GAUSSIAN, a)) {
+        a.nchunks = chunk_count(a.chunks, kind == KIND_GAUSSIAN ? kTiledNchGaussian : kTiledNchPoint, a.nchan);
+        const dim3 grid(a.npairs * a.nchunks);
+        if (kind == KIND_GAUSSIAN)
+            hipLaunchKernelGGL((k_direct_tiled<KIND_GAUSSIAN, kTiledNchGaussian, double>), grid, dim3(256), 0, stream, a);
+        else
+            hipLaunchKernelGGL((k_direct_tiled<KIND_POINT, kTiledNchPoint, double>), grid, dim3(256), 0, stream, a);
         return hipGetLastError();
     }
     return kind == KIND_GAUSSIAN ? (a.narrow ? launch_tiles<KIND_GAUSSIAN, true>(a, part, stream)

@@ -142,6 +142,8 @@ struct TilesChoice {
     double us;
 };
 TilesChoice choose_tiles_form(bool gaussian, const TiledArgs &a, bool may_slice);
+// Whether a's points or Gaussians, in FP64, are so few that the vector kernel takes less time. Host only.
+bool few_components(bool gaussian, const TiledArgs &a);
 // Whether a's Gaussians take less time on the FP64 tile-pair kernel than on the FP32 one. Host only.
 bool fp64_gaussians_faster(const TiledArgs &a);
 // part (nullable) backs slices of the components, which few blocks of many components take.
