@@ -195,11 +195,12 @@ const char *sm_set_direct_variant(int32_t variant);
 const char *sm_tiles_form(int32_t kind, int32_t want_f64, int32_t num_tiles, int32_t num_freqs, const double *freqs,
                           int32_t num_comps, int32_t *form, int32_t *slices);
 
-/* Which form of the FP64 shapelet kernels a call takes for a channel step [Hz] and a mean number of
- * basis-table edges that a component crosses per Hz (both axes): 0 = 2 channels a lane and 2 baselines
- * a wave, 1 = 1 and 1, 2 = 1 and 2, 3 = coefficient sums per channel (per-tile beams alone). Sizes only,
- * no device; used to test every form. No counterpart in the reference. */
-const char *sm_shapelet_form(int32_t per_tile, int32_t num_freqs, double step, double edges_per_hz, int32_t *form);
+/* Which form of the FP64 shapelet kernels a call takes for num_comps components, a channel step [Hz] and
+ * a mean number of basis-table edges that a component crosses per Hz (both axes): 0 = 2 channels a lane
+ * and 2 baselines a wave, 1 = 1 and 1, 2 = 1 and 2, 3 = coefficient sums per channel (per-tile beams
+ * alone). Sizes only, no device; used to test every form. No counterpart in the reference. */
+const char *sm_shapelet_form(int32_t per_tile, int32_t num_comps, int32_t num_freqs, double step,
+                             double edges_per_hz, int32_t *form);
 
 /* Limit in bytes on the per-beam-row-class coherency tables the per-tile-beam paths build
  * (J_r S J_0^H for every class; 64 B per class, component and padded channel). Above it, or

@@ -195,7 +195,7 @@ SIGNATURES = {
     "sm_set_timing": [_P, _I],
     "sm_synchronize": [],
     "sm_set_direct_variant": [_I],
-    "sm_shapelet_form": [_I, _I, _D, _D, C.POINTER(_I)],
+    "sm_shapelet_form": [_I, _I, _I, _D, _D, C.POINTER(_I)],
     "sm_tiles_form": [_I, _I, _I, _I, _P, _I, C.POINTER(_I), C.POINTER(_I)],
     "sm_set_class_table_limit": [C.c_int64],
     "xyzs_to_uvws": [_P, _P, _P, RADec, C.c_int, C.c_int, C.c_int],

@@ -932,11 +932,11 @@ extern "C" const char *sm_tiles_form(int32_t kind, int32_t want_f64, int32_t num
     return nullptr;
 }
 
-extern "C" const char *sm_shapelet_form(int32_t per_tile, int32_t num_freqs, double step, double edges_per_hz,
-                                        int32_t *form) {
+extern "C" const char *sm_shapelet_form(int32_t per_tile, int32_t num_comps, int32_t num_freqs, double step,
+                                        double edges_per_hz, int32_t *form) {
     if (form == nullptr) return "null argument";
     if (num_freqs < 1) return "no channels";
-    *form = choose_shapelet_form(per_tile != 0, num_freqs, step, edges_per_hz);
+    *form = choose_shapelet_form(per_tile != 0, num_comps, num_freqs, step, edges_per_hz);
     return nullptr;
 }
 

@@ -2459,20 +2459,25 @@ static hipError_t launch_shapelets_form(const ShapeletChanArgs &a, hipStream_t s
 //   384 x 80 kHz, 500 m   4.6 4.9 5.5 7.7     24 x 80 kHz, 1500 m      0.93 0.79 0.62 1.36
 //   384 x 80 kHz, 1500 m  6.6 6.3 6.7 7.8     12 x 1.28 MHz, 500 m     1.29 1.00 0.94 1.35
 //   384 x 80 kHz, 3000 m  10.5 9.3 9.4 7.9    12 x 1.28 MHz, 1500 m    3.11 2.20 1.68 1.48
-int choose_shapelet_form(bool per_tile, int nchan, double step, double edges_per_hz) {
+// A group's waves also start and write their visibilities once, which is what a few components cost (us,
+// 128 tiles, 384 channels of 40 kHz, forms 0 to 3): one, shared beam 87 147 142, per-tile beams 105 175 169
+// 96; 16, shared 286 356 378, per-tile 414 478 495 568. `start` holds it, in ms at 128 tiles.
+int choose_shapelet_form(bool per_tile, int ncomp, int nchan, double step, double edges_per_hz) {
     struct Line {
         int span;  // channels of a group
-        double at0, edge, most;
+        double start, at0, edge, most;
     };
-    static const Line kShared[3] = {{64, 0.29, 0.092, 45.0}, {64, 0.37, 0.071, 36.0}, {32, 0.25, 0.069, 20.0}};
-    static const Line kOwn[4] = {{64, 0.56, 0.099, 45.0}, {64, 0.62, 0.075, 37.0}, {32, 0.395, 0.069, 21.0},
-                                 {64, 1.29, 0.0132, 60.0}};
+    static const Line kShared[3] = {
+        {64, 0.0122, 0.29, 0.092, 45.0}, {64, 0.022, 0.37, 0.071, 36.0}, {32, 0.0105, 0.25, 0.069, 20.0}};
+    static const Line kOwn[4] = {{64, 0.014, 0.56, 0.099, 45.0}, {64, 0.026, 0.62, 0.075, 37.0},
+                                 {32, 0.0123, 0.395, 0.069, 21.0}, {64, 0.0107, 1.29, 0.0132, 60.0}};
     int best = 0;
     double t_best = 0.0;
     for (int i = 0; i < (per_tile ? 4 : 3); ++i) {
         const Line &f = per_tile ? kOwn[i] : kShared[i];
         const double edges = edges_per_hz * step * std::min(nchan, f.span);
-        const double t = ((nchan + f.span - 1) / f.span) * (f.at0 + f.edge * fmin(edges, f.most));
+        const double each = (f.at0 + f.edge * fmin(edges, f.most)) / 200.0;
+        const double t = ((nchan + f.span - 1) / f.span) * (f.start + ncomp * each);
         if (i == 0 || t < t_best) {
             best = i;
             t_best = t;
@@ -2519,7 +2524,7 @@ hipError_t launch_shapelet_chan(bool per_tile, const ShapeletChanArgs &a, hipStr
     const bool f32 = a.coh32 != nullptr;
     if (f32 && (a.sbf32 == nullptr || (per_tile && a.beam.coh_cls != nullptr && a.coh_cls32 == nullptr)))
         return hipErrorInvalidValue;
-    const int form = choose_shapelet_form(per_tile, a.nchan, a.step, a.edges_per_hz);
+    const int form = choose_shapelet_form(per_tile, a.ncomp, a.nchan, a.step, a.edges_per_hz);
     if (!f32 && form < 3) return per_tile ? launch_shapelets<true>(form, a, stream) : launch_shapelets<false>(form, a, stream);
     // Per-tile beams: a.ngroups groups of 64 channels; FP32 shared beam: groups of 128 channels.
     const int total = ((a.nbl + 3) / 4) * (per_tile ? a.ngroups : (a.nchan + 127) / 128);

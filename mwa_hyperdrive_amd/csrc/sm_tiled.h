@@ -150,7 +150,7 @@ bool fp64_gaussians_faster(const TiledArgs &a);
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a, DevBuf *part, hipStream_t stream);
 // The form of the FP64 shapelet kernels (0 .. 2: k_shapelets with 2, 1 and 1 channels a lane for 2, 1 and
 // 2 baselines a wave; 3, per-tile beams alone: k_shapelet_chan_tiles). Host only.
-int choose_shapelet_form(bool per_tile, int nchan, double step, double edges_per_hz);
+int choose_shapelet_form(bool per_tile, int ncomp, int nchan, double step, double edges_per_hz);
 // ShapeletChanArgs::edges_per_hz of the components' shapes and baseline UVs, to device memory.
 hipError_t launch_shapelet_edges(int ncomp, int nbl, const double4 *d_shape, const double2 *d_bl_uv, double *d_out,
                                  hipStream_t stream);
