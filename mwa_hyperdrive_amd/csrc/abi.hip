@@ -160,13 +160,16 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
     //   96 channels, 2000 components (96 blocks) 3324 and 2227; 1000 components of every kind of pair, 192
     //   blocks 2137 and 1942, 384 3166 and 3083, 448 to 672 within 1%, 768 5415 and 5572; 256 tiles, 26 such,
     //   10000 components, the kernel alone: 96 channels (448 blocks) 8820 and 7540, 384 (1792) 25750 and 29400;
-    // - shared-beam shapelets, unless a group of 64 channels crosses more than 20 table edges and there are
-    //   several: 200 components, 128 tiles within 3 km, 192 channels of 160 kHz (28 edges) 6280 and 6370, 64
+    // - shared-beam shapelets, unless they are at most three on a large grid (128 tiles, 384 channels: one 76 and
+    //   88, three 114 and 119, ten 254 and 222; 256 tiles, 96 channels: 86 and 120, 137 and 147, 311 and 262; but
+    //   64 tiles, 192 channels: one 24 and 17), or a group of 64 channels crosses more than 20 table edges and
+    //   there are several: 200 components, 128 tiles within 3 km, 192 channels of 160 kHz (28 edges) 6280 and 6370, 64
     //   tiles 1760 and 2180, but 64 channels 2690 and 2540, 384 of 80 kHz (14 edges) 7310 and 7200; within
     //   1.5 km 96 of 160 kHz (14 edges) 2470 and 2350, 24 of 1.28 MHz 3460 and 1740.
     const bool fp32_path = ctx.fp32 && kind != KIND_POINT && ctx.d_bl_subset == nullptr && g_direct_variant == 0;
     const bool either = fp32_path && vis64 == nullptr;
     const double edges_per_hz = ctx.edges_per_hz > 0.0 ? ctx.edges_per_hz : kTypicalEdgesPerHz;
+    const bool few_large = n <= 3 && (size_t)ctx.nbl * ((ctx.nchan + 63) / 64) > 20000;
     const bool many_edges = ctx.nchan > 64 && edges_per_hz * ctx.step * 64 > 20.0;
     auto fp64_pairs = [&](int ntiles, int npairs) {
         TiledArgs t{};
@@ -179,8 +182,9 @@ hipError_t run_type(Kind kind, const TypeInputs &in, const ModelCtx &ctx, DevBuf
         t.part_limit = std::min(kSliceBytes, ctx.part_limit);
         return fp64_gaussians_faster(t);
     };
+    const bool fp64_shapelets = shared_shapelet && !few_large && !many_edges;
     const bool f32 =
-        fp32_path && !(either && ((shared_shapelet && !many_edges) || (shared_tiled && fp64_pairs(ctx.ntiles, ctx.npairs))));
+        fp32_path && !(either && (fp64_shapelets || (shared_tiled && fp64_pairs(ctx.ntiles, ctx.npairs))));
     const bool planes = shared_shapelet && !(f32 && ctx.d_sbf32 != nullptr);
     e = launch_coherency(n, ctx.nchan, ctx.nchan_pad, ctx.d_freqs_pad, in.fb, ctx.beam, !per_tile, coh.as<double>(),
                          stream, planes ? COH_HERMITIAN_PLANES : (hermitian ? COH_HERMITIAN : COH_FULL));

@@ -13,6 +13,7 @@ from mwa_hyperdrive_amd import _lib, synthetic
 from mwa_hyperdrive_amd.modeller import AnalyticBeam, NoBeam, SkyModeller
 from oracle import oracle as orc
 from tests.helpers import rel_err
+from tests.test_gpu_precision_f32_only import shapelets
 from tests.test_gpu_tile_forms import sky
 from tests.test_gpu_tile_pair_forms import form_of
 
@@ -70,3 +71,21 @@ def test_rows_by_columns(nchan, fp64):
     assert np.abs(want).max() > 0
     assert rel_err(alone, want) <= 1e-6
     assert rel_err(alone, both) <= 2e-6
+
+
+# 3160 baselines: 6 groups of 64 channels are below the line of few components, 7 above it.
+@pytest.mark.parametrize("nchan,ncomp,fp64", [(384, 3, True), (385, 3, False), (385, 1, False), (385, 4, True)])
+def test_few_shapelets(nchan, ncomp, fp64):
+    rng = np.random.default_rng(nchan + ncomp)
+    xyzs, freqs = synthetic.tiles(rng, 80, 1000.0), 100e6 + 40e3 * np.arange(nchan)
+    m = SkyModeller(NoBeam(), shapelets(rng, ncomp), 0, xyzs, freqs, [], synthetic.PHASE_CENTRE, 0.0,
+                    synthetic.MWA_LAT_RAD)
+    shape = (nchan, 3160, 8)
+    alone, both = run(m, shape, False), run(m, shape, True)
+    assert np.array_equal(alone, both) == (not fp64)
+    v64 = torch.zeros(shape, dtype=torch.float64, device="cuda")
+    m.model_timestep_with_device(0.2, synthetic.MWA_LAT_RAD, torch.zeros_like(v64, dtype=torch.float32), v64)
+    want = v64.cpu().numpy()
+    assert np.abs(want).max() > 0
+    assert rel_err(alone, want) <= 1e-6
+    assert rel_err(both, want) <= 1e-6
