@@ -770,10 +770,10 @@ static hipError_t launch_tiles(const TiledArgs &a_in, DevBuf *part, hipStream_t 
 
 // 60 tiles, 400 channels: 14 Gaussians 29.9 us, on k_tiles_mfma 32.3, but 20 37.9 and 35.8; 20 points 25.7
 // and 27.7, 28 30.1 and 30.8. 128 tiles, 64 channels (352 blocks), 7 Gaussians 18.3 and 16.6; 768 channels,
-// 24 points 111 and 123.
+// 24 points 111 and 123; 81 tiles, 383 channels, 18 Gaussians 51.8 and 56.7.
 bool few_components(bool g, const TiledArgs &a) {
     const long blocks = (long)a.npairs * chunk_count(a.chunks, g ? kTiledNchGaussian : kTiledNchPoint, a.nchan);
-    return a.vis64 == nullptr && blocks >= 400 && a.ncomp <= (g ? 14 : (blocks < 600 ? 20 : 28));
+    return a.vis64 == nullptr && blocks >= 400 && a.ncomp <= (g ? 18 : (blocks < 600 ? 20 : 28));
 }
 
 hipError_t launch_direct_tiled(Kind kind, const TiledArgs &a_in, DevBuf *part, hipStream_t stream) {

@@ -121,7 +121,7 @@ def test_form_vs_baseline_kernel(form, sliced, last, kind, step, mapped):
 @pytest.mark.parametrize("gaussian,nt,nchan,ncomp,few", [
     (False, 40, 633, 1, True), (False, 40, 632, 1, False), (False, 40, 633, 20, True), (False, 40, 633, 21, False),
     (False, 117, 145, 28, True), (False, 117, 145, 29, False), (False, 117, 144, 28, False),
-    (True, 40, 475, 1, True), (True, 40, 474, 1, False), (True, 117, 95, 14, True), (True, 117, 95, 15, False)])
+    (True, 40, 475, 1, True), (True, 40, 474, 1, False), (True, 117, 95, 18, True), (True, 117, 95, 19, False)])
 def test_few_components_vs_baseline_kernel(gaussian, nt, nchan, ncomp, few, mapped):
     freqs = band(nchan, 40e3)
     assert (form_of(gaussian, nt, freqs, ncomp, want_f64=False)[0] == 5) == few
