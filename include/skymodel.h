@@ -52,7 +52,9 @@ const char *model_autos(int num_tiles, int num_freqs, const double *freqs, const
 /* ------------------------------------------------------------------ 2. f64 variants
  * Same as the drop-ins; d_vis_fb_f64 (nullable, device, [freq][baseline]) is accumulated
  * with the un-demoted f64 sums. No counterpart in the reference: it exposes the f64
- * accumulator that SkyModellerCpu keeps before `Jones::from` (src/model/cpu.rs:335-348). */
+ * accumulator that SkyModellerCpu keeps before `Jones::from` (src/model/cpu.rs:335-348). With
+ * d_vis_fb_f64 null, calls of few components take another FP64 kernel (sm_tiles_form), here and in a
+ * modeller: d_vis_fb then agrees within one FP32 rounding, not always in its last bit. */
 const char *sm_model_points_f64(const Points *comps, const Addresses *a, const UVW *d_uvws,
                                 const JonesF64 *d_beam_jones, JonesF32 *d_vis_fb, JonesF64 *d_vis_fb_f64);
 const char *sm_model_gaussians_f64(const Gaussians *comps, const Addresses *a, const UVW *d_uvws,
