@@ -16,7 +16,9 @@ torch = pytest.importorskip("torch")
 
 from mwa_hyperdrive_amd import _lib, synthetic
 from mwa_hyperdrive_amd.modeller import AnalyticBeam, NoBeam, SkyModeller
+from oracle import oracle as orc
 from tests.helpers import rel_err
+from tests.test_gpu_abi import Buckets, addresses, dt, make_sky, p
 from tests.test_gpu_tile_forms import sky
 
 WIDTH = (16, 8, 8, 8, 4)  # channels of forms 0 .. 4
@@ -131,3 +133,36 @@ def test_few_components_vs_baseline_kernel(gaussian, nt, nchan, ncomp, few, mapp
     alone = run(m, shape, False)[0].cpu().numpy()
     assert np.abs(w64).max() > 0
     assert rel_err(alone, w32) <= 2e-7  # one FP32 rounding on each side
+
+
+# The drop-ins have fixed chunks instead of tables of them.
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,nchan", [("point", 634), ("gaussian", 476)])
+def test_few_components_of_dropins_vs_baseline_kernel(kind, nchan):
+    rng = np.random.default_rng(nchan)
+    nt, lst, pc, freqs = 40, 0.3, synthetic.PHASE_CENTRE, band(nchan, 40e3)
+    assert form_of(kind == "gaussian", nt, freqs, 3, want_f64=False)[0] == 5
+    xyzs = synthetic.tiles(rng, nt, 1000.0)
+    b = Buckets(make_sky(rng, 1, freqs, kind), freqs, pc, xyzs, lst)
+    uvw = dt(orc.cross_uvws(xyzs, lst - pc[0], pc[1]))
+    a, keep = addresses(freqs, len(uvw), 1, np.zeros(nt), np.zeros(nchan), np.arange(nt))
+    args = []
+    for name in ("pl", "cpl", "list"):
+        fields = ["lmn", "fds"] + (["sis"] if name != "list" else []) + (["qs"] if name == "cpl" else [])
+        args += [b.n[name]] + [b.g(name + "_" + f) for f in fields + ([] if kind == "point" else ["gps"])]
+    comps = (_lib.Points if kind == "point" else _lib.Gaussians)(*args)
+
+    def call():
+        vis = torch.zeros((nchan, len(uvw), 8), dtype=torch.float32, device="cuda")
+        _lib.call("sm_model_%ss_f64" % kind, C.byref(comps), C.byref(a), p(uvw), None, p(vis), None)
+        torch.cuda.synchronize()
+        return vis.cpu().numpy()
+
+    alone = call()
+    _lib.call("sm_set_direct_variant", 1)
+    try:
+        want = call()
+    finally:
+        _lib.call("sm_set_direct_variant", 0)
+    assert np.abs(want).max() > 0
+    assert rel_err(alone, want) <= 2e-7  # one FP32 rounding on each side
